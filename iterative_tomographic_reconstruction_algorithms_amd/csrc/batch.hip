@@ -4,7 +4,7 @@
 // A batch holds members, each one distance-driven plan (npix, angles) with its own stack
 // of slices.  One iteration is two persistent launches (forward, back): a fixed grid of
 // blocks pulls work items -- 64 bins of one view of one slice (one 64-thread block), or
-// a 64x64 tile of one slice (256 threads) -- from an atomic counter, largest items
+// a tile of one slice (256 threads) -- from an atomic counter, largest items
 // first, and runs the same per-tile device code as the per-plan kernels.  Every output element is still
 // written by one thread in the reference's accumulation order, so results do not depend
 // on the schedule and equal the per-plan path bit for bit.
@@ -52,6 +52,7 @@ struct itomo_batch {
     int total_slices = 0;
     int nfwd = 0, nback = 0;
     int grid = 0;
+    int back_var = 0;   // one back tile for all members (back_variant_for over all slices)
     std::vector<itomo::BatchMember> h_members;
     std::vector<const itomo_plan*> plans;
     itomo::BatchMember* d_members = nullptr;
@@ -110,10 +111,12 @@ batch_fwd_kernel(const BatchMember* __restrict__ mem, const BatchItem* __restric
     }
 }
 
-__global__ void __launch_bounds__(256)
+template <int T, int P>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(P == 4 ? 4 : P == 2 ? 5 : 1)))
 batch_back_kernel(const BatchMember* __restrict__ mem, const BatchItem* __restrict__ items,
                   int nitems, int* counter, float pc_beta)
 {
+    static_assert(T / P == 16, "256 threads");
     for (;;) {
         const int it = next_item(counter + 1);
         if (it >= nitems) break;
@@ -124,8 +127,8 @@ batch_back_kernel(const BatchMember* __restrict__ mem, const BatchItem* __restri
         e.pc_beta = pc_beta;
         e.partials = m.pb;
         e.blocks_per_slice = m.bps_b;
-        const int nbx = (m.npix + kDdBackTile - 1) / kDdBackTile;
-        dd_back_tile<ITOMO_ARITH_FAST, EPI_SIRT_BACK, false, kDdBackTile, 4>(
+        const int nbx = (m.npix + T - 1) / T;
+        dd_back_tile<ITOMO_ARITH_FAST, EPI_SIRT_BACK, false, T, P>(
             m.geom, m.lstar, m.nang, m.npix, m.work, m.x, (int64_t)m.nang * m.npix,
             (int64_t)m.npix * m.npix, 0, e, w.a, w.b, w.z, w.b * nbx + w.a);
     }
@@ -196,6 +199,14 @@ int itomo_batch_create(itomo_batch** out, int nmembers, const itomo_plan* const*
     size_t scratch_bytes = 0;
     std::vector<size_t> off_xT(nmembers), off_pf(nmembers), off_pb(nmembers);
     auto up = [](size_t v) { return (v + 255) & ~(size_t)255; };
+    size_t tiles64 = 0, tiles32 = 0;
+    for (int m = 0; m < nmembers; ++m)
+        if (plans[m] && nslices[m] > 0) {
+            tiles64 += dd_back_blocks(plans[m]->npix, 64) * nslices[m];
+            tiles32 += dd_back_blocks(plans[m]->npix, 32) * nslices[m];
+        }
+    B->back_var = back_variant_for(tiles64, tiles32);
+    const int tile = kBackTiles[B->back_var][0];
     for (int m = 0; m < nmembers; ++m) {
         const itomo_plan* p = plans[m];
         if (!p || p->projector != ITOMO_PROJ_DD || p->arith != ITOMO_ARITH_FAST) {
@@ -220,7 +231,7 @@ int itomo_batch_create(itomo_batch** out, int nmembers, const itomo_plan* const*
         bm.work = work[m];
         // the batch launches its own shapes whatever the plan's choice
         bm.bps_f = (int)dd_fwd_slots(p->npix, p->nang);
-        bm.bps_b = (int)dd_back_blocks(p->npix, kDdBackTile);
+        bm.bps_b = (int)dd_back_blocks(p->npix, tile);
         B->h_members.push_back(bm);
         B->plans.push_back(p);
         off_xT[m] = scratch_bytes;
@@ -230,7 +241,7 @@ int itomo_batch_create(itomo_batch** out, int nmembers, const itomo_plan* const*
         off_pb[m] = scratch_bytes;
         scratch_bytes += up(sizeof(double) * 3 * (size_t)bm.bps_b * nslices[m]);
         const int nbf = (p->npix + kBatchFwdBlock - 1) / kBatchFwdBlock;
-        const int nbt = (p->npix + kDdBackTile - 1) / kDdBackTile;
+        const int nbt = (p->npix + tile - 1) / tile;
         for (int z = 0; z < nslices[m]; ++z) {
             for (int v = 0; v < p->nang; ++v)
                 for (int a = 0; a < nbf; ++a) fwd.push_back({m, a, v, z});
@@ -309,9 +320,16 @@ int itomo_batch_sirt_iterate(itomo_batch* B, float pc_beta, void* stream)
     reset_counter_kernel<<<1, 1, 0, st>>>(B->d_counter);
     batch_fwd_kernel<<<std::min(B->grid * (256 / kBatchFwdBlock), B->nfwd), kBatchFwdBlock, 0,
                        st>>>(B->d_members, B->d_fwd, B->nfwd, B->d_counter);
-    batch_back_kernel<<<std::min(B->grid, B->nback), 256, 0, st>>>(B->d_members, B->d_back,
-                                                                     B->nback, B->d_counter,
-                                                                     pc_beta);
+    const int bgrid = std::min(B->grid, B->nback);
+    if (B->back_var == 0)
+        batch_back_kernel<64, 4><<<bgrid, 256, 0, st>>>(B->d_members, B->d_back, B->nback,
+                                                        B->d_counter, pc_beta);
+    else if (B->back_var == 1)
+        batch_back_kernel<32, 2><<<bgrid, 256, 0, st>>>(B->d_members, B->d_back, B->nback,
+                                                        B->d_counter, pc_beta);
+    else
+        batch_back_kernel<16, 1><<<bgrid, 256, 0, st>>>(B->d_members, B->d_back, B->nback,
+                                                        B->d_counter, pc_beta);
     batch_finalize_kernel<<<B->total_slices, 256, 0, st>>>(B->d_slices);
     return check_hip(hipGetLastError(), "batch_sirt_iterate launch");
 }

@@ -27,7 +27,7 @@
 namespace itomo {
 
 template <int ARITH, int EPI, bool ONES, int T, int P>
-__global__ void __launch_bounds__((T / P) * (T / P))
+__global__ void __launch_bounds__((T / P) * (T / P)) __attribute__((amdgpu_waves_per_eu(P == 4 ? 4 : P == 2 ? 5 : 1)))
 dd_back_kernel(const DdView* __restrict__ geom, const float* __restrict__ lstar, int nang,
                int npix, const float* __restrict__ sino, float* __restrict__ out,
                int64_t sino_stride, int64_t img_stride, int accumulate, EpiArgs e)
@@ -161,11 +161,13 @@ void launch_back(const Plan& p, const float* sino, float* out, int nslices, int 
                  const EpiArgs& e, hipStream_t st)
 {
     static_assert(kBackTiles[0][0] == 64 && kBackTiles[0][1] == 4 && kBackTiles[1][0] == 32 &&
-                      kBackTiles[1][1] == 2 && kBackTiles[2][0] == 32 && kBackTiles[2][1] == 4,
+                      kBackTiles[1][1] == 2 && kBackTiles[2][0] == 32 && kBackTiles[2][1] == 4 &&
+                      kBackTiles[3][0] == 16 && kBackTiles[3][1] == 1,
                   "variants");
-    switch (p.back_var) {
+    switch (back_variant(p, nslices)) {
     case 1: launch_back_tp<ARITH, EPI, ONES, 32, 2>(p, sino, out, nslices, accumulate, e, st); break;
     case 2: launch_back_tp<ARITH, EPI, ONES, 32, 4>(p, sino, out, nslices, accumulate, e, st); break;
+    case 3: launch_back_tp<ARITH, EPI, ONES, 16, 1>(p, sino, out, nslices, accumulate, e, st); break;
     default: launch_back_tp<ARITH, EPI, ONES, 64, 4>(p, sino, out, nslices, accumulate, e, st); break;
     }
 }
@@ -255,7 +257,7 @@ int dd_forward_epi(const Plan& p, int epi, int ones, const float* image, float* 
 int dd_back_epi(const Plan& p, int epi, int ones, const float* sino, float* out, int nslices,
                 int accumulate, const EpiArgs& e, hipStream_t st, int* blocks_per_slice)
 {
-    const int bps = (int)back_blocks_per_slice(p);
+    const int bps = (int)back_blocks_per_slice(p, nslices);
     if (blocks_per_slice) *blocks_per_slice = bps;
     EpiArgs ee = e;
     ee.blocks_per_slice = bps;

@@ -84,117 +84,190 @@ __device__ __forceinline__ float dd_line_end(const DdView& g, int npix, int nh, 
 // P*ty.., columns P*tx..).  For a row sweep a thread walks its P rows, P consecutive
 // pixels each; for a column sweep its P columns.  Along one line the bin walk is
 // incremental: the first pixel's bin is found once, then each next pixel continues from
-// the previous pixel's last bin.  Views are processed in chunks of kBackViews: the
+// the previous pixel's last bin.  Views are processed in chunks of back_views: the
 // sinogram values the tile can touch in each view (at most back_foot(T) bins) are staged
 // in LDS, with zeros for bins outside [0, npix), so the walk needs no bounds checks.  The
 // accumulation order per pixel (views in list order, bins increasing) is the reference's
 // for every (T, P), so all tilings give bit-identical images.
-constexpr int kBackViews = 32;
+template <int T, int P>
+constexpr int back_views()
+{
+    return T / P == 8 ? 512 / T : (T == 16 ? 64 : 32);
+}
 
 // Staged bins per view: the tile's footprint spans T*(|sin|+|cos|) <= T*sqrt(2) bins,
 // plus 7 for the floors and the +-2 margins of staged_range.
 template <int T>
 constexpr int back_foot() { return (T * 1449) / 1024 + 10; }
 
+// What a tile needs of a view: nothing (it projects outside the detector, or no branch of
+// the reference takes the view), the walk without or with the clip to L*, the walk for views
+// where a pixel may hold two bin keys (with the clip), or a plain sum.
+enum BackClass : int { BACK_SKIP = 0, BACK_WALK, BACK_CLIP, BACK_MULTI, BACK_SUM };
+
+// The class of view g for a tile, and the bins it can touch: the first one, *b_lo, which may
+// lie outside the detector (staged as zeros, so the walks need no clamp), and their number.
+// L* >= min(P[N-1], D[N-1]) on every line, so it clips nothing where the tile's pixels all
+// lie before the last pixel of their lines and project inside the bins [0, npix - 1).
 template <int ARITH, int T>
-__device__ __forceinline__ void staged_range(const DdView& g, int npix, int nh, int r0,
-                                             int q0, int* b_lo, int* cnt)
+__device__ __forceinline__ int staged_range(const DdView& g, int npix, int nh, int r0, int q0,
+                                            int* b_lo, int* cnt)
 {
-    int lo, hi;
-    if (g.kind == DD_ROWSUM) {
-        lo = r0;
-        hi = r0 + T - 1;
-    } else if (g.kind == DD_COLSUM) {
-        lo = q0;
-        hi = q0 + T - 1;
-    } else if (g.kind == DD_SWEEP_ROWS || g.kind == DD_SWEEP_COLS) {
-        // lines are rows (r) or columns (q); pixel boundaries along the line
-        const int l0 = (g.kind == DD_SWEEP_ROWS) ? r0 : q0;
-        const int p0 = (g.kind == DD_SWEEP_ROWS) ? q0 : r0;
-        const float ka = (float)(l0 - nh) + 0.5f, kb = ka + (float)(T - 1);
-        const float K1 = ka * g.t, K2 = kb * g.t;
-        const float kmin = (float)(p0 - nh) - fmaxf(K1, K2);
-        const float kmax = (float)(p0 + T - nh) - fminf(K1, K2);
-        float f1 = floorf(kmin * g.est), f2 = floorf(kmax * g.est);
-        f1 = fminf(fmaxf(f1, (float)(-nh - 4)), (float)(npix - nh + 4));
-        f2 = fminf(fmaxf(f2, (float)(-nh - 4)), (float)(npix - nh + 4));
-        lo = (int)f1 + nh - 2;
-        hi = (int)f2 + nh + 2;
-    } else {
-        lo = 0;
-        hi = -1;
+    *b_lo = 0;
+    *cnt = 0;
+    if (g.kind == DD_ROWSUM || g.kind == DD_COLSUM) {
+        *b_lo = g.kind == DD_ROWSUM ? r0 : q0;
+        *cnt = T;
+        return BACK_SUM;
     }
-    lo = max(lo, -1);
-    hi = min(hi, npix);
+    if (g.kind != DD_SWEEP_ROWS && g.kind != DD_SWEEP_COLS) return BACK_SKIP;
+    // lines are rows (r) or columns (q); pixel boundaries along the line
+    const int l0 = (g.kind == DD_SWEEP_ROWS) ? r0 : q0;
+    const int p0 = (g.kind == DD_SWEEP_ROWS) ? q0 : r0;
+    const float ka = (float)(l0 - nh) + 0.5f, kb = ka + (float)(T - 1);
+    const float K1 = ka * g.t, K2 = kb * g.t;
+    const float kmin = (float)(p0 - nh) - fmaxf(K1, K2);
+    const float kmax = (float)(p0 + T - nh) - fminf(K1, K2);
+    const int lo = (int)floorf(kmin * g.est) + nh - 2;
+    const int hi = (int)floorf(kmax * g.est) + nh + 2;
+    if (hi < 0 || lo >= npix) return BACK_SKIP;
     *b_lo = lo;
-    *cnt = max(0, min(hi - lo + 1, back_foot<T>()));
+    *cnt = min(hi - lo + 1, back_foot<T>());
+    if (g.multi) return BACK_MULTI;
+    return hi <= npix - 2 && p0 + T < npix ? BACK_WALK : BACK_CLIP;
 }
 
-// One line of P pixels with along-line indices p0..p0+P-1, accumulating into
-// a[0], a[STRIDE], ..., a[(P-1)*STRIDE].  S points at LDS such that S[d] is bin d of
-// this view (zero outside [0, npix)); Ls is the line's L*.
-//
-// Bins are at least as wide as pixels (1/|sin| or 1/|cos| >= 1), so a pixel crosses at
-// most one bin boundary, except when the two widths agree to rounding (views flagged
-// `multi`, the MULTI instance): there a loop picks up the further crossings.  Bins are
-// visited in increasing order either way.  Past the last bin the weights vanish by the
-// L* clip (Ls <= D[N]), so the walk needs no bound there.
-//
-// The walk keeps the bin that holds the pixel's left end lo (D_lo <= lo < D_hi), so
-// every overlap starts at lo or at a crossed key; the one exception, a left end below
-// bin -1, reads a staged zero.  A weight max(R - L, 0) of zero leaves the sum unchanged,
-// so no overlap needs a test.
-template <int ARITH, int P, int STRIDE, bool MULTI>
-__device__ __forceinline__ void walk_line(const DdView& g, int npix, int nh, float K, float Ls,
-                                          int p0, const float* S, float* a)
+// Constants of a walked view as the walk reads them from LDS: (rinv, t) in FAST
+// and (b, a) in IEEE arithmetic, est, and the index offset of the view's staged bins.
+template <int ARITH>
+__device__ __forceinline__ float4 walk_pack(const DdView& g, int base)
 {
-    float x = (float)(p0 - nh);
-    float lo = __fsub_rn(x, K);
-    // (index - nh) of the bin holding lo (D_j <= lo < D_j+1), then the clamp to
-    // [-1, npix] (bins -1 and npix read staged zeros).  In index units the estimate
-    // lo*est is off from lo/(bin width) by a relative 2^-22 (est * rinv = 1 + 2^-23 at
-    // most) and the keys by a relative 2^-24; with |j| <= 2*16384 that stays below 0.01,
-    // so floor(lo*est + 1/2) is j or j + 1 and one test against D_fd settles it.
-    float fd = floorf(__fadd_rn(__fmul_rn(lo, g.est), 0.5f));
-    fd = (lo < key_Df<ARITH>(g, fd)) ? __fsub_rn(fd, 1.0f) : fd;
-    fd = __builtin_amdgcn_fmed3f(fd, (float)(-nh - 1), (float)(npix - nh));
-    // fr = (index - nh) of the current bin's right key Dhi; the bin is (int)fr + nh - 1
-    // (fr is an integer-valued float, the conversion exact)
-    float fr = __fadd_rn(fd, 1.0f);
-    float Dhi = key_Df<ARITH>(g, fr);
-    const int dbase = nh - 1;
-#define ITOMO_PIX(acc)                                                                  \
-    {                                                                                   \
-        x = __fadd_rn(x, 1.0f);                                                         \
-        const float hi = __fsub_rn(x, K);                                               \
-        const float hc = fminf(hi, Ls);                                                 \
-        const int d = (int)fr + dbase;                                                  \
-        const float s0 = S[d], s1 = S[d + 1];                                           \
-        acc = accum<ARITH>(fmaxf(__fsub_rn(fminf(hc, Dhi), lo), 0.0f), s0, acc);        \
-        const float fr2 = __fadd_rn(fr, 1.0f);                                          \
-        const float Dhi2 = key_Df<ARITH>(g, fr2);                                       \
-        /* one crossing at most: the span ends in (Dhi, Dhi2] when it crosses */        \
-        const float R2 = MULTI ? fminf(hc, Dhi2) : hc;                                  \
-        acc = accum<ARITH>(fmaxf(__fsub_rn(R2, Dhi), 0.0f), s1, acc);                   \
-        const bool cross = Dhi < hi;                                                    \
-        fr = cross ? fr2 : fr;                                                          \
-        Dhi = cross ? Dhi2 : Dhi;                                                       \
-        if (MULTI) {                                                                    \
-            int dm = d + 1;                                                             \
-            while (cross && dm < npix && Dhi < hi) {                                    \
-                ++dm;                                                                   \
-                const float Dlo = Dhi;                                                  \
-                fr = __fadd_rn(fr, 1.0f);                                               \
-                Dhi = key_Df<ARITH>(g, fr);                                             \
-                acc = accum<ARITH>(fmaxf(__fsub_rn(fminf(hc, Dhi), Dlo), 0.0f), S[dm],  \
-                                   acc);                                                \
-            }                                                                           \
-        }                                                                               \
-        lo = hi;                                                                        \
+    if (ARITH == ITOMO_ARITH_FAST) return make_float4(g.rinv, g.t, g.est, __int_as_float(base));
+    return make_float4(g.b, g.a, g.est, __int_as_float(base));
+}
+
+template <int ARITH>
+__device__ __forceinline__ DdView walk_unpack(float4 c)
+{
+    DdView g;
+    if (ARITH == ITOMO_ARITH_FAST) {
+        g.rinv = c.x;
+        g.t = c.y;
+    } else {
+        g.b = c.x;
+        g.a = c.y;
     }
+    g.est = c.z;
+    return g;
+}
+
+// jr = (index - nh) of the right key of the bin that holds a pixel's left end lo
+// (D_jr-1 <= lo < D_jr).  In index units the estimate lo*est is off from lo/(bin width) by a
+// relative 2^-22 (est * rinv = 1 + 2^-23 at most) and the keys by a relative 2^-24; with
+// |j| <= 2*16384 that stays below 0.01, so floor(lo*est + 1/2) is the bin or the one after it
+// and one test against its key settles it.
+template <int ARITH>
+__device__ __forceinline__ int walk_first(const DdView& g, float lo)
+{
+    float fd = floorf(__fadd_rn(__fmul_rn(lo, g.est), 0.5f));
+    // the integer comes from this very float: left to itself the compiler fuses the rounded
+    // sum, the floor and the conversion into an instruction that rounds otherwise
+    asm("" : "+v"(fd));
+    int jr = (int)fd + 1;
+    jr -= lo < key_Df<ARITH>(g, fd);
+    return jr;
+}
+
+// The P x P pixels of a thread in a walked view (see staged_range): lines u, u + 1, ... and
+// along each line the pixels from x0; pixel k of line i goes to a[i * LS + k * KS].  S[jr] is
+// the value of the bin whose right key has index jr (zero outside the detector); Ls[i] is
+// L* of line i.  A pixel [lo, hi] gives that bin the weight m - lo and the next one hi - m with
+// m = min(hi, Dhi): where it does not reach past Dhi the second is exactly 0, where it does
+// they are that pixel's own overlaps, end minus start.  (Bins are at least as wide as pixels,
+// so a pixel reaches one bin key at most, except where the two widths agree to rounding:
+// MULTI takes a third bin the same way; three keys in a pixel would need bins of half a
+// pixel.)  CLIP: hi is clipped to L* first, and a pixel that starts past L* gets the weight 0.
+// A weight of 0 leaves the sum unchanged, so no overlap needs a test.  11 VALU operations per
+// pixel, CLIP 13.  The lines advance side by side, and a step's values are added one step
+// later, so that the P chains (key, compare, next bin) and the LDS reads hide behind each
+// other.
+template <int ARITH, int P, int LS, int KS, bool CLIP, bool MULTI = false>
+__device__ __forceinline__ void walk_tile(const DdView& g, float u, float x0, const float* S,
+                                          const float* Ls, float* a)
+{
+    // taken anew per call: the compiler would otherwise keep every u + i and x0 + k of both
+    // sweep directions in registers across the views
+    asm("" : "+v"(u), "+v"(x0));
+    float K[P], lo[P], end[P];
+    int jr[P];
 #pragma unroll
-    for (int k = 0; k < P; ++k) ITOMO_PIX(a[k * STRIDE])
-#undef ITOMO_PIX
+    for (int i = 0; i < P; ++i) {
+        K[i] = key_K<ARITH>(g, __fadd_rn(u, (float)i));
+        lo[i] = __fsub_rn(x0, K[i]);
+        jr[i] = walk_first<ARITH>(g, lo[i]);
+        if (CLIP) end[i] = Ls[i];
+    }
+    float w0[P], w1[P], w2[P], s0[P], s1[P], s2[P];
+#pragma unroll
+    for (int k = 0; k <= P; ++k) {
+        float v0[P], v1[P], v2[P], t0[P], t1[P], t2[P];
+        if (k < P) {
+#pragma unroll
+            for (int i = 0; i < P; ++i) {
+                t0[i] = S[jr[i]];
+                t1[i] = S[jr[i] + 1];
+                const float Dhi = key_Df<ARITH>(g, (float)jr[i]);
+                const float hi = __fsub_rn(__fadd_rn(x0, (float)(k + 1)), K[i]);
+                const float hc = CLIP ? fminf(hi, end[i]) : hi;
+                const float m = fminf(hc, Dhi);
+                v0[i] = __fsub_rn(m, lo[i]);
+                if (CLIP) v0[i] = fmaxf(v0[i], 0.0f);
+                if (MULTI) {
+                    const float Dhi2 = key_Df<ARITH>(g, (float)(jr[i] + 1));
+                    const float m2 = fminf(hc, Dhi2);
+                    t2[i] = Dhi2 < hc ? S[jr[i] + 2] : 0.0f;
+                    v1[i] = fmaxf(__fsub_rn(m2, Dhi), 0.0f);
+                    v2[i] = __fsub_rn(hc, m2);
+                    jr[i] += Dhi2 < hi;
+                } else {
+                    v1[i] = __fsub_rn(hc, m);
+                }
+                jr[i] += Dhi < hi;
+                // kept as one value (a carry add): the compiler would otherwise track the
+                // LDS address and the key's index apart
+                asm("" : "+v"(jr[i]));
+                lo[i] = hi;
+            }
+        }
+        if (k > 0) {
+#pragma unroll
+            for (int i = 0; i < P; ++i) {
+                float& acc = a[i * LS + (k - 1) * KS];
+                acc = accum<ARITH>(w0[i], s0[i], acc);
+                acc = accum<ARITH>(w1[i], s1[i], acc);
+                if (MULTI) acc = accum<ARITH>(w2[i], s2[i], acc);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < P; ++i) {
+            w0[i] = v0[i];
+            w1[i] = v1[i];
+            s0[i] = t0[i];
+            s1[i] = t1[i];
+            if (MULTI) {
+                w2[i] = v2[i];
+                s2[i] = t2[i];
+            }
+        }
+    }
+}
+
+// A wave-uniform 64-bit value as scalars.
+__device__ __forceinline__ unsigned long long uniform64(unsigned long long m)
+{
+    const unsigned lo = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)m);
+    const unsigned hi = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(m >> 32));
+    return lo | (unsigned long long)hi << 32;
 }
 
 // One T x T tile (tile column bx, tile row by) of slice z; blk indexes its FP64
@@ -207,10 +280,16 @@ __device__ __forceinline__ void dd_back_tile(const DdView* __restrict__ geom,
                                              int64_t img_stride, int accumulate,
                                              const EpiArgs& e, int bx, int by, int z, int blk)
 {
-    constexpr int TP = T / P, NT = TP * TP, FOOT = back_foot<T>();
+    constexpr int TP = T / P, NT = TP * TP, FOOT = back_foot<T>(), kBackViews = back_views<T, P>();
     __shared__ float sS[kBackViews][FOOT];
     __shared__ int sLo[kBackViews];
     __shared__ int sCnt[kBackViews];
+    __shared__ int sRow[kBackViews];
+    __shared__ int sLine[kBackViews];
+    __shared__ float4 sGeo[kBackViews];      // walked views: see walk_pack
+    // bit v: view v of the chunk is walked, walked with the clip, skipped, sweeps rows, has
+    // two keys in a pixel
+    __shared__ unsigned long long sMask[5];
     __shared__ float sLs[kBackViews][T];   // L* of the tile's lines per view
 
     const int tid = threadIdx.x;
@@ -260,66 +339,145 @@ __device__ __forceinline__ void dd_back_tile(const DdView* __restrict__ geom,
     for (int v0 = 0; v0 < nang; v0 += kBackViews) {
         const int nv = min(kBackViews, nang - v0);
         __syncthreads();  // previous chunk fully consumed
-        if (tid < nv) {
-            int lo, cnt;
-            staged_range<ARITH, T>(geom[v0 + tid], npix, nh, r0, q0, &lo, &cnt);
-            sLo[tid] = lo;
-            sCnt[tid] = cnt;
+        if (tid < 64) {
+            int cls = BACK_SKIP;
+            bool rows = false;
+            if (tid < nv) {
+                int lo, cnt;
+                const DdView g = geom[v0 + tid];
+                cls = staged_range<ARITH, T>(g, npix, nh, r0, q0, &lo, &cnt);
+                sLo[tid] = lo;
+                sCnt[tid] = cnt;
+                sRow[tid] = g.row;
+                sLine[tid] = g.kind == DD_SWEEP_COLS ? q0 : r0;
+                rows = g.kind == DD_SWEEP_ROWS;
+                sGeo[tid] = walk_pack<ARITH>(g, tid * FOOT - lo + nh - 1);
+            }
+            const unsigned long long b0 = __ballot(cls == BACK_WALK || cls == BACK_CLIP),
+                                     b1 = __ballot(cls == BACK_CLIP),
+                                     b2 = __ballot(cls == BACK_SKIP), b3 = __ballot(rows),
+                                     b4 = __ballot(cls == BACK_MULTI);
+            if (tid == 0) {
+                sMask[0] = b0;
+                sMask[1] = b1;
+                sMask[2] = b2;
+                sMask[3] = b3;
+                sMask[4] = b4;
+            }
         }
         __syncthreads();
-        for (int k = tid; k < nv * FOOT; k += NT) {
-            const int v = k / FOOT, j = k - v * FOOT;
-            const int d = sLo[v] + j;
-            float val = 0.0f;
-            if (j < sCnt[v] && d >= 0 && d < npix)
-                val = ONES ? 1.0f : sino[(int64_t)geom[v0 + v].row * npix + d];
-            sS[v][j] = val;
+        const unsigned long long walked = uniform64(sMask[0]), clipped = uniform64(sMask[1]),
+                                 skipped = uniform64(sMask[2]), rowviews = uniform64(sMask[3]),
+                                 multi = uniform64(sMask[4]);
+        // Four loads at a time: one by one, each waits for its own latency at the barriers'
+        // expense; all at once, they take the registers of the walk.
+        constexpr int U = NT == 64 ? 8 : 4;
+#pragma unroll 1
+        for (int k0 = tid; k0 < nv * FOOT; k0 += U * NT) {
+            float val[U];
+#pragma unroll
+            for (int r = 0; r < U; ++r) {
+                const int k = k0 + r * NT, v = k / FOOT, j = k - v * FOOT;
+                val[r] = 0.0f;
+                if (v < nv) {
+                    const int d = sLo[v] + j;
+                    if (j < sCnt[v] && d >= 0 && d < npix)
+                        val[r] = ONES ? 1.0f : sino[(int64_t)sRow[v] * npix + d];
+                }
+            }
+#pragma unroll
+            for (int r = 0; r < U; ++r)
+                if (k0 + r * NT < nv * FOOT) (&sS[0][0])[k0 + r * NT] = val[r];
         }
-        for (int k = tid; k < nv * T; k += NT) {
-            const int v = k / T, l = k - v * T;
-            const int line = (geom[v0 + v].kind == DD_SWEEP_COLS ? q0 : r0) + l;
-            sLs[v][l] = line < npix ? lstar[(int64_t)(v0 + v) * npix + line] : 0.0f;
+#pragma unroll 1
+        for (int k0 = tid; k0 < nv * T; k0 += U * NT) {
+            float val[U];
+#pragma unroll
+            for (int r = 0; r < U; ++r) {
+                const int k = k0 + r * NT, v = k / T, l = k - v * T;
+                val[r] = INFINITY;   // no clip
+                if (v < nv && !(((walked & ~clipped) | skipped) >> v & 1)) {
+                    const int line = sLine[v] + l;
+                    if (line < npix) val[r] = lstar[(int64_t)(v0 + v) * npix + line];
+                }
+            }
+#pragma unroll
+            for (int r = 0; r < U; ++r)
+                if (k0 + r * NT < nv * T) (&sLs[0][0])[k0 + r * NT] = val[r];
         }
         __syncthreads();
         for (int v = 0; v < nv; ++v) {
-            const DdView g = geom[v0 + v];
+            if ((skipped >> v) & 1) continue;
+            if constexpr (P == 1) {
+                // One pixel per thread: G consecutive walked views are formed side by side and
+                // added in view order.
+                constexpr int G = 4;
+                constexpr unsigned ALL = (1u << G) - 1;
+                if (v + G <= nv && ((walked >> v) & ALL) == ALL) {
+                    float wa[G], wb[G], sa[G], sb[G];
+                    const bool clip = ((clipped >> v) & ALL) != 0;
+#pragma unroll
+                    for (int k = 0; k < G; ++k) {
+                        const float4 c = sGeo[v + k];
+                        const DdView g = walk_unpack<ARITH>(c);
+                        const float* S = &sS[0][0] + __float_as_int(c.w);
+                        const bool rows = (rowviews >> (v + k)) & 1;
+                        const float K = key_K<ARITH>(g, line_coord(rows ? rr : cc, nh));
+                        const float x = (float)((rows ? cc : rr) - nh);
+                        const float lo = __fsub_rn(x, K);
+                        const int jr = walk_first<ARITH>(g, lo);
+                        sa[k] = S[jr];
+                        sb[k] = S[jr + 1];
+                        float hi = __fsub_rn(__fadd_rn(x, 1.0f), K);
+                        if (clip) hi = fminf(hi, sLs[v + k][rows ? ty : tx]);
+                        const float m = fminf(hi, key_Df<ARITH>(g, (float)jr));
+                        wa[k] = fmaxf(__fsub_rn(m, lo), 0.0f);
+                        wb[k] = __fsub_rn(hi, m);
+                    }
+#pragma unroll
+                    for (int k = 0; k < G; ++k) {
+                        acc[0][0] = accum<ARITH>(wa[k], sa[k], acc[0][0]);
+                        acc[0][0] = accum<ARITH>(wb[k], sb[k], acc[0][0]);
+                    }
+                    v += G - 1;
+                    continue;
+                }
+            }
+            if (((walked | multi) >> v) & 1) {
+                const float4 c = sGeo[v];
+                const DdView g = walk_unpack<ARITH>(c);
+                const float* S = &sS[0][0] + __float_as_int(c.w);
+                if ((rowviews >> v) & 1) {
+                    const float u = line_coord(rr, nh), x0 = (float)(cc - nh);
+                    const float* Ls = &sLs[v][P * ty];
+                    if ((multi >> v) & 1)
+                        walk_tile<ARITH, P, P, 1, true, true>(g, u, x0, S, Ls, &acc[0][0]);
+                    else if ((clipped >> v) & 1)
+                        walk_tile<ARITH, P, P, 1, true>(g, u, x0, S, Ls, &acc[0][0]);
+                    else
+                        walk_tile<ARITH, P, P, 1, false>(g, u, x0, S, Ls, &acc[0][0]);
+                } else {
+                    const float u = line_coord(cc, nh), x0 = (float)(rr - nh);
+                    const float* Ls = &sLs[v][P * tx];
+                    if ((multi >> v) & 1)
+                        walk_tile<ARITH, P, 1, P, true, true>(g, u, x0, S, Ls, &acc[0][0]);
+                    else if ((clipped >> v) & 1)
+                        walk_tile<ARITH, P, 1, P, true>(g, u, x0, S, Ls, &acc[0][0]);
+                    else
+                        walk_tile<ARITH, P, 1, P, false>(g, u, x0, S, Ls, &acc[0][0]);
+                }
+                continue;
+            }
+            const int kind = geom[v0 + v].kind;
             const float* S = &sS[v][0] - sLo[v];
-            if (g.kind == DD_SWEEP_ROWS) {
-                if (g.multi) {
-#pragma unroll
-                    for (int i = 0; i < P; ++i)
-                        walk_line<ARITH, P, 1, true>(g, npix, nh,
-                                                     key_K<ARITH>(g, line_coord(rr + i, nh)),
-                                                     sLs[v][P * ty + i], cc, S, &acc[i][0]);
-                } else {
-#pragma unroll
-                    for (int i = 0; i < P; ++i)
-                        walk_line<ARITH, P, 1, false>(g, npix, nh,
-                                                      key_K<ARITH>(g, line_coord(rr + i, nh)),
-                                                      sLs[v][P * ty + i], cc, S, &acc[i][0]);
-                }
-            } else if (g.kind == DD_SWEEP_COLS) {
-                if (g.multi) {
-#pragma unroll
-                    for (int j = 0; j < P; ++j)
-                        walk_line<ARITH, P, P, true>(g, npix, nh,
-                                                     key_K<ARITH>(g, line_coord(cc + j, nh)),
-                                                     sLs[v][P * tx + j], rr, S, &acc[0][j]);
-                } else {
-#pragma unroll
-                    for (int j = 0; j < P; ++j)
-                        walk_line<ARITH, P, P, false>(g, npix, nh,
-                                                      key_K<ARITH>(g, line_coord(cc + j, nh)),
-                                                      sLs[v][P * tx + j], rr, S, &acc[0][j]);
-                }
-            } else if (g.kind == DD_ROWSUM) {
+            if (kind == DD_ROWSUM) {
 #pragma unroll
                 for (int i = 0; i < P; ++i) {
                     const float sv = (rr + i < npix) ? S[rr + i] : 0.0f;
 #pragma unroll
                     for (int j = 0; j < P; ++j) acc[i][j] = __fadd_rn(acc[i][j], sv);
                 }
-            } else if (g.kind == DD_COLSUM) {
+            } else if (kind == DD_COLSUM) {
 #pragma unroll
                 for (int j = 0; j < P; ++j) {
                     const float sv = (cc + j < npix) ? S[cc + j] : 0.0f;

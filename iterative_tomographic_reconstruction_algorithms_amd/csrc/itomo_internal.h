@@ -97,7 +97,7 @@ struct Plan {
     hipStream_t aux_stream;
     hipEvent_t ev_fork, ev_join;
     int fwd_var;     // distance-driven launch shapes (kFwdBins / kBackTiles index)
-    int back_var;
+    int back_var;    // kBackAuto: chosen per launch (back_variant)
     int method;      // pixel-driven: 0 nearest bin, 1 linear split (radon_pd.c:57-85)
     // Device scratch owned by the plan (FP64 partial sums, ray-driven back-projection
     // image).  Grown on first use; a plan must not be used from two streams at once.
@@ -141,10 +141,10 @@ int plan_scratch(const Plan& p, size_t bytes, void** ptr, hipStream_t st);
 //   back:    kBackTiles[v] = {T, P}: T x T pixel tile per block, P x P per thread.
 constexpr int kNumFwdVariants = 3;
 constexpr int kFwdBins[kNumFwdVariants] = {256, 128, 64};
-constexpr int kNumBackVariants = 3;
-constexpr int kBackTiles[kNumBackVariants][2] = {{64, 4}, {32, 2}, {32, 4}};
+constexpr int kNumBackVariants = 4;
+constexpr int kBackTiles[kNumBackVariants][2] = {{64, 4}, {32, 2}, {32, 4}, {16, 1}};
 constexpr int kDdFwdBlock = 256;            // default forward shape
-constexpr int kDdBackTile = 64;             // default back tile (also the batch's)
+constexpr int kBackAuto = -1;
 constexpr int kRdBlock = 64;
 constexpr int kEpiChunk = 256 * 8;          // pixels per elementwise-epilogue block
 
@@ -163,6 +163,27 @@ inline size_t dd_back_blocks(int npix, int tile)
     return t * t;
 }
 
+// Back tile for `pixels` pixels in a launch (npix^2 x slices, rounded up to tiles): the
+// largest that still gives the 256 compute units blocks enough.  A wave alone on its SIMD
+// issues about every 8th cycle, four together about every 2nd, so 64 x 64 tiles (1.6 times
+// the work per instruction of single pixels) pay from 3 blocks of 4 waves per compute unit,
+// 32 x 32 tiles from 1.5.  64/32/16 tiles, in us: 363^2 x 251 207/96/57, 363^2 x 3 slices
+// 202/100/88, 512^2 x 360 288/137/92, 724^2 x 512 406/223/221, 1024^2 x 720 578/360/507,
+// 1448^2 x 900 1010/850/1181, 1024^2 x 900 x 4 slices 1287/1437/2235, 2048^2 x 1800
+// 2500/2970/4434.
+inline int back_variant_for(size_t tiles64, size_t tiles32)
+{
+    if (tiles64 >= 768) return 0;
+    return tiles32 >= 384 ? 1 : 3;
+}
+
+inline int back_variant(const Plan& p, int nslices)
+{
+    if (p.back_var != kBackAuto) return p.back_var;
+    return back_variant_for(dd_back_blocks(p.npix, 64) * nslices,
+                            dd_back_blocks(p.npix, 32) * nslices);
+}
+
 inline size_t fwd_blocks_per_slice(const Plan& p)
 {
     if (p.projector == ITOMO_PROJ_DD) return dd_fwd_slots(p.npix, p.nang);
@@ -178,10 +199,10 @@ inline size_t pd_back_blocks(int npix)
     return (size_t)((npix + 63) / 64) * (size_t)((npix + 3) / 4);
 }
 
-inline size_t back_blocks_per_slice(const Plan& p)
+inline size_t back_blocks_per_slice(const Plan& p, int nslices)
 {
     const size_t n2 = (size_t)p.npix * p.npix;
-    if (p.projector == ITOMO_PROJ_DD) return dd_back_blocks(p.npix, kBackTiles[p.back_var][0]);
+    if (p.projector == ITOMO_PROJ_DD) return dd_back_blocks(p.npix, kBackTiles[back_variant(p, nslices)][0]);
     if (p.projector == ITOMO_PROJ_PD || p.projector == ITOMO_PROJ_SS)
         return pd_back_blocks(p.npix);
     return (n2 + kEpiChunk - 1) / kEpiChunk;

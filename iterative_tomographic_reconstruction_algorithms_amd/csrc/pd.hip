@@ -349,7 +349,7 @@ int pd_forward_epi(const Plan& p, int epi, int ones, const float* image, float* 
 int pd_back_epi(const Plan& p, int epi, int ones, const float* sino, float* out, int nslices,
                 int accumulate, const EpiArgs& e, hipStream_t st, int* blocks_per_slice)
 {
-    const int bps = (int)back_blocks_per_slice(p);
+    const int bps = (int)back_blocks_per_slice(p, nslices);
     if (blocks_per_slice) *blocks_per_slice = bps;
     EpiArgs ee = e;
     ee.blocks_per_slice = bps;

@@ -254,7 +254,7 @@ ScratchLayout scratch_layout(const Plan& p, int nslices)
     const size_t nxt = n2 * ns;
     const size_t nf = fwd_blocks_per_slice(p) * 3 * ns;
     // back partials also serve the elementwise SPS update (one slot per kEpiChunk pixels)
-    const size_t nbb = back_blocks_per_slice(p), nbe = (n2 + kEpiChunk - 1) / kEpiChunk;
+    const size_t nbb = back_blocks_per_slice(p, nslices), nbe = (n2 + kEpiChunk - 1) / kEpiChunk;
     const size_t nb = (nbb > nbe ? nbb : nbe) * 3 * ns;
     const size_t ni = p.projector == ITOMO_PROJ_RD ? n2 * ns : 0;
     auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
@@ -337,6 +337,7 @@ static int plan_create(itomo_plan** out, int projector, int npix, const float* a
     p->nang = nang;
     p->arith = arith;
     p->method = method;
+    if (projector == ITOMO_PROJ_DD) p->back_var = kBackAuto;
     size_t bytes = 0;
     int st = ITOMO_OK;
     if (projector == ITOMO_PROJ_DD) {
@@ -510,7 +511,7 @@ int itomo_plan_get_shapes(const itomo_plan* p, int* fwd_variant, int* back_varia
     if (!p || !fwd_variant || !back_variant)
         return set_error(ITOMO_EINVAL, "plan_get_shapes: null pointer");
     *fwd_variant = p->fwd_var;
-    *back_variant = p->back_var;
+    *back_variant = itomo::back_variant(*p, 1);
     return ITOMO_OK;
 }
 
