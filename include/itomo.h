@@ -124,7 +124,7 @@ int itomo_plan_trig(const itomo_plan *plan, float *s_host, float *c_host);
  * C has no launch shapes; used by the autotuner).  Forward variant f in
  * [0, ITOMO_FWD_VARIANTS): 256 / 128 / 64 bins per block.  Back variant b in
  * [0, ITOMO_BACK_VARIANTS): 64x64 tile with 4x4 pixels per thread / 32x32 with 2x2 /
- * 32x32 with 4x4 / 16x16 with one.  A plan starts with 256 bins and a back tile chosen per
+ * 32x32 with 4x4 / 16x16 with one.  A plan starts with 64 bins and a back tile chosen per
  * call from the number of pixels in it (get_shapes reports the choice for one slice).
  * Every shape produces bit-identical projections and iterates; FP64
  * monitor sums follow the block partition and may differ in the last bits.

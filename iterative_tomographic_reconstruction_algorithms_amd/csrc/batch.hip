@@ -87,10 +87,11 @@ __device__ __forceinline__ int next_item(int* counter)
     return it;
 }
 
-// Five waves per SIMD (96 registers, three of them spilled): the kernel holds every
-// forward path and the fused update, and left to itself the compiler takes 129
-// registers, room for three waves.  Measured on the 1024^2 x 900 stack: 69.0 ms per
-// iteration at four waves, 63.9 at five, 70.7 at six (18 registers spilled).
+// Five waves per SIMD (96 registers): the kernel holds every forward path and the fused
+// update.  Measured on 16 slices of 1024^2 x 900 (forward and back): 14.68 ms per iteration at
+// four waves, 14.47 at five, 15.03 at six, 16.23 at eight.  PATH: kFwdSmall up to kFwdBigWaves
+// items, kFwdMixed beyond, as the per-plan launches choose.
+template <int PATH>
 __global__ void __launch_bounds__(kBatchFwdBlock) __attribute__((amdgpu_waves_per_eu(5)))
 batch_fwd_kernel(const BatchMember* __restrict__ mem, const BatchItem* __restrict__ items,
                  int nitems, int* counter)
@@ -105,7 +106,7 @@ batch_fwd_kernel(const BatchMember* __restrict__ mem, const BatchItem* __restric
         e.w = m.R;
         e.partials = m.pf;
         e.blocks_per_slice = m.bps_f;
-        dd_fwd_block<ITOMO_ARITH_FAST, EPI_SIRT_FWD, false, kBatchFwdBlock>(
+        dd_fwd_block<ITOMO_ARITH_FAST, EPI_SIRT_FWD, false, kBatchFwdBlock, PATH>(
             m.geom, m.lstar, m.nang, m.npix, m.x, m.xT, m.work, (int64_t)m.npix * m.npix,
             (int64_t)m.nang * m.npix, 0, e, w.a, w.b, w.z);
     }
@@ -318,8 +319,13 @@ int itomo_batch_sirt_iterate(itomo_batch* B, float pc_beta, void* stream)
         transpose_kernel_b<<<tg, tb, 0, st>>>(bm.x, bm.xT, bm.npix, (int64_t)bm.npix * bm.npix);
     }
     reset_counter_kernel<<<1, 1, 0, st>>>(B->d_counter);
-    batch_fwd_kernel<<<std::min(B->grid * (256 / kBatchFwdBlock), B->nfwd), kBatchFwdBlock, 0,
-                       st>>>(B->d_members, B->d_fwd, B->nfwd, B->d_counter);
+    const int fgrid = std::min(B->grid * (256 / kBatchFwdBlock), B->nfwd);
+    if (B->nfwd <= kFwdBigWaves)
+        batch_fwd_kernel<kFwdSmall><<<fgrid, kBatchFwdBlock, 0, st>>>(B->d_members, B->d_fwd,
+                                                                      B->nfwd, B->d_counter);
+    else
+        batch_fwd_kernel<kFwdMixed><<<fgrid, kBatchFwdBlock, 0, st>>>(B->d_members, B->d_fwd,
+                                                                      B->nfwd, B->d_counter);
     const int bgrid = std::min(B->grid, B->nback);
     if (B->back_var == 0)
         batch_back_kernel<64, 4><<<bgrid, 256, 0, st>>>(B->d_members, B->d_back, B->nback,

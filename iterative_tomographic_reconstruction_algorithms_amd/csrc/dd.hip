@@ -21,7 +21,6 @@
 // epilogue.h), with FP64 partial sums reduced per block in a fixed order.
 #include <vector>
 
-
 #include "dd_device.h"
 
 namespace itomo {
@@ -88,61 +87,44 @@ void launch_fwd_path(const Plan& p, const float* image, const float* imageT, flo
                      int nslices, int accumulate, const EpiArgs& e, const int* views,
                      int nviews, hipStream_t st)
 {
+    if (nviews == 0) return;
     dim3 block(B), grid((p.npix + B - 1) / B, nviews, nslices);
     dd_fwd_kernel<ARITH, EPI, ONES, B, PATH><<<grid, block, 0, st>>>(
         (const DdView*)p.d_geom, p.d_lstar, p.nang, p.npix, image, imageT, out,
         (int64_t)p.npix * p.npix, (int64_t)p.nang * p.npix, accumulate, e, views);
 }
 
-// Views with more than 8 candidate pixels per bin and line go to a launch of their own
-// (see kPathMain); with unit input, one launch takes every view.  The wide launch is small
-// (a tenth of the views at 2048^2 x 1800) and its blocks are long, so on its own it
-// leaves most of the GPU idle: it runs on the plan's second stream beside the main launch
-// (both write disjoint sinogram rows), forked from and joined back into `st`.  It always
-// uses 64-bin blocks: a block walks every line any of its bins meets, and a wide view's
-// bins meet few lines each (about npix / w of them for bins w pixels wide, against
-// npix / w + B for a block), so wider blocks only add lines that weigh zero.
+// One launch for small problems and unit input, two for large ones (kFwdBigWaves); the
+// diagonal views always run in 64-bin blocks there.
 template <int ARITH, int EPI, bool ONES, int B>
-int launch_fwd_b(const Plan& p, const float* image, const float* imageT, float* out,
-                 int nslices, int accumulate, const EpiArgs& e, hipStream_t st)
+void launch_fwd_b(const Plan& p, const float* image, const float* imageT, float* out,
+                  int nslices, int accumulate, const EpiArgs& e, hipStream_t st)
 {
-    if (ONES || !p.d_vlist || p.n_gather == 0) {
-        launch_fwd_path<ARITH, EPI, ONES, B, kPathAll>(p, image, imageT, out, nslices,
-                                                       accumulate, e, nullptr, p.nang, st);
-        return ITOMO_OK;
+    const int64_t waves = (int64_t)((p.npix + 63) / 64) * p.nang * nslices;
+    if (ONES || waves <= kFwdBigWaves) {
+        launch_fwd_path<ARITH, EPI, ONES, B, kFwdSmall>(p, image, imageT, out, nslices,
+                                                        accumulate, e, nullptr, p.nang, st);
+        return;
     }
-    hipStream_t wide_st = st;
-    if (p.n_staged > 0 && p.aux_stream) {
-        int rc = check_hip(hipEventRecord(p.ev_fork, st), "dd forward: fork");
-        if (!rc) rc = check_hip(hipStreamWaitEvent(p.aux_stream, p.ev_fork, 0), "dd forward: fork");
-        if (rc) return rc;
-        wide_st = p.aux_stream;
+    if constexpr (!ONES) {
+        launch_fwd_path<ARITH, EPI, ONES, 64, kFwdDiag>(p, image, imageT, out, nslices,
+                                                        accumulate, e, p.d_vlist + p.n_staged,
+                                                        p.nang - p.n_staged, st);
+        launch_fwd_path<ARITH, EPI, ONES, B, kFwdStaged>(p, image, imageT, out, nslices,
+                                                         accumulate, e, p.d_vlist, p.n_staged,
+                                                         st);
     }
-    // the main launch is issued first: the wide launch's long blocks then take the slots
-    // the main launch's blocks leave, rather than holding slots from its start
-    if (p.n_staged > 0)
-        launch_fwd_path<ARITH, EPI, ONES, B, kPathMain>(p, image, imageT, out, nslices,
-                                                        accumulate, e, p.d_vlist, p.n_staged, st);
-    launch_fwd_path<ARITH, EPI, ONES, 64, kPathWide>(p, image, imageT, out, nslices, accumulate,
-                                                     e, p.d_vlist + p.n_staged, p.n_gather,
-                                                     wide_st);
-    if (wide_st != st) {
-        int rc = check_hip(hipEventRecord(p.ev_join, wide_st), "dd forward: join");
-        if (!rc) rc = check_hip(hipStreamWaitEvent(st, p.ev_join, 0), "dd forward: join");
-        if (rc) return rc;
-    }
-    return ITOMO_OK;
 }
 
 template <int ARITH, int EPI, bool ONES>
-int launch_fwd(const Plan& p, const float* image, const float* imageT, float* out,
+void launch_fwd(const Plan& p, const float* image, const float* imageT, float* out,
                int nslices, int accumulate, const EpiArgs& e, hipStream_t st)
 {
     static_assert(kFwdBins[0] == 256 && kFwdBins[1] == 128 && kFwdBins[2] == 64, "variants");
     switch (p.fwd_var) {
-    case 1: return launch_fwd_b<ARITH, EPI, ONES, 128>(p, image, imageT, out, nslices, accumulate, e, st);
-    case 2: return launch_fwd_b<ARITH, EPI, ONES, 64>(p, image, imageT, out, nslices, accumulate, e, st);
-    default: return launch_fwd_b<ARITH, EPI, ONES, 256>(p, image, imageT, out, nslices, accumulate, e, st);
+    case 1: launch_fwd_b<ARITH, EPI, ONES, 128>(p, image, imageT, out, nslices, accumulate, e, st); break;
+    case 2: launch_fwd_b<ARITH, EPI, ONES, 64>(p, image, imageT, out, nslices, accumulate, e, st); break;
+    default: launch_fwd_b<ARITH, EPI, ONES, 256>(p, image, imageT, out, nslices, accumulate, e, st); break;
     }
 }
 
@@ -178,12 +160,15 @@ int dispatch_fwd(const Plan& p, int epi, int ones, const float* image, const flo
 {
     switch (epi) {
     case EPI_STORE:
-        if (ones) return launch_fwd<ARITH, EPI_STORE, true>(p, image, imageT, out, nslices, accumulate, e, st);
-        return launch_fwd<ARITH, EPI_STORE, false>(p, image, imageT, out, nslices, accumulate, e, st);
+        if (ones) launch_fwd<ARITH, EPI_STORE, true>(p, image, imageT, out, nslices, accumulate, e, st);
+        else launch_fwd<ARITH, EPI_STORE, false>(p, image, imageT, out, nslices, accumulate, e, st);
+        return ITOMO_OK;
     case EPI_RECIP:
-        return launch_fwd<ARITH, EPI_RECIP, true>(p, image, imageT, out, nslices, 0, e, st);
+        launch_fwd<ARITH, EPI_RECIP, true>(p, image, imageT, out, nslices, 0, e, st);
+        return ITOMO_OK;
     case EPI_MLEM_FWD:
-        return launch_fwd<ARITH, EPI_MLEM_FWD, false>(p, image, imageT, out, nslices, 0, e, st);
+        launch_fwd<ARITH, EPI_MLEM_FWD, false>(p, image, imageT, out, nslices, 0, e, st);
+        return ITOMO_OK;
     }
     return set_error(ITOMO_EINVAL, "dd forward: unsupported epilogue %d", epi);
 }
@@ -287,16 +272,15 @@ int dd_build_view_lists(Plan& p)
     const DdView* g = (const DdView*)p.h_geom;
     std::vector<int> v;
     v.reserve(p.nang);
-    auto wide = [&](int k) {
+    auto diag = [&](int k) {
         return (g[k].kind == DD_SWEEP_ROWS || g[k].kind == DD_SWEEP_COLS) &&
-               g[k].ncand > kFwdMainMaxCand;
+               g[k].ncand > kFwdStagedMaxCand;
     };
     for (int k = 0; k < p.nang; ++k)
-        if (!wide(k)) v.push_back(k);
+        if (!diag(k)) v.push_back(k);
     p.n_staged = (int)v.size();
     for (int k = 0; k < p.nang; ++k)
-        if (wide(k)) v.push_back(k);
-    p.n_gather = p.nang - p.n_staged;
+        if (diag(k)) v.push_back(k);
     int rc = check_hip(hipMalloc(&p.d_vlist, (size_t)p.nang * sizeof(int)), "plan_create: hipMalloc");
     if (rc) return rc;
     return check_hip(hipMemcpy(p.d_vlist, v.data(), (size_t)p.nang * sizeof(int),

@@ -538,33 +538,6 @@ __device__ __forceinline__ float4 load_px4(__amdgpu_buffer_rsrc_t rs, int idx)
                        __int_as_float(v[3]));
 }
 
-// v[0 .. NC) = image[idx .. idx+NC) of one slice (total pixels; out of range: 0), idx >= 0,
-// with 16-byte loads: a bin's candidates on one line are consecutive pixels, so one load
-// instruction fetches four of them.  A run that reaches the end of the slice is read
-// element by element.
-template <int NC>
-__device__ __forceinline__ void load_run(__amdgpu_buffer_rsrc_t rs, int idx, int total,
-                                         float* v)
-{
-#pragma unroll
-    for (int k4 = 0; k4 < NC; k4 += 4) {
-        const int i = idx + k4;
-        float4 f;
-        if (i + 3 < total) {
-            f = load_px4(rs, i);
-        } else {
-            f.x = load_px(rs, i);
-            f.y = load_px(rs, i + 1);
-            f.z = load_px(rs, i + 2);
-            f.w = load_px(rs, i + 3);
-        }
-        v[k4] = f.x;
-        if (k4 + 1 < NC) v[k4 + 1] = f.y;
-        if (k4 + 2 < NC) v[k4 + 2] = f.z;
-        if (k4 + 3 < NC) v[k4 + 3] = f.w;
-    }
-}
-
 // One candidate pixel of a bin [Dlo, Dhi] on a line with offset K: the pixel spans
 // [x-K, x+1-K].  Dhc is the bin's right end clipped to the line's L*.  Advances x.
 // The first candidate (Rp = x-K, its left end, on entry) can start left of Dlo and gets
@@ -616,81 +589,161 @@ __device__ __forceinline__ float first_pixel_near(float Dlo, float Dlh, float K,
     return __builtin_amdgcn_fmed3f(fe, (float)(-nh), (float)(npix - 1 - nh));
 }
 
-constexpr int kFwdLines = 4;   // lines whose gathers are in flight together
-
-// Most candidate pixels per bin and line of a view in the main forward launch; wider
-// views run in a launch of their own and read their candidates with 16-byte loads.
-constexpr int kFwdMainMaxCand = 8;
-
-// Gather-form forward of one bin over lines [i_lo, i_hi] for views with at most NC
-// candidate pixels per bin and line, GL lines per group (see dd_fwd_block).
-template <int ARITH, bool ONES, int NC, int GL>
-__device__ __forceinline__ float fwd_grouped(const __amdgpu_buffer_rsrc_t rs, const DdView& g,
-                                             const float* __restrict__ ls, int i_lo, int i_hi,
-                                             int npix, int nh, float Dlo, float Dhi,
-                                             bool last_bin, float acc)
+// Forward projection of unit pixels: one bin over its own lines [i_lo, i_hi], at most NC
+// candidate pixels per line (0: g.ncand of them).
+template <int ARITH, int NC>
+__device__ __forceinline__ float fwd_ones(const DdView& g, const float* __restrict__ ls,
+                                          int i_lo, int i_hi, int npix, int nh, float Dlo,
+                                          float Dhi, bool last_bin, float acc)
 {
     const float xNm1 = (float)(npix - 1 - nh);
     const float Dlh = __fadd_rn(Dlo, 0.5f);
     float u = line_coord(i_lo, nh);
-    int lbase = i_lo * npix;
-    int i = i_lo;
-    for (; i + GL - 1 <= i_hi; i += GL) {
-        float K[GL], xq[GL], v[GL][NC];
-#pragma unroll
-        for (int l = 0; l < GL; ++l) {
-            K[l] = key_K<ARITH>(g, u);
-            u = __fadd_rn(u, 1.0f);
-            xq[l] = first_pixel_near(Dlo, Dlh, K[l], nh, npix);
-            const int q = (int)xq[l] + nh;
-            if (ONES || NC <= kFwdMainMaxCand) {
-#pragma unroll
-                for (int k = 0; k < NC; ++k) v[l][k] = ONES ? 1.0f : load_px(rs, lbase + q + k);
-            } else {
-                load_run<NC>(rs, lbase + q, npix * npix, v[l]);
-            }
-            lbase += npix;
-        }
-#pragma unroll
-        for (int l = 0; l < GL; ++l) {
-            float Dhc = Dhi;
-            if (last_bin || Dhi > __fsub_rn(xNm1, K[l])) Dhc = fminf(Dhi, ls[i + l]);
-            float xk = xq[l], Rp = __fsub_rn(xq[l], K[l]);
-#pragma unroll
-            for (int k = 0; k < NC; ++k)
-                acc = cand_step<ARITH>(k == 0, xk, Rp, K[l], Dlo, Dhc, v[l][k], acc);
-        }
-    }
-    for (; i <= i_hi; ++i, u = __fadd_rn(u, 1.0f), lbase += npix) {
+    for (int i = i_lo; i <= i_hi; ++i, u = __fadd_rn(u, 1.0f)) {
         const float K = key_K<ARITH>(g, u);
-        const float x = first_pixel_near(Dlo, Dlh, K, nh, npix);
-        const int q = (int)x + nh;
+        float x = NC ? first_pixel_near(Dlo, Dlh, K, nh, npix) : first_pixel(Dlo, K, nh, npix);
         float Dhc = Dhi;
         if (last_bin || Dhi > __fsub_rn(xNm1, K)) Dhc = fminf(Dhi, ls[i]);
-        float v[NC];
-        if (ONES || NC <= kFwdMainMaxCand) {
+        float Rp = __fsub_rn(x, K);
+        if (NC) {
 #pragma unroll
-            for (int k = 0; k < NC; ++k) v[k] = ONES ? 1.0f : load_px(rs, lbase + q + k);
+            for (int k = 0; k < NC; ++k)
+                acc = cand_step<ARITH>(k == 0, x, Rp, K, Dlo, Dhc, 1.0f, acc);
         } else {
-            load_run<NC>(rs, lbase + q, npix * npix, v);
+            for (int k = 0; k < g.ncand; ++k)
+                acc = cand_step<ARITH>(k == 0, x, Rp, K, Dlo, Dhc, 1.0f, acc);
         }
-        float xk = x, Rp = __fsub_rn(x, K);
+    }
+    return acc;
+}
+
+// Forward projection of one sweep view with wide bins (w = |rinv| pixels, at most NC
+// candidates per bin and line, NC = 0: g.ncand of them), along diagonals.
+//
+// A bin w pixels wide meets only about npix/w lines, and the next bin's lines start
+// |1/cos| or |1/sin| (between 1 and sqrt(2) for w >= sqrt(2), towards 1 as w grows) lines
+// further on.  So the 64 lanes of a wave, 64 consecutive bins, step together along
+// diagonals: in step k lane d takes line L(d) + k, where L(d) is its own first line.  Every
+// step then serves all lanes (a block that walks the union of its bins' lines, as the
+// staged path does, spends npix/w + 64 line steps where npix/w are needed; staged, the wide
+// views alone took 94 us at 64^2 x 45 where the whole forward now takes 16), and the lanes' first pixels on their lines agree to within a line's shift.
+// Hence candidate j of the wave lies in 64 neighbouring lines at nearly the same place
+// along the line: `img` is the orientation in which neighbouring lines are neighbours in
+// memory (the transpose of what the staged path reads), and candidate j of the whole wave
+// is one nearly contiguous load.  No LDS, no barriers; bounds: vector L1 accesses (one
+// 4-byte load per candidate and lane) and the five VALU operations of a candidate.
+//
+// Lines outside the image (a lane's diagonal before its first or after its last line) load
+// nothing and get the right end -1e30, which makes every weight 0.  Away from the end of
+// the line (q + NC < npix for every lane) the candidates need no bounds check and L* does
+// not clip (see dd_fwd_block); the last bin of a view always takes the checked form.
+template <int ARITH, int NC, int GL>
+__device__ __forceinline__ float fwd_diag(const DdView& g, const float* __restrict__ ls,
+                                          int npix, int nh, const float* __restrict__ img,
+                                          int d, float acc)
+{
+    constexpr float kNone = -1e30f;
+    const __amdgpu_buffer_rsrc_t rs = image_rsrc(img, npix);
+    const int dk = min(d, npix - 1);
+    const float Dlo = key_D<ARITH>(g, dk - nh);
+    const float Dhi = key_D<ARITH>(g, dk + 1 - nh);
+    const float Dlh = __fadd_rn(Dlo, 0.5f);
+    const bool last_bin = dk == npix - 1;
+    // Lines whose pixel span [x0 - K, xN - K] meets [Dlo, Dhi]: K_i = (i - nh + 1/2) t lies
+    // between x0 - Dhi and xN - Dlo, a range of (npix + w)/|t| lines; a sixteenth of a line
+    // of margin at each end covers every rounding of a key (below 0.01 lines, npix <= 32766).
+    const double rt = 1.0 / (double)g.t;
+    const double e0 = ((double)(-nh) - (double)Dhi) * rt;
+    const double e1 = ((double)(npix - nh) - (double)Dlo) * rt;
+    const int L = (int)floor(fmin(e0, e1) + ((double)nh - 0.5625)) + 1;
+    const int steps = (int)floor(((double)npix + (double)g.rinv) * fabs(rt) + 0.14) + 1;
+    // L is monotonic in the bin: its extremes are in the first and the last lane
+    const int La = __builtin_amdgcn_readlane(L, 0), Lb = __builtin_amdgcn_readlane(L, 63);
+    const int k0 = max(0, -max(La, Lb));
+    const int k1 = min(steps - 1, npix - 1 - min(La, Lb));
+    const int stride = npix * 4;
+    if constexpr (NC > 0) {
+        for (int k = k0; k <= k1; k += GL) {
+            float K[GL], xq[GL], Dhc[GL], v[GL][NC];
+            int q[GL], vo[GL];
+            bool ok[GL];
+            bool edge = last_bin;
 #pragma unroll
-        for (int k = 0; k < NC; ++k)
-            acc = cand_step<ARITH>(k == 0, xk, Rp, K, Dlo, Dhc, v[k], acc);
+            for (int l = 0; l < GL; ++l) {
+                const int i = L + k + l;
+                ok[l] = (unsigned)i < (unsigned)npix;
+                K[l] = key_K<ARITH>(g, line_coord(i, nh));
+                xq[l] = first_pixel_near(Dlo, Dlh, K[l], nh, npix);
+                q[l] = (int)xq[l] + nh;
+                edge |= ok[l] && q[l] >= npix - NC;
+                vo[l] = ok[l] ? (int)((__umul24(q[l], npix) + (unsigned)i) * 4u) : -1;
+            }
+            if (!__any(edge)) {
+#pragma unroll
+                for (int l = 0; l < GL; ++l) {
+                    Dhc[l] = ok[l] ? Dhi : kNone;
+#pragma unroll
+                    for (int j = 0; j < NC; ++j)
+                        v[l][j] = __int_as_float((int)__builtin_amdgcn_raw_buffer_load_b32(
+                            rs, vo[l], j * stride, 0));
+                }
+            } else {
+#pragma unroll
+                for (int l = 0; l < GL; ++l) {
+                    Dhc[l] = ok[l] ? fminf(Dhi, ls[ok[l] ? L + k + l : 0]) : kNone;
+#pragma unroll
+                    for (int j = 0; j < NC; ++j)
+                        v[l][j] = __int_as_float((int)__builtin_amdgcn_raw_buffer_load_b32(
+                            rs, ok[l] && q[l] + j < npix ? vo[l] + j * stride : -1, 0, 0));
+                }
+            }
+#pragma unroll
+            for (int l = 0; l < GL; ++l) {
+                float xk = xq[l], Rp = __fsub_rn(xq[l], K[l]);
+#pragma unroll
+                for (int j = 0; j < NC; ++j)
+                    acc = cand_step<ARITH>(j == 0, xk, Rp, K[l], Dlo, Dhc[l], v[l][j], acc);
+            }
+        }
+    } else {
+        constexpr int CH = 16;   // candidates loaded together
+        for (int k = k0; k <= k1; ++k) {
+            const int i = L + k;
+            const bool ok = (unsigned)i < (unsigned)npix;
+            const float K = key_K<ARITH>(g, line_coord(i, nh));
+            const float x = first_pixel(Dlo, K, nh, npix);
+            const int q = (int)x + nh;
+            const int vo = ok ? (int)((__umul24(q, npix) + (unsigned)i) * 4u) : -1;
+            float Dhc = ok ? Dhi : kNone;
+            if (__any(last_bin || (ok && q >= npix - g.ncand)))
+                Dhc = ok ? fminf(Dhi, ls[ok ? i : 0]) : kNone;
+            float xk = x, Rp = __fsub_rn(x, K);
+            for (int j0 = 0; j0 < g.ncand; j0 += CH) {
+                float v[CH];
+                if (!__any(ok && q + j0 + CH > npix)) {
+#pragma unroll
+                    for (int j = 0; j < CH; ++j)
+                        v[j] = __int_as_float((int)__builtin_amdgcn_raw_buffer_load_b32(
+                            rs, vo, (j0 + j) * stride, 0));
+                } else {
+#pragma unroll
+                    for (int j = 0; j < CH; ++j)
+                        v[j] = __int_as_float((int)__builtin_amdgcn_raw_buffer_load_b32(
+                            rs, ok && q + j0 + j < npix ? vo + (j0 + j) * stride : -1, 0, 0));
+                }
+#pragma unroll
+                for (int j = 0; j < CH; ++j)
+                    acc = cand_step<ARITH>(j0 + j == 0, xk, Rp, K, Dlo, Dhc, v[j], acc);
+            }
+        }
     }
     return acc;
 }
 
 // LDS of the staged forward path: 16 floats per thread of the block (64 B bytes for B
-// threads, 4 KB per wave), shared by every candidate count; the launch of the widest
-// views, which runs alone, stages 32 floats per thread.
+// threads, 4 KB per wave), shared by every candidate count.
 template <int B>
 constexpr int fwd_stage_floats() { return 16 * B; }
-template <int B>
-constexpr int fwd_stage_floats_wide() { return 32 * B; }
-constexpr int kFwdStagedMaxCand = 6;  // views with more candidates take the gather path
-constexpr int kFwdStagedWideMaxCand = 32;
 constexpr int kFwdStageMaxLines = 8;
 
 // Pixels of the staged window beyond (NC-1)*B, so that it holds every candidate of a
@@ -703,25 +756,30 @@ constexpr int fwd_window_extra()
 
 // Forward projection of one sweep view with at most NC candidate pixels per bin and line
 // (bins narrower than w < NC - 1.25 pixels), for the B bins [bx*B, +B) of a block.
-// Lines are processed in chunks of FL: for each line of a chunk the block first copies
-// the window of W pixels its bins can touch into LDS with 16-byte loads (one contiguous
+// Lines are processed in chunks of FL: for each line of a chunk the block copies the
+// window of W pixels its bins can touch into LDS with 16-byte loads (one contiguous
 // row segment per line; the window starts at q0, the first bin's estimated first pixel
 // minus 2, rounded down to a multiple of 4), then every thread reads its candidates from
 // LDS.  A bin's first candidate lies less than B*w + 6 pixels past q0: less than
 // (B-1)*w + 1 + 5 for a bin that starts on the line, and for the last bin up to one bin
 // width more where it starts left of the line's first pixel and its first candidate is
 // clamped up to that pixel.  With W = (NC-1)*B + max(0, NC + 7 - B/4) >= B*w + 6 + NC
-// the window holds every candidate of every bin that meets the line (offsets are
-// clamped into it all the same; a bin that misses the line weights all its candidates
-// by zero).  Lines run over the union of the block's per-bin line ranges; lines that
-// miss a bin add nothing to it.  Every thread of the block takes part (inactive
-// threads, past the last bin, compute a copy of the last bin and store nothing).
-// sImg holds FLOATS floats; sQ0, sQb and sL kFwdStageMaxLines entries.
+// the window holds every candidate of every bin that meets the line.  q0 itself is kept in
+// [-(W - NC), npix - 1], which moves it only on lines that every bin of the block misses, so
+// that each first candidate, clamped into the line, lies in the window, whatever the bin.
+// Lines run over the union of the block's per-bin line ranges; lines that
+// miss a bin add nothing to it.  A chunk always runs all its FL lines (straight-line code, so
+// the LDS reads of one line hide behind the sums of another): those past the image get the
+// line end kNoLine, which makes every weight 0.  Every thread of the block takes part
+// (inactive threads, past the last bin, compute a copy of the last bin and store nothing).
+// sImg holds FLOATS floats, sMeta kFwdStageMaxLines entries {byte offset of pixel 0, L*}.
+constexpr float kNoLine = -1e30f;
+
 template <int ARITH, int B, int NC, int FLOATS>
 __device__ __forceinline__ float fwd_staged(const DdView& g, const float* __restrict__ ls,
                                             int npix, int nh, __amdgpu_buffer_rsrc_t rs,
-                                            int bx, int d, float acc, float* sImg, int* sQ0,
-                                            int* sQb, float* sL)
+                                            int bx, int d, float acc, float* sImg,
+                                            float2* sMeta)
 {
     constexpr int W = (NC - 1) * B + fwd_window_extra<B, NC>();
     constexpr int FL = FLOATS / W < kFwdStageMaxLines ? FLOATS / W : kFwdStageMaxLines;
@@ -737,99 +795,119 @@ __device__ __forceinline__ float fwd_staged(const DdView& g, const float* __rest
     const float D0lo = key_D<ARITH>(g, d0 - nh);
     const float D1hi = key_D<ARITH>(g, d1 + 1 - nh);
     const float x0 = (float)(-nh), xN = (float)(npix - nh);
-    double ua = ((double)x0 - (double)D1hi) / (double)g.t;
-    double ub = ((double)xN - (double)D0lo) / (double)g.t;
+    const double rt = 1.0 / (double)g.t;
+    double ua = ((double)x0 - (double)D1hi) * rt;
+    double ub = ((double)xN - (double)D0lo) * rt;
     if (ua > ub) { const double tmp = ua; ua = ub; ub = tmp; }
     ua = fmin(fmax(ua + nh - 0.5, -4.0), (double)npix + 4.0);
     ub = fmin(fmax(ub + nh - 0.5, -4.0), (double)npix + 4.0);
     const int i_lo = max(0, (int)floor(ua) - 2);
     const int i_hi = min(npix - 1, (int)ceil(ub) + 2);
-    float u = line_coord(i_lo, nh);
-    for (int c0 = i_lo; c0 <= i_hi; c0 += FL) {
-        const int ncl = min(FL, i_hi - c0 + 1);
-        __syncthreads();  // the previous chunk is consumed
-        if (tid < ncl) {
-            const float K = key_K<ARITH>(g, line_coord(c0 + tid, nh));
-            const float est = fminf(fmaxf(floorf(__fadd_rn(D0lo, K)), (float)(-nh - W)),
-                                    (float)(npix - nh + W));
-            const int q0 = ((int)est + nh - 2) & ~3;
-            sQ0[tid] = q0;
-            sQb[tid] = 4 * (nh - q0 + tid * W);   // byte offset of pixel 0 in sImg
-            sL[tid] = ls[c0 + tid];
-        }
-        __syncthreads();
-        // every thread loads its window pieces into registers first, then stores them:
-        // the loads of one chunk are all in flight together
-        float4 v[PER];
+    const int total = npix * npix;
+
+    float4 v[PER];
+    float2 meta;
+    // First pixel of the window of line i.
+    auto start = [&](int i) {
+        const int q = (int)floorf(__fadd_rn(D0lo, key_K<ARITH>(g, line_coord(i, nh)))) + nh - 2;
+        return min(max(q, -((W - NC) & ~3)), npix - 1) & ~3;
+    };
+    // Every load of a chunk is in flight before any is stored.  A window that starts left of
+    // the row gets zeros there; past the row's end it holds the next row, never weighted;
+    // outside the slice the loads return 0.
+    auto load = [&](int c0) {
+        // a piece may straddle the slice's end (the last window ends before this index)
+        const bool ragged = (npix & 3) && (c0 + FL + 1) * npix + W >= total;
 #pragma unroll
         for (int r = 0; r < PER; ++r) {
             const int k = tid + r * B;
             const int l = k / (W / 4), j4 = k - l * (W / 4);
-            v[r] = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (k < N4 && l < ncl) {
-                const int q = sQ0[l] + 4 * j4;
-                // a window that starts left of the row reads zeros there (negative index
-                // -> out of range); past the row's end it reads the next row: never
-                // weighted
-                const int idx = (c0 + l) * npix + q;
-                if (q >= 0 && idx + 3 < npix * npix) {
-                    v[r] = load_px4(rs, idx);
-                } else if (q >= 0) {  // straddles the end of the slice: per-element checks
-                    v[r].x = load_px(rs, idx);
-                    v[r].y = load_px(rs, idx + 1);
-                    v[r].z = load_px(rs, idx + 2);
-                    v[r].w = load_px(rs, idx + 3);
-                }
+            const int i = c0 + l;
+            const int q = start(i) + 4 * j4;
+            const int idx = i * npix + q;
+            const bool ok = (N4 % B == 0 || k < N4) && i < npix && q >= 0;
+            if (!ragged || !ok || idx + 3 < total) {
+                v[r] = load_px4(rs, ok ? idx : 0x3fffffff);
+            } else {
+                v[r].x = load_px(rs, idx);
+                v[r].y = load_px(rs, idx + 1);
+                v[r].z = load_px(rs, idx + 2);
+                v[r].w = load_px(rs, idx + 3);
             }
         }
+        const int i = c0 + tid;
+        if (tid < FL) {
+            meta.x = __int_as_float(4 * (nh - start(i) + tid * W));
+            meta.y = i < npix ? ls[i] : kNoLine;
+        }
+    };
+    auto store = [&]() {
 #pragma unroll
         for (int r = 0; r < PER; ++r) {
             const int k = tid + r * B;
-            const int l = k / (W / 4), j4 = k - l * (W / 4);
-            if (k < N4 && l < ncl) *(float4*)&sImg[l * W + 4 * j4] = v[r];
+            if (N4 % B == 0 || k < N4) *(float4*)&sImg[4 * k] = v[r];
         }
+        if (tid < FL) sMeta[tid] = meta;
+    };
+
+    for (int c0 = i_lo; c0 <= i_hi; c0 += FL) {
+        load(c0);
+        __syncthreads();  // the previous chunk is consumed
+        store();
         __syncthreads();
+        float Kp = 0.0f, xp = 0.0f, ep = 0.0f, pv[NC];
 #pragma unroll
-        for (int l = 0; l < FL; ++l) {
-            if (l < ncl) {
-                const float K = key_K<ARITH>(g, u);
-                const float x = first_pixel_near(Dlo, Dlh, K, nh, npix);
-                // byte offset of the first candidate in sImg, clamped into the line's window
-                const int ob = min(max(((int)x << 2) + sQb[l], 4 * l * W), 4 * (l * W + W - NC));
-                const float* wp = (const float*)((const char*)sImg + ob);
+        for (int l = 0; l <= FL; ++l) {
+            float K = 0.0f, x = 0.0f, e = 0.0f, val[NC];
+            if (l < FL) {
+                K = key_K<ARITH>(g, line_coord(c0 + l, nh));
+                x = first_pixel_near(Dlo, Dlh, K, nh, npix);
+                const float2 m = sMeta[l];
+                e = m.y;
+                const float* wp =
+                    (const float*)((const char*)sImg + (((int)x << 2) + __float_as_int(m.x)));
+#pragma unroll
+                for (int k = 0; k < NC; ++k) val[k] = wp[k];
+            }
+            if (l > 0) {
                 // clipping every weight's right end to L* is the exact rule; it changes
                 // only the weights that end at the line's dropped segment
-                const float Dhc = fminf(Dhi, sL[l]);
-                float xk = x, Rp = __fsub_rn(x, K);
+                const float Dhc = fminf(Dhi, ep);
+                float xk = xp, Rp = __fsub_rn(xp, Kp);
 #pragma unroll
                 for (int k = 0; k < NC; ++k)
-                    acc = cand_step<ARITH>(k == 0, xk, Rp, K, Dlo, Dhc, wp[k], acc);
+                    acc = cand_step<ARITH>(k == 0, xk, Rp, Kp, Dlo, Dhc, pv[k], acc);
             }
-            u = __fadd_rn(u, 1.0f);
+            Kp = K;
+            xp = x;
+            ep = e;
+#pragma unroll
+            for (int k = 0; k < NC; ++k) pv[k] = val[k];
         }
     }
     return acc;
 }
 
-// Forward projection: one thread per (bin, view blockIdx.y, slice blockIdx.z).
-// Lines are image rows for row sweeps and image columns for column sweeps; column
-// sweeps (and row sums) read the transposed image so that the lanes of a wave, which
-// hold consecutive bins, read consecutive addresses.
+// Which views a forward launch handles (block-uniform) and how.  Views with at most
+// fwd_staged_max(path) candidates are staged, the others go along diagonals.  A staged block
+// reads each line once through LDS, a diagonal one through the L1; staging wins for up to 6
+// candidates once the launch fills the GPU, the diagonals from 4 on while it does not (their
+// chains are shorter).  Staged up to 6 against up to 3, in us: 363^2 x 251 x 3 slices (4518
+// waves) 123 and 112, 724^2 x 512 (6144) 245 and 223, 1024^2 x 720 (11520) 531 and 525,
+// 1448^2 x 900 (20700) 1186 and 1364, 2048^2 x 1800 (57600) 4432 and 6014.  The line is drawn
+// at kFwdBigWaves.  A launch beyond it is split in two, each kernel with its own registers and
+// LDS: kFwdStaged and kFwdDiag; kFwdMixed holds both (the persistent batch).
+constexpr int kFwdSmall = 0, kFwdStaged = 1, kFwdDiag = 2, kFwdMixed = 3;
+constexpr int64_t kFwdBigWaves = 10240;
+constexpr int kFwdStagedMaxCand = 6;
+constexpr int fwd_staged_max(int path) { return path == kFwdSmall ? 3 : kFwdStagedMaxCand; }
+
+// Forward projection: one thread per (bin, view, slice).
+// Lines are image rows for row sweeps and image columns for column sweeps.  Each path reads
+// the image or its transpose, whichever makes the lanes of a wave, which hold consecutive
+// bins, read consecutive addresses.
 // Bins [bx*B, +B) of view `view`, slice z, one per thread; blk indexes the partials.
-// Which views a forward launch handles (block-uniform): all of them, the views with at
-// most kFwdMainMaxCand candidate pixels per bin and line (kPathMain), or the wider ones
-// (kPathWide).  The wide views' larger staging windows and deep load groups need LDS and
-// registers; compiled into a kernel of their own they leave the main kernel's occupancy
-// alone.
-constexpr int kPathAll = 0, kPathMain = 1, kPathWide = 2;
-
-// Whether the grouped gather with NC candidates is compiled into launch PATH.
-constexpr bool fwd_in_path(int path, int nc)
-{
-    return path == kPathAll || ((path == kPathMain) == (nc <= kFwdMainMaxCand));
-}
-
-template <int ARITH, int EPI, bool ONES, int B, int PATH = kPathAll>
+template <int ARITH, int EPI, bool ONES, int B, int PATH>
 __device__ __forceinline__ void dd_fwd_block(const DdView* __restrict__ geom,
                                              const float* __restrict__ lstar, int nang,
                                              int npix, const float* __restrict__ image,
@@ -849,52 +927,48 @@ __device__ __forceinline__ void dd_fwd_block(const DdView* __restrict__ geom,
     double p0 = 0.0;
 
     const bool sweep = g.kind == DD_SWEEP_ROWS || g.kind == DD_SWEEP_COLS;
-    const bool staged =
-        !ONES && sweep &&
-        (PATH == kPathWide ? g.ncand <= kFwdStagedWideMaxCand : g.ncand <= kFwdStagedMaxCand);
-    if (staged) {
-        // block-uniform: every thread joins the LDS-staged path; the epilogue inputs
-        // are loaded first so that their latency hides behind the sweep
-        constexpr int FLOATS =
-            PATH == kPathWide ? fwd_stage_floats_wide<B>() : fwd_stage_floats<B>();
-        __shared__ __attribute__((aligned(16))) float sImg[FLOATS];
-        __shared__ int sQ0[kFwdStageMaxLines], sQb[kFwdStageMaxLines];
-        __shared__ float sL[kFwdStageMaxLines];
+    if (!ONES && sweep) {
+        // block-uniform: every thread joins (threads past the last bin compute a copy of
+        // it and store nothing); the epilogue inputs are loaded first so that their latency
+        // hides behind the sweep
         const EpiFwdIn pre = active ? epi_fwd_load<EPI>(o, soff, z, e) : EpiFwdIn{0.0f, 0.0f};
-        const __amdgpu_buffer_rsrc_t rs =
-            image_rsrc((g.kind == DD_SWEEP_ROWS) ? image : imageT, npix);
         float acc = (EPI == EPI_STORE && accumulate && active) ? out[soff + o] : 0.0f;
         const float* ls = lstar + (int64_t)view * npix;
         const int nc = g.ncand;
-        if constexpr (PATH == kPathWide) {
-            // the launch of views with more than 8 candidates; up to 32 are staged (one
-            // or two lines per chunk), wider views take the gather path
-            static_assert(kFwdStagedWideMaxCand == 32, "staged candidate counts");
-            if (nc <= 12)
-                acc = fwd_staged<ARITH, B, 12, FLOATS>(g, ls, npix, nh, rs, bx, d, acc, sImg,
-                                                       sQ0, sQb, sL);
-            else if (nc <= 16)
-                acc = fwd_staged<ARITH, B, 16, FLOATS>(g, ls, npix, nh, rs, bx, d, acc, sImg,
-                                                       sQ0, sQb, sL);
-            else if (nc <= 24)
-                acc = fwd_staged<ARITH, B, 24, FLOATS>(g, ls, npix, nh, rs, bx, d, acc, sImg,
-                                                       sQ0, sQb, sL);
-            else
-                acc = fwd_staged<ARITH, B, 32, FLOATS>(g, ls, npix, nh, rs, bx, d, acc, sImg,
-                                                       sQ0, sQb, sL);
+        constexpr int SMAX = fwd_staged_max(PATH);
+        if (PATH == kFwdStaged || (PATH != kFwdDiag && nc <= SMAX)) {
+            if constexpr (PATH != kFwdDiag) {
+                constexpr int FLOATS = fwd_stage_floats<B>();
+                __shared__ __attribute__((aligned(16))) float sImg[FLOATS];
+                __shared__ float2 sMeta[kFwdStageMaxLines];
+                const __amdgpu_buffer_rsrc_t rs =
+                    image_rsrc((g.kind == DD_SWEEP_ROWS) ? image : imageT, npix);
+                if (nc <= 3)
+                    acc = fwd_staged<ARITH, B, 3, FLOATS>(g, ls, npix, nh, rs, bx, d, acc, sImg,
+                                                          sMeta);
+                else if (SMAX >= 4 && nc == 4)
+                    acc = fwd_staged<ARITH, B, 4, FLOATS>(g, ls, npix, nh, rs, bx, d, acc, sImg,
+                                                          sMeta);
+                else if (SMAX >= 5)
+                    acc = fwd_staged<ARITH, B, 6, FLOATS>(g, ls, npix, nh, rs, bx, d, acc, sImg,
+                                                          sMeta);
+            }
         } else {
-            // 3, 4 or up to kFwdStagedMaxCand candidates (staging 7-8 measured slower than
-            // the gather path)
-            static_assert(kFwdStagedMaxCand == 6, "staged candidate counts");
-            if (nc <= 3)
-                acc = fwd_staged<ARITH, B, 3, FLOATS>(g, ls, npix, nh, rs, bx, d, acc, sImg,
-                                                      sQ0, sQb, sL);
-            else if (nc == 4)
-                acc = fwd_staged<ARITH, B, 4, FLOATS>(g, ls, npix, nh, rs, bx, d, acc, sImg,
-                                                      sQ0, sQb, sL);
-            else
-                acc = fwd_staged<ARITH, B, 6, FLOATS>(g, ls, npix, nh, rs, bx, d, acc, sImg,
-                                                      sQ0, sQb, sL);
+            const float* img = (g.kind == DD_SWEEP_ROWS) ? imageT : image;
+#define ITOMO_DIAG(NC, GL) acc = fwd_diag<ARITH, NC, GL>(g, ls, npix, nh, img, d, acc)
+            if (SMAX < 4 && nc <= 4) ITOMO_DIAG(4, 4);
+            else if (SMAX < 5 && nc <= 5) ITOMO_DIAG(5, 4);
+            else if (SMAX < 6 && nc <= 6) ITOMO_DIAG(6, 3);
+            else if (nc <= 7) ITOMO_DIAG(7, 2);
+            else if (nc <= 8) ITOMO_DIAG(8, 2);
+            else if (nc <= 10) ITOMO_DIAG(10, 2);
+            else if (nc <= 12) ITOMO_DIAG(12, 2);
+            else if (nc <= 16) ITOMO_DIAG(16, 1);
+            else if (nc <= 20) ITOMO_DIAG(20, 1);
+            else if (nc <= 24) ITOMO_DIAG(24, 1);
+            else if (nc <= 32) ITOMO_DIAG(32, 1);
+            else ITOMO_DIAG(0, 1);
+#undef ITOMO_DIAG
         }
         if (active) out[soff + o] = epi_forward<EPI>(acc, pre, &p0);
     } else if (active) {
@@ -908,9 +982,7 @@ __device__ __forceinline__ void dd_fwd_block(const DdView* __restrict__ geom,
             const float* p = image + d;
             for (int j = 0; j < npix; ++j)
                 acc = __fadd_rn(acc, ONES ? 1.0f : p[(int64_t)j * npix]);
-        } else if (g.kind == DD_SWEEP_ROWS || g.kind == DD_SWEEP_COLS) {
-            const __amdgpu_buffer_rsrc_t rs =
-                image_rsrc((g.kind == DD_SWEEP_ROWS) ? image : imageT, npix);
+        } else if (sweep) {   // unit pixels
             const float Dlo = key_D<ARITH>(g, d - nh);
             const float Dhi = key_D<ARITH>(g, d + 1 - nh);
             const float* ls = lstar + (int64_t)view * npix;
@@ -932,53 +1004,16 @@ __device__ __forceinline__ void dd_fwd_block(const DdView* __restrict__ geom,
             // is needed only where Dhi exceeds that bound: the line's last pixel or the
             // last bin.
             const int nc = g.ncand;
-            const bool last_bin = d == npix - 1;
-            const float xNm1 = (float)(npix - 1 - nh);
-            float u = line_coord(i_lo, nh);
-            int lbase = i_lo * npix;
-            // Up to 16 candidates: lines in groups, all their loads issued before the first
-            // is consumed, so a wave keeps several gathers in flight; the lines are then
-            // accumulated in increasing order.  Candidates past the bin add nothing.
-            // Instances whose candidate counts the staged path takes in this launch are
-            // left out (they would only add registers).
-            constexpr int SMAX = ONES ? 0
-                                 : (PATH == kPathWide ? kFwdStagedWideMaxCand
-                                                      : kFwdStagedMaxCand);
-            if (fwd_in_path(PATH, 3) && 3 > SMAX && nc <= 3)
-                acc = fwd_grouped<ARITH, ONES, 3, kFwdLines>(rs, g, ls, i_lo, i_hi, npix, nh, Dlo,
-                                                           Dhi, last_bin, acc);
-            else if (fwd_in_path(PATH, 4) && 4 > SMAX && nc == 4)
-                acc = fwd_grouped<ARITH, ONES, 4, 6>(rs, g, ls, i_lo, i_hi, npix, nh, Dlo, Dhi,
-                                                     last_bin, acc);
-            else if (fwd_in_path(PATH, 6) && 6 > SMAX && nc <= 6)
-                acc = fwd_grouped<ARITH, ONES, 6, 4>(rs, g, ls, i_lo, i_hi, npix, nh, Dlo, Dhi,
-                                                     last_bin, acc);
-            else if (fwd_in_path(PATH, 8) && 8 > SMAX && nc <= 8)
-                acc = fwd_grouped<ARITH, ONES, 8, 3>(rs, g, ls, i_lo, i_hi, npix, nh, Dlo, Dhi,
-                                                     last_bin, acc);
-            else if (fwd_in_path(PATH, 12) && 12 > SMAX && nc <= 12)
-                acc = fwd_grouped<ARITH, ONES, 12, 2>(rs, g, ls, i_lo, i_hi, npix, nh, Dlo, Dhi,
-                                                      last_bin, acc);
-            else if (fwd_in_path(PATH, 16) && 16 > SMAX && nc <= 16)
-                acc = fwd_grouped<ARITH, ONES, 16, 2>(rs, g, ls, i_lo, i_hi, npix, nh, Dlo, Dhi,
-                                                      last_bin, acc);
-            else {
-                for (int i = i_lo; i <= i_hi; ++i, u = __fadd_rn(u, 1.0f), lbase += npix) {
-                    const float K = key_K<ARITH>(g, u);
-                    const float x = first_pixel(Dlo, K, nh, npix);
-                    const int q = (int)x + nh;
-                    float Dhc = Dhi;
-                    if (last_bin || Dhi > __fsub_rn(xNm1, K)) Dhc = fminf(Dhi, ls[i]);
-                    float xk = x, Rp = __fsub_rn(x, K);
-                    for (int k0 = 0; k0 < nc; k0 += 4) {
-                        float v[4] = {1.0f, 1.0f, 1.0f, 1.0f};
-                        if (!ONES) load_run<4>(rs, lbase + q + k0, npix * npix, v);
-#pragma unroll
-                        for (int k = 0; k < 4; ++k)
-                            acc = cand_step<ARITH>(k0 + k == 0, xk, Rp, K, Dlo, Dhc, v[k], acc);
-                    }
-                }
-            }
+            const bool last = d == npix - 1;
+#define ITOMO_ONES(NC) acc = fwd_ones<ARITH, NC>(g, ls, i_lo, i_hi, npix, nh, Dlo, Dhi, last, acc)
+            if (nc <= 3) ITOMO_ONES(3);
+            else if (nc == 4) ITOMO_ONES(4);
+            else if (nc <= 6) ITOMO_ONES(6);
+            else if (nc <= 8) ITOMO_ONES(8);
+            else if (nc <= 12) ITOMO_ONES(12);
+            else if (nc <= 16) ITOMO_ONES(16);
+            else ITOMO_ONES(0);
+#undef ITOMO_ONES
         }
         out[soff + o] = epi_forward<EPI>(acc, o, soff, z, e, &p0);
     }

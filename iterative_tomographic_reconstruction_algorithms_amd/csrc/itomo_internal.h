@@ -89,13 +89,8 @@ struct Plan {
     float* d_lstar;  // distance-driven: [view][line] start of the dropped segment
     int* d_range;    // slant-stacking: [view][bin] stepped range [u0, u1) (int2), clipped
                      // to the image
-    int* d_vlist;    // distance-driven: views of the main forward launch, then the wide ones
-    int n_staged, n_gather;  // (more than 8 candidate pixels per bin and line)
-    // Distance-driven plans with both kinds of views: the wide views' forward launch runs
-    // on this second stream (default priority), forked from and joined back into the
-    // caller's stream by the two events, beside the main launch.
-    hipStream_t aux_stream;
-    hipEvent_t ev_fork, ev_join;
+    int* d_vlist;    // distance-driven: the forward's staged views, then its diagonal ones
+    int n_staged;
     int fwd_var;     // distance-driven launch shapes (kFwdBins / kBackTiles index)
     int back_var;    // kBackAuto: chosen per launch (back_variant)
     int method;      // pixel-driven: 0 nearest bin, 1 linear split (radon_pd.c:57-85)
@@ -143,7 +138,8 @@ constexpr int kNumFwdVariants = 3;
 constexpr int kFwdBins[kNumFwdVariants] = {256, 128, 64};
 constexpr int kNumBackVariants = 4;
 constexpr int kBackTiles[kNumBackVariants][2] = {{64, 4}, {32, 2}, {32, 4}, {16, 1}};
-constexpr int kDdFwdBlock = 256;            // default forward shape
+constexpr int kDdFwdDefault = 2;            // 64 bins: the fastest or within 2% of it from 64^2
+                                            // to 2048^2 (256-bin blocks: 9-50% slower)
 constexpr int kBackAuto = -1;
 constexpr int kRdBlock = 64;
 constexpr int kEpiChunk = 256 * 8;          // pixels per elementwise-epilogue block

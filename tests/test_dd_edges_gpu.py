@@ -45,3 +45,31 @@ def test_chosen_back_tile_depends_on_the_launch_only_in_speed(nz):
     got = p.back(torch.from_numpy(y).cuda()).cpu().numpy()
     for z in (0, nz // 2, nz - 1):
         np.testing.assert_array_equal(got[z], O.dd_back(y[z], np.fft.ifftshift(ANGLES), O.FAST))
+
+
+@pytest.mark.parametrize("arith", ["fast", "ieee"])
+@pytest.mark.parametrize("n", [1, 2, 3, 15, 33, 63, 64, 65, 127, 130, 190])
+def test_forward_matches_oracle(n, arith):
+    mode = O.FAST if arith == "fast" else O.IEEE
+    x, _ = arrays(n, ANGLES.size)
+    want = O.dd_forward(x[0], np.fft.ifftshift(ANGLES), mode)
+    p = Plan("dd", n, ANGLES, arith)
+    xt = torch.from_numpy(x).cuda()
+    for f in range(L.FWD_VARIANTS):
+        p.set_shapes(f, p.shapes[1])
+        np.testing.assert_array_equal(p.forward(xt).cpu().numpy()[0], want, err_msg="shape %d" % f)
+
+
+@pytest.mark.parametrize("n,nz", [(65, 190), (130, 120), (17, 400)])
+def test_large_launches_match_oracle(n, nz):
+    # more than 10240 waves of 64 bins: the staged and the diagonal views run in launches of
+    # their own, and views with 4 to 6 candidates are staged
+    x, _ = arrays(n, ANGLES.size, nz)
+    assert (n + 63) // 64 * ANGLES.size * nz > 10240
+    p = Plan("dd", n, ANGLES)
+    for f in range(L.FWD_VARIANTS):
+        p.set_shapes(f, p.shapes[1])
+        got = p.forward(torch.from_numpy(x).cuda()).cpu().numpy()
+        for z in (0, nz // 2, nz - 1):
+            np.testing.assert_array_equal(
+                got[z], O.dd_forward(x[z], np.fft.ifftshift(ANGLES), O.FAST))
