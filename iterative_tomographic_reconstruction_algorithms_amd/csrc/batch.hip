@@ -89,8 +89,8 @@ __device__ __forceinline__ int next_item(int* counter)
 
 // Five waves per SIMD (96 registers): the kernel holds every forward path and the fused
 // update.  Measured on 16 slices of 1024^2 x 900 (forward and back): 14.68 ms per iteration at
-// four waves, 14.47 at five, 15.03 at six, 16.23 at eight.  PATH: kFwdSmall up to kFwdBigWaves
-// items, kFwdMixed beyond, as the per-plan launches choose.
+// four waves, 14.47 at five, 15.03 at six, 16.23 at eight.  PATH: kFwdSmall up to kFwdLargeWaves
+// items, kFwdLarge beyond, as the per-plan launches choose.
 template <int PATH>
 __global__ void __launch_bounds__(kBatchFwdBlock) __attribute__((amdgpu_waves_per_eu(5)))
 batch_fwd_kernel(const BatchMember* __restrict__ mem, const BatchItem* __restrict__ items,
@@ -320,11 +320,11 @@ int itomo_batch_sirt_iterate(itomo_batch* B, float pc_beta, void* stream)
     }
     reset_counter_kernel<<<1, 1, 0, st>>>(B->d_counter);
     const int fgrid = std::min(B->grid * (256 / kBatchFwdBlock), B->nfwd);
-    if (B->nfwd <= kFwdBigWaves)
+    if (B->nfwd <= kFwdLargeWaves)
         batch_fwd_kernel<kFwdSmall><<<fgrid, kBatchFwdBlock, 0, st>>>(B->d_members, B->d_fwd,
                                                                       B->nfwd, B->d_counter);
     else
-        batch_fwd_kernel<kFwdMixed><<<fgrid, kBatchFwdBlock, 0, st>>>(B->d_members, B->d_fwd,
+        batch_fwd_kernel<kFwdLarge><<<fgrid, kBatchFwdBlock, 0, st>>>(B->d_members, B->d_fwd,
                                                                       B->nfwd, B->d_counter);
     const int bgrid = std::min(B->grid, B->nback);
     if (B->back_var == 0)

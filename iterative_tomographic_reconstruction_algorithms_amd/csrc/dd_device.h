@@ -225,9 +225,10 @@ __device__ __forceinline__ void walk_tile(const DdView& g, float u, float x0, co
                 if (MULTI) {
                     const float Dhi2 = key_Df<ARITH>(g, (float)(jr[i] + 1));
                     const float m2 = fminf(hc, Dhi2);
-                    t2[i] = Dhi2 < hc ? S[jr[i] + 2] : 0.0f;
+                    const float third = S[jr[i] + 2];   // read by every lane, used by few
                     v1[i] = fmaxf(__fsub_rn(m2, Dhi), 0.0f);
                     v2[i] = __fsub_rn(hc, m2);
+                    t2[i] = Dhi2 < hc ? third : 0.0f;
                     jr[i] += Dhi2 < hi;
                 } else {
                     v1[i] = __fsub_rn(hc, m);
@@ -888,19 +889,18 @@ __device__ __forceinline__ float fwd_staged(const DdView& g, const float* __rest
     return acc;
 }
 
-// Which views a forward launch handles (block-uniform) and how.  Views with at most
-// fwd_staged_max(path) candidates are staged, the others go along diagonals.  A staged block
-// reads each line once through LDS, a diagonal one through the L1; staging wins for up to 6
-// candidates once the launch fills the GPU, the diagonals from 4 on while it does not (their
-// chains are shorter).  Staged up to 6 against up to 3, in us: 363^2 x 251 x 3 slices (4518
-// waves) 123 and 112, 724^2 x 512 (6144) 245 and 223, 1024^2 x 720 (11520) 531 and 525,
-// 1448^2 x 900 (20700) 1186 and 1364, 2048^2 x 1800 (57600) 4432 and 6014.  The line is drawn
-// at kFwdBigWaves.  A launch beyond it is split in two, each kernel with its own registers and
-// LDS: kFwdStaged and kFwdDiag; kFwdMixed holds both (the persistent batch).
-constexpr int kFwdSmall = 0, kFwdStaged = 1, kFwdDiag = 2, kFwdMixed = 3;
-constexpr int64_t kFwdBigWaves = 10240;
-constexpr int kFwdStagedMaxCand = 6;
-constexpr int fwd_staged_max(int path) { return path == kFwdSmall ? 3 : kFwdStagedMaxCand; }
+// How a forward launch takes its views: those with at most fwd_staged_max(path) candidates are
+// staged, the others go along diagonals.  A staged block reads each line once through LDS, a
+// diagonal one through the L1; staging wins for up to 6 candidates once the launch fills the
+// GPU, the diagonals from 4 on while it does not (their chains are shorter).  Staged up to 6
+// against up to 3, in us: 363^2 x 251 x 3 slices (4518 waves) 123 and 112, 724^2 x 512 (6144)
+// 245 and 223, 1024^2 x 720 (11520) 531 and 525, 1448^2 x 900 (20700) 1186 and 1364,
+// 2048^2 x 1800 (57600) 4432 and 6014; the line is drawn at kFwdLargeWaves.  Both kinds of views
+// share one launch: their waves wait for different units.  (The diagonal ones in a launch of
+// their own: 4967 us at 2048^2 x 1800 after the staged ones, 4603 beside them on another stream.)
+constexpr int kFwdSmall = 0, kFwdLarge = 1;
+constexpr int64_t kFwdLargeWaves = 10240;
+constexpr int fwd_staged_max(int path) { return path == kFwdSmall ? 3 : 6; }
 
 // Forward projection: one thread per (bin, view, slice).
 // Lines are image rows for row sweeps and image columns for column sweeps.  Each path reads
@@ -936,23 +936,21 @@ __device__ __forceinline__ void dd_fwd_block(const DdView* __restrict__ geom,
         const float* ls = lstar + (int64_t)view * npix;
         const int nc = g.ncand;
         constexpr int SMAX = fwd_staged_max(PATH);
-        if (PATH == kFwdStaged || (PATH != kFwdDiag && nc <= SMAX)) {
-            if constexpr (PATH != kFwdDiag) {
-                constexpr int FLOATS = fwd_stage_floats<B>();
-                __shared__ __attribute__((aligned(16))) float sImg[FLOATS];
-                __shared__ float2 sMeta[kFwdStageMaxLines];
-                const __amdgpu_buffer_rsrc_t rs =
-                    image_rsrc((g.kind == DD_SWEEP_ROWS) ? image : imageT, npix);
-                if (nc <= 3)
-                    acc = fwd_staged<ARITH, B, 3, FLOATS>(g, ls, npix, nh, rs, bx, d, acc, sImg,
-                                                          sMeta);
-                else if (SMAX >= 4 && nc == 4)
-                    acc = fwd_staged<ARITH, B, 4, FLOATS>(g, ls, npix, nh, rs, bx, d, acc, sImg,
-                                                          sMeta);
-                else if (SMAX >= 5)
-                    acc = fwd_staged<ARITH, B, 6, FLOATS>(g, ls, npix, nh, rs, bx, d, acc, sImg,
-                                                          sMeta);
-            }
+        if (nc <= SMAX) {
+            constexpr int FLOATS = fwd_stage_floats<B>();
+            __shared__ __attribute__((aligned(16))) float sImg[FLOATS];
+            __shared__ float2 sMeta[kFwdStageMaxLines];
+            const __amdgpu_buffer_rsrc_t rs =
+                image_rsrc((g.kind == DD_SWEEP_ROWS) ? image : imageT, npix);
+            if (nc <= 3)
+                acc = fwd_staged<ARITH, B, 3, FLOATS>(g, ls, npix, nh, rs, bx, d, acc, sImg,
+                                                      sMeta);
+            else if (SMAX >= 4 && nc == 4)
+                acc = fwd_staged<ARITH, B, 4, FLOATS>(g, ls, npix, nh, rs, bx, d, acc, sImg,
+                                                      sMeta);
+            else if (SMAX >= 5)
+                acc = fwd_staged<ARITH, B, 6, FLOATS>(g, ls, npix, nh, rs, bx, d, acc, sImg,
+                                                      sMeta);
         } else {
             const float* img = (g.kind == DD_SWEEP_ROWS) ? imageT : image;
 #define ITOMO_DIAG(NC, GL) acc = fwd_diag<ARITH, NC, GL>(g, ls, npix, nh, img, d, acc)

@@ -62,8 +62,7 @@ def test_forward_matches_oracle(n, arith):
 
 @pytest.mark.parametrize("n,nz", [(65, 190), (130, 120), (17, 400)])
 def test_large_launches_match_oracle(n, nz):
-    # more than 10240 waves of 64 bins: the staged and the diagonal views run in launches of
-    # their own, and views with 4 to 6 candidates are staged
+    # more than 10240 waves of 64 bins: views with 4 to 6 candidates are staged
     x, _ = arrays(n, ANGLES.size, nz)
     assert (n + 63) // 64 * ANGLES.size * nz > 10240
     p = Plan("dd", n, ANGLES)
