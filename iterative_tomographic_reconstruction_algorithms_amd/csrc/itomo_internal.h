@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 #include <cstdint>
+#include <mutex>
 
 #include "itomo.h"
 
@@ -110,6 +111,11 @@ struct Plan {
     mutable int64_t* rdb_off;
     mutable int* rdb_cnt;
     mutable size_t rd_mat_bytes;
+    // Pixel-driven and slant-stacking plans: the buffer of TransposedCopy, grown on first use.
+    mutable std::mutex copy_mutex;
+    mutable float* copy;
+    mutable size_t copy_bytes;
+    mutable hipEvent_t copy_read;  // recorded behind the last launch that reads the copy
 };
 
 // Largest ray-driven system matrix a plan caches (forward and back entries together).
@@ -120,6 +126,26 @@ int rd_matrix_ensure(const Plan& p, hipStream_t st);
 void rd_matrix_free(const Plan& p);
 // out = the transposes of nslices npix x npix images (npix^2 apart); stream-ordered.
 int launch_transpose(const float* in, float* out, int npix, int nslices, hipStream_t st);
+// The transposed copies of a call's images, in a buffer of the plan, from the constructor to
+// the destructor: get() is null where there is none, because it is not wanted, st is capturing
+// (a replay would share the buffer unseen) or memory is short; the caller then reads the image
+// as it is.  Calls of one plan on several threads or streams take the buffer in turn: the
+// object holds the plan's lock, the copy waits for the last reader and the destructor marks
+// the new one, so the caller enqueues what reads the copy before the object ends.
+class TransposedCopy {
+public:
+    TransposedCopy(const Plan& p, bool wanted, const float* image, int nslices, hipStream_t st);
+    ~TransposedCopy();
+    TransposedCopy(const TransposedCopy&) = delete;
+    TransposedCopy& operator=(const TransposedCopy&) = delete;
+    const float* get() const { return copy_; }
+
+private:
+    const Plan& p_;
+    hipStream_t st_;
+    const float* copy_ = nullptr;
+    std::unique_lock<std::mutex> lock_;
+};
 // Marks the matrix as held by a graph when st is capturing.
 void rd_matrix_note_use(const Plan& p, hipStream_t st);
 // Whether a caller-owned scratch region is active on this thread (no allocation then).

@@ -24,15 +24,25 @@
 // sinogram row.  That is reproduced (the forward thread of row r also gathers the
 // overflow of views r-1 and r+1); flat indices outside the array, where the reference
 // writes out of bounds, are skipped.
+//
+// Both are bound by instruction issue, about a third of it FP64 (every update converts, adds
+// and rounds), so the loops are straight-line: candidates are evaluated several at a time, a
+// hit selects the updated sum instead of branching to it, and the products, exact in
+// double, are formed once for a sample's two additions.  Method 1, us before and after that and
+// the transposed copy: 64^2 x 45 views forward 62 -> 55, back 31 -> 23; 511^2 x 360 741 -> 595
+// and 320 -> 237; 1024^2 x 720 5517 -> 3551 and 1810 -> 1379.
 #include "epilogue.h"
 
 namespace itomo {
 
-constexpr int kPdFwdBlock = 256;
+constexpr int kPdFwdBlock = 64;
 constexpr int kPdBackX = 64, kPdBackY = 4;
 
-// Signed distance of sample (x, y) from the central ray (radon_pd.c:44-55).
-template <int ARITH>
+// Signed distance of sample (x, y) from the central ray (radon_pd.c:44-55).  PLAIN: the view's
+// angle is neither 0 nor pi/2, so only the comparison with the ray decides the sign.
+constexpr int kPdPlain = kPdLt | kPdGt;
+
+template <int ARITH, bool PLAIN>
 __device__ __forceinline__ float pd_t(const PdView& g, float x, float y)
 {
     const float xs = __fmul_rn(x, g.s);
@@ -44,9 +54,15 @@ __device__ __forceinline__ float pd_t(const PdView& g, float x, float y)
         t = fabsf(__fsub_rn(xs, __fmul_rn(y, g.c)));
         q = __fdiv_rn(xs, g.c);
     }
-    const bool keep = ((g.flags & (kPdLt | kPdGt)) && y > q) ||
-                      ((g.flags & kPdZero) && y > 0.0f) || ((g.flags & kPdHalf) && x < 0.0f);
+    const bool keep = PLAIN ? y > q
+                            : ((g.flags & kPdPlain) && y > q) || ((g.flags & kPdZero) && y > 0.0f) ||
+                                  ((g.flags & kPdHalf) && x < 0.0f);
     return keep ? t : -t;
+}
+
+__device__ __forceinline__ bool pd_plain(const PdView& g)
+{
+    return (g.flags & kPdPlain) && !(g.flags & ~kPdPlain);
 }
 
 // Method 0 bin: round(nh - 0.5 - t) (radon_pd.c:58).  nh - 0.5 - t is exact in double.
@@ -88,47 +104,24 @@ __device__ __forceinline__ float pd_acc(float acc, float w, float v)
     return (float)__fma_rn((double)w, __dmul_rn((double)v, 0.25), (double)acc);
 }
 
-// Contribution of pixel value px at centre (x0, y0) to bin e (e >= 1 for method 1; any
-// integer for method 0, e = the bin index before the flat-index overflow).
-template <int ARITH, int METHOD>
-__device__ __forceinline__ float pd_fwd_pixel(const PdView& g, int nh, float nhf, float x0,
-                                              float y0, int e, float px, float acc)
+// Sum of one view's samples that land in bin e, in the reference's (i, j, k) order.  Memory
+// row m (= npix-1-i), column j of the image is img[m * sm + j * sj].
+//
+// Method 1: a sample at t1 = nh - t adds the weight of its lower bin lf = floor(t1), uf - t1,
+// when lf = e, and that of its upper bin, t1 - lf, when uf = e.  So it hits e when t1 lies in
+// (e-1, e+1), with weight min((e+1) - t1, t1 - (e-1)) -- the same two subtractions, the
+// smaller being the one that applies -- except t1 = e, where lf = uf and both weights are 0.
+// lf == uf stands for two zero-weight terms in the reference; one is added here (x + 0 = x).
+template <int ARITH, int METHOD, bool ONES, bool PLAIN>
+__device__ __forceinline__ float pd_fwd_bin(const PdView& g, int npix, const float* __restrict__ img, int sm,
+                            int sj, int e, float acc)
 {
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        const float d = h ? 0.25f : -0.25f;
-        const float t = pd_t<ARITH>(g, __fadd_rn(d, x0), __fadd_rn(d, y0));
-        if (METHOD == 0) {
-            if (pd_nearest<ARITH>(nh, t) == e) {  // samples 2h and 2h+1 coincide
-                acc = pd_acc(acc, 1.0f, px);
-                acc = pd_acc(acc, 1.0f, px);
-            }
-        } else {
-            const PdSplit s = pd_split<ARITH>(nhf, t);
-            const float ef = (float)e;
-            const bool hl = s.lf == ef, hu = s.uf == ef;
-            // lf == uf only for an integer t1, where both weights are 0: one zero-weight
-            // term then stands for the reference's two (x + 0 = x; a non-finite pixel
-            // gives NaN either way)
-            const float w = hl ? s.wl : s.wu;
-            if (hl || hu) {
-                acc = pd_acc(acc, w, px);
-                acc = pd_acc(acc, w, px);
-            }
-        }
-    }
-    return acc;
-}
-
-// Sum of one view's samples that land in bin e, in the reference's (i, j, k) order.
-template <int ARITH, int METHOD, bool ONES>
-__device__ float pd_fwd_bin(const PdView& g, int npix, const float* __restrict__ image,
-                            int e, float acc)
-{
+    constexpr int U = 3;   // a row of a steep view (|sin| > |cos|) has at most 3 candidates
     const int nh = npix >> 1;
-    const float nhf = (float)nh;
+    const float nhf = (float)nh, ef = (float)e;
+    const float em1 = ef - 1.0f, ep1 = ef + 1.0f;
     // The samples of a pixel sit at t(x0, y0) +- dshift; float rounding of t, of the sign
-    // test and of nh - t stays far below npix * 2^-18.
+    // test, of nh - t and of the column bounds stays far below npix * 2^-18.
     const double half = 1.0 + g.dshift + 0.01 + npix * 0x1p-18;
     const double mid = (double)(nh - e);
     const double tl = mid - half, th = mid + half;
@@ -145,52 +138,90 @@ __device__ float pd_fwd_bin(const PdView& g, int npix, const float* __restrict__
     }
     // column range of row i: x0 between (C*y0 - th)/S and (C*y0 - tl)/S, in column units
     // j = x0 + nh - 1/2: j_lo/hi = a*y0 + b_lo/hi
-    const double rs = g.rsdir, a = C * rs, off = nh - 0.5;
-    const double b_lo = (rs > 0.0 ? -th : -tl) * rs + off;
-    const double b_hi = (rs > 0.0 ? -tl : -th) * rs + off;
+    const double rs = g.rsdir, off = nh - 0.5;
+    const float a = (float)(C * rs);
+    const float b_lo = (float)((rs > 0.0 ? -th : -tl) * rs + off);
+    const float b_hi = (float)((rs > 0.0 ? -tl : -th) * rs + off);
+    const float jmax = (float)(npix - 1);
     for (int i = i0; i <= i1; ++i) {
         const float y0 = __fadd_rn((float)(i - nh), 0.5f);
         int j0, j1;
         if (rs != 0.0) {
-            j0 = (int)fmin(fmax(0.0, ceil(fma((double)y0, a, b_lo))), (double)npix);
-            j1 = (int)fmax(-1.0, fmin((double)(npix - 1), floor(fma((double)y0, a, b_hi))));
+            j0 = (int)fminf(fmaxf(0.0f, ceilf(__builtin_fmaf(y0, a, b_lo))), jmax + 1.0f);
+            j1 = (int)fmaxf(-1.0f, fminf(jmax, floorf(__builtin_fmaf(y0, a, b_hi))));
         } else {
             const double yc = (double)y0 * C;
             const bool in = yc > tl && yc < th;
             j0 = in ? 0 : 1;
             j1 = in ? npix - 1 : 0;
         }
-        const float* __restrict__ row = image + (int64_t)(npix - 1 - i) * npix;
-        for (int j = j0; j <= j1; ++j) {
-            const float px = ONES ? 1.0f : row[j];
-            const float x0 = __fadd_rn((float)(j - nh), 0.5f);
-            acc = pd_fwd_pixel<ARITH, METHOD>(g, nh, nhf, x0, y0, e, px, acc);
+        // indices below 2^15 times strides below 2^15
+        const unsigned row = __umul24(npix - 1 - i, sm);
+        for (; j0 <= j1; j0 += U) {
+            float px[U];
+#pragma unroll
+            for (int k = 0; k < U; ++k)
+                px[k] = ONES ? 1.0f : img[row + __umul24(min(j0 + k, j1), sj)];
+#pragma unroll
+            for (int k = 0; k < U; ++k) {
+                const float x0 = __fadd_rn((float)(j0 + k - nh), 0.5f);
+                const double v = (double)px[k];
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const float d = h ? 0.25f : -0.25f;
+                    const float t = pd_t<ARITH, PLAIN>(g, __fadd_rn(d, x0), __fadd_rn(d, y0));
+                    bool hit;
+                    double w;
+                    if (METHOD == 0) {
+                        hit = pd_nearest<ARITH>(nh, t) == e;   // samples 2h and 2h+1 coincide
+                        w = __dmul_rn(0.25, v);
+                    } else {
+                        const float t1 = __fsub_rn(nhf, t);
+                        const float m = fminf(__fsub_rn(ep1, t1), __fsub_rn(t1, em1));
+                        hit = m > 0.0f;
+                        // exact: a weight above 2^-25, a quarter of it, 24 x 24 bits
+                        w = (double)__fmul_rn(t1 == ef ? 0.0f : m, 0.25f) * v;
+                    }
+                    hit = hit && j0 + k <= j1;
+                    const float once = (float)((double)acc + w);
+                    const float twice = (float)((double)once + w);
+                    acc = hit ? twice : acc;
+                }
+            }
         }
     }
     return acc;
 }
 
-// One thread per (sinogram row r, bin b).  Epilogues: STORE, RECIP.
+// One thread per (sinogram row r, bin b).  Epilogues: STORE, RECIP.  Neighbouring bins of a
+// flat view (|cos| > |sin|) lie in neighbouring image rows: those views read the transposed
+// copy (when there is one), so that a wave's loads are contiguous.
 template <int ARITH, int METHOD, int EPI, bool ONES>
 __global__ void __launch_bounds__(kPdFwdBlock)
 pd_fwd_kernel(const PdView* __restrict__ geom, int npix, int nang,
-              const float* __restrict__ image, float* __restrict__ out, int64_t img_stride,
-              int64_t sino_stride, int accumulate, EpiArgs e)
+              const float* __restrict__ image, const float* __restrict__ imageT,
+              float* __restrict__ out, int64_t img_stride, int64_t sino_stride, int accumulate,
+              EpiArgs e)
 {
     const int b = blockIdx.x * kPdFwdBlock + threadIdx.x;
     if (b >= npix) return;
     const int r = blockIdx.y, z = blockIdx.z;
-    image += (int64_t)z * img_stride;
+    auto bin = [&](int v, int bin_e, float acc) {
+        const PdView g = geom[v];
+        const bool flat = imageT && fabsf(g.c) > fabsf(g.s);
+        const float* img = (flat ? imageT : image) + (int64_t)z * img_stride;
+        const int sm = flat ? 1 : npix, sj = flat ? npix : 1;
+        return pd_plain(g) ? pd_fwd_bin<ARITH, METHOD, ONES, true>(g, npix, img, sm, sj, bin_e, acc)
+                           : pd_fwd_bin<ARITH, METHOD, ONES, false>(g, npix, img, sm, sj, bin_e, acc);
+    };
     const int64_t soff = (int64_t)z * sino_stride, o = (int64_t)r * npix + b;
     float acc = (EPI == EPI_STORE && accumulate) ? out[soff + o] : 0.0f;
     if (METHOD == 0) {
         // view r-1 overflows into row r at bins l = b + npix, view r+1 at l = b - npix
         for (int vs = r - 1; vs <= r + 1; ++vs)
-            if (vs >= 0 && vs < nang)
-                acc = pd_fwd_bin<ARITH, 0, ONES>(geom[vs], npix, image, b + (r - vs) * npix,
-                                                 acc);
+            if (vs >= 0 && vs < nang) acc = bin(vs, b + (r - vs) * npix, acc);
     } else if (b > 0) {  // bin 0 never receives anything (radon_pd.c:74)
-        acc = pd_fwd_bin<ARITH, 1, ONES>(geom[r], npix, image, b, acc);
+        acc = bin(r, b, acc);
     }
     double p0 = 0.0;
     out[soff + o] = epi_forward<EPI>(acc, o, soff, z, e, &p0);
@@ -219,29 +250,64 @@ pd_back_kernel(const PdView* __restrict__ geom, int npix, int nang,
         for (int v = 0; v < nang; ++v) {
             const PdView g = geom[v];
             const float* __restrict__ rowp = sino + (int64_t)v * npix;
+            const bool plain = pd_plain(g);
+            float ts[2];
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
                 const float d = h ? 0.25f : -0.25f;
-                const float t = pd_t<ARITH>(g, __fadd_rn(d, x0), __fadd_rn(d, y0));
-                if (METHOD == 0) {
-                    const int64_t f = (int64_t)v * npix + pd_nearest<ARITH>(nh, t);
+                const float xs = __fadd_rn(d, x0), ys = __fadd_rn(d, y0);
+                ts[h] = plain ? pd_t<ARITH, true>(g, xs, ys) : pd_t<ARITH, false>(g, xs, ys);
+            }
+            if (METHOD == 0) {
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const int64_t f = (int64_t)v * npix + pd_nearest<ARITH>(nh, ts[h]);
                     if (f >= 0 && f < ntot) {
                         const float sv = ONES ? 1.0f : sino[f];
                         acc = pd_acc(acc, 1.0f, sv);
                         acc = pd_acc(acc, 1.0f, sv);
                     }
-                } else {
-                    const PdSplit s = pd_split<ARITH>(nhf, t);
-                    const bool okl = s.lf >= 1.0f && s.lf < npixf;
-                    const bool oku = s.uf >= 1.0f && s.uf < npixf;
-                    const float sl = okl ? (ONES ? 1.0f : rowp[(int)s.lf]) : 0.0f;
-                    const float su = oku ? (ONES ? 1.0f : rowp[(int)s.uf]) : 0.0f;
+                }
+            } else {
+                // both samples' products first (exact in double), then the eight additions; a
+                // bin outside [1, npix) reads as 0, which adds nothing
+                PdSplit s[2];
+                float sl[2] = {1.0f, 1.0f}, su[2] = {1.0f, 1.0f};
+                bool inside = true;
 #pragma unroll
-                    for (int rep = 0; rep < 2; ++rep) {
-                        if (okl) acc = pd_acc(acc, s.wl, sl);
-                        if (oku) acc = pd_acc(acc, s.wu, su);
+                for (int h = 0; h < 2; ++h) {
+                    s[h] = pd_split<ARITH>(nhf, ts[h]);
+                    inside = inside && s[h].lf >= 1.0f && s[h].uf < npixf;
+                }
+                if (__all(inside)) {
+#pragma unroll
+                    for (int h = 0; h < 2; ++h)
+                        if (!ONES) {
+                            sl[h] = rowp[(unsigned)(int)s[h].lf];
+                            su[h] = rowp[(unsigned)(int)s[h].uf];
+                        }
+                } else {
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        const bool okl = s[h].lf >= 1.0f && s[h].lf < npixf;
+                        const bool oku = s[h].uf >= 1.0f && s[h].uf < npixf;
+                        sl[h] = okl ? (ONES ? 1.0f : rowp[(int)s[h].lf]) : 0.0f;
+                        su[h] = oku ? (ONES ? 1.0f : rowp[(int)s[h].uf]) : 0.0f;
                     }
                 }
+                double pl[2], pu[2];
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    pl[h] = (double)__fmul_rn(s[h].wl, 0.25f) * (double)sl[h];
+                    pu[h] = (double)__fmul_rn(s[h].wu, 0.25f) * (double)su[h];
+                }
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+#pragma unroll
+                    for (int rep = 0; rep < 2; ++rep) {
+                        acc = (float)((double)acc + pl[h]);
+                        acc = (float)((double)acc + pu[h]);
+                    }
             }
         }
         const float xo = epi_updates_x(EPI) ? out[ioff + o] : 0.0f;
@@ -256,26 +322,26 @@ pd_back_kernel(const PdView* __restrict__ geom, int npix, int nang,
 namespace {
 
 template <int ARITH, int METHOD, int EPI, bool ONES>
-void launch_pd_fwd(const Plan& p, const float* image, float* out, int nslices, int accumulate,
-                   const EpiArgs& e, hipStream_t st)
+void launch_pd_fwd(const Plan& p, const float* image, const float* imageT, float* out,
+                   int nslices, int accumulate, const EpiArgs& e, hipStream_t st)
 {
     dim3 grid((p.npix + kPdFwdBlock - 1) / kPdFwdBlock, p.nang, nslices);
     pd_fwd_kernel<ARITH, METHOD, EPI, ONES><<<grid, kPdFwdBlock, 0, st>>>(
-        (const PdView*)p.d_geom, p.npix, p.nang, image, out, (int64_t)p.npix * p.npix,
+        (const PdView*)p.d_geom, p.npix, p.nang, image, imageT, out, (int64_t)p.npix * p.npix,
         (int64_t)p.nang * p.npix, accumulate, e);
 }
 
 template <int ARITH, int METHOD>
-int dispatch_pd_fwd(const Plan& p, int epi, int ones, const float* image, float* out,
-                    int nslices, int accumulate, const EpiArgs& e, hipStream_t st)
+int dispatch_pd_fwd(const Plan& p, int epi, int ones, const float* image, const float* imageT,
+                    float* out, int nslices, int accumulate, const EpiArgs& e, hipStream_t st)
 {
     if (epi == EPI_STORE) {
-        if (ones) launch_pd_fwd<ARITH, METHOD, EPI_STORE, true>(p, image, out, nslices, accumulate, e, st);
-        else launch_pd_fwd<ARITH, METHOD, EPI_STORE, false>(p, image, out, nslices, accumulate, e, st);
+        if (ones) launch_pd_fwd<ARITH, METHOD, EPI_STORE, true>(p, image, imageT, out, nslices, accumulate, e, st);
+        else launch_pd_fwd<ARITH, METHOD, EPI_STORE, false>(p, image, imageT, out, nslices, accumulate, e, st);
         return ITOMO_OK;
     }
     if (epi == EPI_RECIP && ones) {
-        launch_pd_fwd<ARITH, METHOD, EPI_RECIP, true>(p, image, out, nslices, 0, e, st);
+        launch_pd_fwd<ARITH, METHOD, EPI_RECIP, true>(p, image, imageT, out, nslices, 0, e, st);
         return ITOMO_OK;
     }
     return set_error(ITOMO_EINVAL, "pd forward: unsupported epilogue %d", epi);
@@ -320,6 +386,14 @@ int dispatch_pd_back(const Plan& p, int epi, int ones, const float* sino, float*
 
 }  // namespace
 
+// Whether a forward call reads a transposed copy for its flat views: from about 8192 waves (us
+// with and without: 511^2 x 360, 2880 waves, 597 and 593; 512^2 x 361 x 2 slices, 5776, 991 and
+// 989; 1024^2 x 720, 11520, 3552 and 3902).
+static bool pd_transposes(const Plan& p, int nslices)
+{
+    return (int64_t)((p.npix + 63) / 64) * p.nang * nslices >= 8192;
+}
+
 int pd_forward_epi(const Plan& p, int epi, int ones, const float* image, float* out,
                    int nslices, int accumulate, const EpiArgs& e, hipStream_t st,
                    int* blocks_per_slice)
@@ -333,15 +407,17 @@ int pd_forward_epi(const Plan& p, int epi, int ones, const float* image, float* 
                                         blocks_per_slice);
     }
     if (blocks_per_slice) *blocks_per_slice = 0;
+    const TransposedCopy tc(p, !ones && pd_transposes(p, nslices), image, nslices, st);
+    const float* imageT = tc.get();
     int rc;
     if (p.arith == ITOMO_ARITH_FAST)
         rc = p.method == 0
-                 ? dispatch_pd_fwd<ITOMO_ARITH_FAST, 0>(p, epi, ones, image, out, nslices, accumulate, e, st)
-                 : dispatch_pd_fwd<ITOMO_ARITH_FAST, 1>(p, epi, ones, image, out, nslices, accumulate, e, st);
+                 ? dispatch_pd_fwd<ITOMO_ARITH_FAST, 0>(p, epi, ones, image, imageT, out, nslices, accumulate, e, st)
+                 : dispatch_pd_fwd<ITOMO_ARITH_FAST, 1>(p, epi, ones, image, imageT, out, nslices, accumulate, e, st);
     else
         rc = p.method == 0
-                 ? dispatch_pd_fwd<ITOMO_ARITH_IEEE, 0>(p, epi, ones, image, out, nslices, accumulate, e, st)
-                 : dispatch_pd_fwd<ITOMO_ARITH_IEEE, 1>(p, epi, ones, image, out, nslices, accumulate, e, st);
+                 ? dispatch_pd_fwd<ITOMO_ARITH_IEEE, 0>(p, epi, ones, image, imageT, out, nslices, accumulate, e, st)
+                 : dispatch_pd_fwd<ITOMO_ARITH_IEEE, 1>(p, epi, ones, image, imageT, out, nslices, accumulate, e, st);
     if (rc) return rc;
     return check_hip(hipGetLastError(), "pd forward launch");
 }

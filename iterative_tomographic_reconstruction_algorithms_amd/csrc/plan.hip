@@ -299,6 +299,54 @@ int get_scratch(const Plan& p, int nslices, Scratch* s, hipStream_t st)
     return ITOMO_OK;
 }
 
+TransposedCopy::TransposedCopy(const Plan& p, bool wanted, const float* image, int nslices,
+                               hipStream_t st)
+    : p_(p), st_(st)
+{
+    if (!wanted) return;
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &cs) != hipSuccess) {
+        (void)hipGetLastError();
+        return;
+    }
+    if (cs != hipStreamCaptureStatusNone) return;
+    lock_ = std::unique_lock<std::mutex>(p.copy_mutex);
+    if (!p.copy_read &&
+        hipEventCreateWithFlags(&p.copy_read, hipEventDisableTiming) != hipSuccess) {
+        (void)hipGetLastError();
+        p.copy_read = nullptr;
+        return;
+    }
+    const size_t bytes = sizeof(float) * (size_t)p.npix * p.npix * nslices;
+    if (bytes > p.copy_bytes) {
+        if (p.copy) {
+            (void)hipEventSynchronize(p.copy_read);  // queued launches may still read it
+            (void)hipFree(p.copy);
+        }
+        p.copy_bytes = 0;
+        if (hipMalloc(&p.copy, bytes) != hipSuccess) {
+            (void)hipGetLastError();
+            p.copy = nullptr;
+            return;
+        }
+        p.copy_bytes = bytes;
+    }
+    if (hipStreamWaitEvent(st, p.copy_read, 0) != hipSuccess ||
+        launch_transpose(image, p.copy, p.npix, nslices, st) != ITOMO_OK) {
+        (void)hipGetLastError();
+        return;
+    }
+    copy_ = p.copy;
+}
+
+TransposedCopy::~TransposedCopy()
+{
+    if (copy_ && hipEventRecord(p_.copy_read, st_) != hipSuccess) {
+        (void)hipGetLastError();
+        (void)hipStreamSynchronize(st_);  // no mark: nothing may be left to read the copy
+    }
+}
+
 }  // namespace itomo
 
 using namespace itomo;
@@ -444,6 +492,14 @@ int itomo_plan_destroy(itomo_plan* p)
     }
     if (p->scratch) {
         int st2 = check_hip(hipFree(p->scratch), "plan_destroy: hipFree scratch");
+        if (!st) st = st2;
+    }
+    if (p->copy) {
+        int st2 = check_hip(hipFree(p->copy), "plan_destroy: hipFree copy");
+        if (!st) st = st2;
+    }
+    if (p->copy_read) {
+        int st2 = check_hip(hipEventDestroy(p->copy_read), "plan_destroy: event");
         if (!st) st = st2;
     }
     rd_matrix_free(*p);
