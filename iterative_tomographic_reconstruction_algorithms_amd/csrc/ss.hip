@@ -12,16 +12,22 @@
 // Arithmetic is the reference's, operation for operation (ARITH FAST: its -ffast-math
 // build; IEEE: the C as written); every update rounds to float after a double sum.
 //   forward: one thread per bin steps u in order -- the reference's own loop;
-//   back:    one thread per pixel gathers, per view in order, the 2-4 bins whose line
+//   back:    one thread per pixel gathers, per view in order, the up to 3 bins whose line
 //            can reach it, in increasing t: each (view, bin) reaches a pixel at most once,
 //            so the pixel receives the reference's terms in the reference's order.
 // No atomics; both directions are bit-identical to the reference wherever its samples
 // stay inside the image.
+//
+// The forward is bound by its gathers (a lane per bin reads the sampled index, so one of the
+// two view families strides by rows) and the back by instruction issue; us before and after
+// lockstep steps, the transposed copy and the two or three candidate bins, method 1:
+// 511^2 x 360 views forward 346 -> 231, back 397 -> 331; 512^2 x 361 x 2 slices 767 -> 306 and
+// 540 -> 441; 1024^2 x 720 3398 -> 1126 and 2301 -> 1665; 64^2 x 45 19 -> 19.5 and 43 -> 40.
 #include "epilogue.h"
 
 namespace itomo {
 
-constexpr int kSsFwdBlock = 256;
+constexpr int kSsFwdBlock = 64;
 constexpr int kSsBackX = 64, kSsBackY = 4;
 
 // Sampled coordinate of stepped index u on line t (radon_ss.c:124,135,162,173).
@@ -76,47 +82,82 @@ __device__ __forceinline__ float ss_upd0(float acc, double rab, float v)
     return (float)__dadd_rn((double)acc, __dmul_rn(rab, (double)v));
 }
 
-// One thread per (sinogram row, bin).  Epilogues: STORE, RECIP.
+// One thread per (sinogram row, bin).  Epilogues: STORE, RECIP.  The lanes of a wave, 64
+// neighbouring bins, step the same u together, from the first lane's start to the last
+// lane's end, and read the orientation in which the sampled index is contiguous (imageT, when
+// there is one, for views that step columns): a wave's loads are then nearly contiguous, and
+// four steps' loads are in flight before the first is added.
 template <int ARITH, int METHOD, int EPI, bool ONES>
 __global__ void __launch_bounds__(kSsFwdBlock)
 ss_fwd_kernel(const SsView* __restrict__ geom, const int2* __restrict__ range, int npix,
-              int nang, const float* __restrict__ image, float* __restrict__ out,
-              int64_t img_stride, int64_t sino_stride, int accumulate, EpiArgs e)
+              int nang, const float* __restrict__ image, const float* __restrict__ imageT,
+              float* __restrict__ out, int64_t img_stride, int64_t sino_stride, int accumulate,
+              EpiArgs e)
 {
+    constexpr int U = 4;
     const int k = blockIdx.x * kSsFwdBlock + threadIdx.x;
-    if (k >= npix) return;
+    const bool active = k < npix;
     const int r = blockIdx.y, z = blockIdx.z;
     const int v = nang - 1 - r;
-    image += (int64_t)z * img_stride;
     const int64_t soff = (int64_t)z * sino_stride, o = (int64_t)r * npix + k;
-    float acc = (EPI == EPI_STORE && accumulate) ? out[soff + o] : 0.0f;
+    float acc = (EPI == EPI_STORE && accumulate && active) ? out[soff + o] : 0.0f;
     const int nh = npix >> 1;
-    if (k < 2 * nh) {  // odd npix: the last bin has no line (radon_ss.c:109)
-        const SsView g = geom[v];
-        const int2 ur = range[(int64_t)v * npix + k];
-        const float tf = (float)(k - nh);
-        // stepped index u -> image (stepped, sampled) strides
-        const int64_t ss = g.ybranch ? npix : 1, sq = g.ybranch ? 1 : npix;
-        for (int u = ur.x; u < ur.y; ++u) {
+    const SsView g = geom[v];
+    // odd npix: the last bin has no line (radon_ss.c:109)
+    int2 ur = make_int2(0, 0);
+    if (k < 2 * nh) ur = range[(int64_t)v * npix + k];
+    int first = ur.x < ur.y ? ur.x : npix, last = ur.x < ur.y ? ur.y : -npix;
+    for (int off = 32; off > 0; off >>= 1) {
+        first = min(first, __shfl_xor(first, off, 64));
+        last = max(last, __shfl_xor(last, off, 64));
+    }
+    const float tf = (float)(k - nh);
+    // stepped index u -> image (stepped, sampled) strides
+    const bool flip = imageT && !g.ybranch;
+    const float* __restrict__ img = (flip ? imageT : image) + (int64_t)z * img_stride;
+    const int ss = g.ybranch || flip ? npix : 1, sq = g.ybranch || flip ? 1 : npix;
+    for (int u0 = first; u0 < last; u0 += U) {
+        float fa[U], fb[U], wa[U], wb[U];
+        bool oa[U], ob[U];
+#pragma unroll
+        for (int c = 0; c < U; ++c) {
+            const int u = u0 + c;
+            const bool in = u >= ur.x && u < ur.y;
             const float q = ss_q<ARITH>(g, u, tf);
-            const float* __restrict__ line = image + (int64_t)(u + nh) * ss;
+            const float* __restrict__ line = img + (unsigned)((u + nh) * ss);
+            fb[c] = 1.0f;
+            wb[c] = 0.0f;
             if (METHOD == 0) {
                 const int p = ss_round<ARITH>(q) + nh;
-                if (p >= 0 && p < npix)
-                    acc = ss_upd0<ARITH>(acc, g.rab, ONES ? 1.0f : line[p * sq]);
+                oa[c] = in && p >= 0 && p < npix;
+                ob[c] = false;
+                fa[c] = ONES || !oa[c] ? 1.0f : line[__umul24(p, sq)];
+                wa[c] = 1.0f;
             } else {
                 float fl, w, wl;
                 ss_split<ARITH>(q, fl, w, wl);
                 const int p = (int)fl + nh;
-                if (p >= 0 && p <= npix - 1)
-                    acc = ss_fwd_upd<ARITH>(acc, wl, g.rab, ONES ? 1.0f : line[p * sq]);
-                if (p + 1 >= 0 && p + 1 <= npix - 1)
-                    acc = ss_fwd_upd<ARITH>(acc, w, g.rab, ONES ? 1.0f : line[(p + 1) * sq]);
+                oa[c] = in && p >= 0 && p <= npix - 1;
+                ob[c] = in && p + 1 >= 0 && p + 1 <= npix - 1;
+                fa[c] = ONES || !oa[c] ? 1.0f : line[__umul24(p, sq)];
+                fb[c] = ONES || !ob[c] ? 1.0f : line[__umul24(p + 1, sq)];
+                wa[c] = wl;
+                wb[c] = w;
+            }
+        }
+#pragma unroll
+        for (int c = 0; c < U; ++c) {
+            const float na = METHOD == 0 ? ss_upd0<ARITH>(acc, g.rab, fa[c])
+                                         : ss_fwd_upd<ARITH>(acc, wa[c], g.rab, fa[c]);
+            acc = oa[c] ? na : acc;
+            if (METHOD != 0) {
+                const float nb = ss_fwd_upd<ARITH>(acc, wb[c], g.rab, fb[c]);
+                acc = ob[c] ? nb : acc;
             }
         }
     }
     double p0 = 0.0;
-    out[soff + o] = epi_forward<EPI>(acc, o, soff, z, e, &p0);
+    if (active) out[soff + o] = epi_forward<EPI>(acc, o, soff, z, e, &p0);
 }
 
 // One thread per pixel (memory row R, column Q); 64 columns x 4 rows per block.
@@ -134,38 +175,59 @@ ss_back_kernel(const SsView* __restrict__ geom, const int2* __restrict__ range, 
     double p1 = 0.0, p2 = 0.0;
     if (Q < npix && R < npix) {
         const int nh = npix >> 1;
-        // bins whose line passes within |b| * (1 + margin) of the pixel centre in the
-        // sampled coordinate: t = u a + q b with q in [P - 1, P + 1]
-        const double margin = 0.01 + npix * 0x1p-16;
+        // Bins whose line passes within |b| (and a margin) of the pixel centre in the sampled
+        // coordinate, t = u a + q b with q in [P - 1, P + 1]: the integers within |b| <= 1 of
+        // tc = u a + P b, so two of them, or three where |b| is within the margin of 1 (float
+        // rounding of tc and q stays below npix * 2^-21).  Each is then decided exactly.  A
+        // pixel two or more pixels inside the image needs no look at the bins' ranges: a line
+        // that samples next to it enters and leaves the square at least one step from u.
+        const float margin = 0.01f + npix * 0x1p-18f;
         float acc = (EPI == EPI_STORE && accumulate) ? out[ioff + o] : 0.0f;
+        const bool inner = Q >= 2 && R >= 2 && Q < 2 * nh - 3 && R < 2 * nh - 3;
         for (int v = 0; v < nang; ++v) {
             const SsView g = geom[v];
             const int u = (g.ybranch ? R : Q) - nh;  // stepped
             const int P = (g.ybranch ? Q : R) - nh;  // sampled
-            const double tc = (double)u * g.a + (double)P * g.b;
-            const double hw = fabs((double)g.b) * (1.0 + margin) + margin;
-            const int t0 = (int)fmax((double)-nh, ceil(tc - hw));
-            const int t1 = (int)fmin((double)(nh - 1), floor(tc + hw));
+            const float tc = __builtin_fmaf((float)u, g.a, __fmul_rn((float)P, g.b));
+            const float hw = __builtin_fmaf(fabsf(g.b), 1.0f + margin, margin);
+            const float tf = ceilf(tc - hw);
             const float* __restrict__ row = sino + (int64_t)(nang - 1 - v) * npix;
             const int2* __restrict__ rg = range + (int64_t)v * npix;
-            for (int t = t0; t <= t1; ++t) {
-                const int k = t + nh;
-                const int2 ur = rg[k];
-                if (u < ur.x || u >= ur.y) continue;
-                const float q = ss_q<ARITH>(g, u, (float)t);
+            float wt[3], val[3];
+            bool ok[3];
+            auto look = [&](int c) {
+                const float tcf = __fadd_rn(tf, (float)c);
+                const int t = (int)tcf, k = t + nh;
+                ok[c] = t >= -nh && t < nh;
+                const float q = ss_q<ARITH>(g, u, tcf);
                 if (METHOD == 0) {
-                    if (ss_round<ARITH>(q) == P)
-                        acc = ss_upd0<ARITH>(acc, g.rab, ONES ? 1.0f : row[k]);
+                    ok[c] = ok[c] && ss_round<ARITH>(q) == P;
+                    wt[c] = 1.0f;
                 } else {
                     float fl, w, wl;
                     ss_split<ARITH>(q, fl, w, wl);
                     const int p = (int)fl;
-                    if (p == P)
-                        acc = ss_back_upd<ARITH>(acc, wl, g.rab, ONES ? 1.0f : row[k]);
-                    else if (p + 1 == P)
-                        acc = ss_back_upd<ARITH>(acc, w, g.rab, ONES ? 1.0f : row[k]);
+                    ok[c] = ok[c] && (p == P || p + 1 == P);
+                    wt[c] = p == P ? wl : w;
                 }
-            }
+                if (!inner && ok[c]) {
+                    const int2 ur = rg[k];
+                    ok[c] = u >= ur.x && u < ur.y;
+                }
+                val[c] = ONES || !ok[c] ? 1.0f : row[k];
+            };
+            auto add = [&](int c) {
+                const float na = METHOD == 0 ? ss_upd0<ARITH>(acc, g.rab, val[c])
+                                             : ss_back_upd<ARITH>(acc, wt[c], g.rab, val[c]);
+                acc = ok[c] ? na : acc;
+            };
+            look(0);
+            look(1);
+            const bool third = __any(tf + 2.0f <= tc + hw);
+            if (third) look(2);
+            add(0);
+            add(1);
+            if (third) add(2);
         }
         const float xo = epi_updates_x(EPI) ? out[ioff + o] : 0.0f;
         out[ioff + o] = epi_back<EPI>(acc, xo, o, z, e, &p1, &p2);
@@ -179,26 +241,26 @@ ss_back_kernel(const SsView* __restrict__ geom, const int2* __restrict__ range, 
 namespace {
 
 template <int ARITH, int METHOD, int EPI, bool ONES>
-void launch_ss_fwd(const Plan& p, const float* image, float* out, int nslices, int accumulate,
-                   const EpiArgs& e, hipStream_t st)
+void launch_ss_fwd(const Plan& p, const float* image, const float* imageT, float* out,
+                   int nslices, int accumulate, const EpiArgs& e, hipStream_t st)
 {
     dim3 grid((p.npix + kSsFwdBlock - 1) / kSsFwdBlock, p.nang, nslices);
     ss_fwd_kernel<ARITH, METHOD, EPI, ONES><<<grid, kSsFwdBlock, 0, st>>>(
-        (const SsView*)p.d_geom, (const int2*)p.d_range, p.npix, p.nang, image, out,
+        (const SsView*)p.d_geom, (const int2*)p.d_range, p.npix, p.nang, image, imageT, out,
         (int64_t)p.npix * p.npix, (int64_t)p.nang * p.npix, accumulate, e);
 }
 
 template <int ARITH, int METHOD>
-int dispatch_ss_fwd(const Plan& p, int epi, int ones, const float* image, float* out,
-                    int nslices, int accumulate, const EpiArgs& e, hipStream_t st)
+int dispatch_ss_fwd(const Plan& p, int epi, int ones, const float* image, const float* imageT,
+                    float* out, int nslices, int accumulate, const EpiArgs& e, hipStream_t st)
 {
     if (epi == EPI_STORE) {
-        if (ones) launch_ss_fwd<ARITH, METHOD, EPI_STORE, true>(p, image, out, nslices, accumulate, e, st);
-        else launch_ss_fwd<ARITH, METHOD, EPI_STORE, false>(p, image, out, nslices, accumulate, e, st);
+        if (ones) launch_ss_fwd<ARITH, METHOD, EPI_STORE, true>(p, image, imageT, out, nslices, accumulate, e, st);
+        else launch_ss_fwd<ARITH, METHOD, EPI_STORE, false>(p, image, imageT, out, nslices, accumulate, e, st);
         return ITOMO_OK;
     }
     if (epi == EPI_RECIP && ones) {
-        launch_ss_fwd<ARITH, METHOD, EPI_RECIP, true>(p, image, out, nslices, 0, e, st);
+        launch_ss_fwd<ARITH, METHOD, EPI_RECIP, true>(p, image, imageT, out, nslices, 0, e, st);
         return ITOMO_OK;
     }
     return set_error(ITOMO_EINVAL, "ss forward: unsupported epilogue %d", epi);
@@ -243,6 +305,14 @@ int dispatch_ss_back(const Plan& p, int epi, int ones, const float* sino, float*
 
 }  // namespace
 
+// Whether a forward call reads a transposed copy: once its waves fill the GPU, contiguous loads
+// are worth the copy (us with and without: 257^2 x 180 102 and 85, 511^2 x 360 230 and 255,
+// 512^2 x 361 x 2 slices 306 and 569, 1024^2 x 720 1125 and 2196).
+static bool ss_transposes(const Plan& p, int nslices)
+{
+    return (int64_t)((p.npix + 63) / 64) * p.nang * nslices >= 2048;
+}
+
 int ss_forward_epi(const Plan& p, int epi, int ones, const float* image, float* out,
                    int nslices, int accumulate, const EpiArgs& e, hipStream_t st,
                    int* blocks_per_slice)
@@ -255,15 +325,17 @@ int ss_forward_epi(const Plan& p, int epi, int ones, const float* image, float* 
                                         blocks_per_slice);
     }
     if (blocks_per_slice) *blocks_per_slice = 0;
+    const TransposedCopy tc(p, !ones && ss_transposes(p, nslices), image, nslices, st);
+    const float* imageT = tc.get();
     int rc;
     if (p.arith == ITOMO_ARITH_FAST)
         rc = p.method == 0
-                 ? dispatch_ss_fwd<ITOMO_ARITH_FAST, 0>(p, epi, ones, image, out, nslices, accumulate, e, st)
-                 : dispatch_ss_fwd<ITOMO_ARITH_FAST, 1>(p, epi, ones, image, out, nslices, accumulate, e, st);
+                 ? dispatch_ss_fwd<ITOMO_ARITH_FAST, 0>(p, epi, ones, image, imageT, out, nslices, accumulate, e, st)
+                 : dispatch_ss_fwd<ITOMO_ARITH_FAST, 1>(p, epi, ones, image, imageT, out, nslices, accumulate, e, st);
     else
         rc = p.method == 0
-                 ? dispatch_ss_fwd<ITOMO_ARITH_IEEE, 0>(p, epi, ones, image, out, nslices, accumulate, e, st)
-                 : dispatch_ss_fwd<ITOMO_ARITH_IEEE, 1>(p, epi, ones, image, out, nslices, accumulate, e, st);
+                 ? dispatch_ss_fwd<ITOMO_ARITH_IEEE, 0>(p, epi, ones, image, imageT, out, nslices, accumulate, e, st)
+                 : dispatch_ss_fwd<ITOMO_ARITH_IEEE, 1>(p, epi, ones, image, imageT, out, nslices, accumulate, e, st);
     if (rc) return rc;
     return check_hip(hipGetLastError(), "ss forward launch");
 }
