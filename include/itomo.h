@@ -136,7 +136,7 @@ int itomo_plan_set_shapes(itomo_plan *plan, int fwd_variant, int back_variant);
 int itomo_plan_get_shapes(const itomo_plan *plan, int *fwd_variant, int *back_variant);
 
 /* Ray-driven plans cache the projector's exact system matrix in HBM (both directions,
- * 8 bytes per walk step, at most 8 GiB together) on their first iteration call and
+ * 4 bytes per walk step, at most 5 GiB together) on their first iteration call and
  * replay it in every later projection, bitwise equal to the walks.  No counterpart in
  * the reference (whose radon_rd.c walks every time).  mode: ITOMO_RDM_QUERY reports the
  * cached bytes (0 if none), ITOMO_RDM_BUILD builds it now (synchronous on stream; 0

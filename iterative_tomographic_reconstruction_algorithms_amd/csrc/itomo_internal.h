@@ -99,17 +99,14 @@ struct Plan {
     mutable size_t scratch_bytes;
     // Ray-driven plans: the projector's exact system matrix cached in HBM (rd.hip), built
     // on the first iteration call when it fits kRdMatrixMaxBytes.  Forward rows (one per
-    // bin) and back columns (one per pixel) in chunks of 64 outputs, entry j of lane k of
-    // a chunk at off[chunk] + 64 j + k, cnt[out] = the output's own number of entries; an
-    // entry is {input index, length bits}.
+    // bin) and back columns (one per pixel) in chunks of 64 outputs, 32-bit words from
+    // off[chunk] to off[chunk + 1].
     mutable int rd_mat_state;   // 0: not tried, 1: built, -1: declined
     mutable int rd_mat_pinned;  // 1 once a stream capture has recorded a launch using it
-    mutable int2* rdf_ent;
+    mutable unsigned* rdf_ent;
     mutable int64_t* rdf_off;
-    mutable int* rdf_cnt;
-    mutable int2* rdb_ent;
+    mutable unsigned* rdb_ent;
     mutable int64_t* rdb_off;
-    mutable int* rdb_cnt;
     mutable size_t rd_mat_bytes;
     // Pixel-driven and slant-stacking plans: the buffer of TransposedCopy, grown on first use.
     mutable std::mutex copy_mutex;
@@ -118,8 +115,8 @@ struct Plan {
     mutable hipEvent_t copy_read;  // recorded behind the last launch that reads the copy
 };
 
-// Largest ray-driven system matrix a plan caches (forward and back entries together).
-constexpr size_t kRdMatrixMaxBytes = (size_t)8 << 30;
+// Largest ray-driven system matrix a plan caches (forward and back words together).
+constexpr size_t kRdMatrixMaxBytes = (size_t)5 << 30;
 // Builds the ray-driven system matrix of p if not tried yet and allowed (no caller-owned
 // scratch region active); synchronous.  Returns ITOMO_OK whether built or declined.
 int rd_matrix_ensure(const Plan& p, hipStream_t st);

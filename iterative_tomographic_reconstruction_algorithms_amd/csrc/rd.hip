@@ -16,6 +16,7 @@
 // parameters, computed exactly as the walk computes them.  Updates reach each pixel in
 // the reference's own order: both projections are bit-identical to the reference's.
 #include <algorithm>
+#include <new>
 #include <vector>
 
 #include "epilogue.h"
@@ -164,62 +165,122 @@ __device__ float rd_walk(float acc, const float* __restrict__ img_in, int npix,
     return acc;
 }
 
-// Ray views whose neighbouring bins lie in neighbouring image rows (|sin| > |cos|: sub-ray
-// i lies on y c - x s = tau(i), so one bin further moves a step of (-s, c) in (row,
-// column)) record their forward entries against the transposed image, so that the 64
-// lanes of a wave (64 neighbouring bins) gather from neighbouring addresses.
-__device__ __forceinline__ bool rd_fwd_transposed(const RdView& g)
+// Whether a bin's forward words index the transposed image.  After equally many steps the walks
+// that start on the square's x edges are in the same image row, in neighbouring columns, and
+// those that start on its y edges in the same column: the latter read the transposed copy, so
+// that the lanes of a wave (64 neighbouring bins) gather from neighbouring addresses.  (Chosen
+// per view, by the steeper axis, and with the sub-rays of a list unaligned, a wave's gather
+// touches up to 64 lines: 256^2 x 304 views, 263 us a call against 158.)
+template <int ARITH>
+__device__ __forceinline__ bool rd_fwd_transposed(const RdView& g, int b, int npix)
 {
-    return g.kind == RD_RAYS && fabsf(g.s) > fabsf(g.c);
+    float p1[2], p2[2];
+    rd_endpoints<ARITH>(6 * b + 3, npix, g, p1, p2);
+    return fabsf(p1[0]) != (float)(int)(npix * 0.5);
 }
 
 // The cached system matrix of a plan (see rd_matrix_ensure), or all null.
 struct RdMat {
-    const int2* ent;
+    const unsigned* ent;
     const int64_t* off;
-    const int* cnt;
 };
 
-// Replays one output's cached entries e[0], e[64], ... (n of them) into acc, in order.
-// The chain of updates is serial (each rounds to float), so the latency of the entry
-// loads and of the gathers they index is hidden by keeping kReplayDepth of each in
-// flight: a batch's gathers and the next batch's entry loads are issued before the
-// batch's updates.  Entries with the top bit set belong to a row-sum or column-sum view
-// and are added plainly.
-constexpr int kReplayDepth = 32;
+// A matrix word: two bits of code, 30 of payload.  A credited length l is a float in [0, 2),
+// whose two top bits are zero (the recording counts any that is not, and the matrix is then
+// declined), so a step and its length fit 32 bits without loss.
+//   forward: codes 0, 1, 2 move the image index by a, b, a + b (RdSteps) and credit l there;
+//   back:    codes 0, 1 move the sinogram index by 0, 1 and credit l from there, code 2 sets
+//            it and adds the bin plainly (row-sum and column-sum views);
+//   both:    code 3 sets the index and credits nothing (starts, and the padding).
+constexpr unsigned kRdPayload = 0x3fffffffu;
+constexpr int kRdBatch = 16;               // words of a lane handled together, four 16-byte loads
+constexpr int kRdRing = 4;                 // batches in registers; lists are padded to a ring
+constexpr int kRdPad = kRdBatch * kRdRing;
 
-template <int ARITH, bool ONES, bool BACK>
-__device__ __forceinline__ float rd_replay(float acc, const int2* __restrict__ e, int n,
-                                           const float* __restrict__ src)
+// The index steps of a bin's forward words: (row, column) moves along the view's usual walk.
+struct RdSteps {
+    int a, b;
+};
+
+__device__ __forceinline__ RdSteps rd_fwd_steps(const RdView& g, int npix, bool transposed)
 {
-    int2 q[kReplayDepth];
+    const int si = transposed ? 1 : npix, sj = transposed ? npix : 1;
+    return {g.lt_half_pi ? si : -si, sj};
+}
+
+// Replays one output's words (nb batches of them, a multiple of kRdRing) into acc, in order.
+// What bounds it is the stream of words: it is read once per call, and there are only about as
+// many waves as SIMDs (a bin or a pixel is one serial chain of rounded updates), so each wave
+// keeps three batches of its lanes' words in flight (12 KB) and the gathers of one batch while
+// it updates the one before.  No load is predicated: batches past the end repeat the last one
+// and the padding gathers index 0.
+template <int ARITH, bool ONES, bool BACK>
+__device__ __forceinline__ float rd_replay(float acc, const uint4* __restrict__ e, int nb,
+                                           const float* __restrict__ src, unsigned last,
+                                           RdSteps st)
+{
+    if (nb <= 0) return acc;
+    unsigned q[kRdRing][kRdBatch];
+    float v[2][kRdBatch];
+    unsigned idx = 0;
+    const int ab = st.a + st.b;
+    auto load = [&](unsigned (&d)[kRdBatch], int batch) {
+        const uint4* p = e + (int64_t)min(batch, nb - 1) * (kRdBatch / 4 * 64);
 #pragma unroll
-    for (int u = 0; u < kReplayDepth; ++u)
-        q[u] = u < n ? e[(int64_t)u * 64] : make_int2(0, 0);
-    for (int j = 0; j < n; j += kReplayDepth) {
-        float v[kReplayDepth];
+        for (int g = 0; g < kRdBatch / 4; ++g) {
+            const uint4 w = p[g * 64];
+            d[4 * g] = w.x;
+            d[4 * g + 1] = w.y;
+            d[4 * g + 2] = w.z;
+            d[4 * g + 3] = w.w;
+        }
+    };
+    auto gather = [&](const unsigned (&d)[kRdBatch], float (&x)[kRdBatch]) {
 #pragma unroll
-        for (int u = 0; u < kReplayDepth; ++u)
-            v[u] = (ONES || j + u >= n) ? 1.0f : src[q[u].x & 0x7fffffff];
-        int2 qn[kReplayDepth];
-#pragma unroll
-        for (int u = 0; u < kReplayDepth; ++u)
-            qn[u] = j + kReplayDepth + u < n ? e[(int64_t)(j + kReplayDepth + u) * 64]
-                                             : make_int2(0, 0);
-#pragma unroll
-        for (int u = 0; u < kReplayDepth; ++u) {
-            if (j + u < n) {
-                const float l = __int_as_float(q[u].y);
-                if (q[u].x < 0)
-                    acc = __fadd_rn(acc, v[u]);
-                else if (BACK)
-                    acc = rd_back_update<ARITH>(acc, v[u], l);
-                else
-                    acc = rd_fwd_update<ARITH>(acc, v[u], l);
+        for (int u = 0; u < kRdBatch; ++u) {
+            const unsigned w = d[u], pay = w & kRdPayload;
+            if (BACK) {
+                idx = w >= 0x80000000u ? pay : idx + (w >> 30);
+                x[u] = ONES ? 1.0f : src[idx];
+            } else {
+                const int step = w >= 0x80000000u ? ab : (w & 0x40000000u) ? st.b : st.a;
+                idx = w >= 0xc0000000u ? pay : idx + (unsigned)step;
+                x[u] = ONES ? 1.0f : src[min(idx, last)];   // a start may lie one step outside
             }
-            q[u] = qn[u];
+        }
+    };
+    auto update = [&](const unsigned (&d)[kRdBatch], const float (&x)[kRdBatch]) {
+#pragma unroll
+        for (int u = 0; u < kRdBatch; ++u) {
+            const float l = __uint_as_float(d[u] & kRdPayload);
+            float n;
+            if (BACK)
+                n = d[u] >= 0x80000000u ? __fadd_rn(acc, x[u]) : rd_back_update<ARITH>(acc, x[u], l);
+            else
+                n = rd_fwd_update<ARITH>(acc, x[u], l);
+            acc = d[u] >= 0xc0000000u ? acc : n;
+        }
+    };
+#pragma unroll
+    for (int r = 0; r < kRdRing - 1; ++r) load(q[r], r);
+#pragma unroll
+    for (int u = 0; u < kRdBatch; ++u) {
+        q[kRdRing - 1][u] = 0xc0000000u;
+        v[1][u] = 0.0f;
+    }
+#pragma unroll 1
+    for (int j = 0; j < nb; j += kRdRing) {
+#pragma unroll
+        for (int r = 0; r < kRdRing; ++r) {
+            constexpr int kPrev = kRdRing - 1;
+            gather(q[r], v[r & 1]);
+            __builtin_amdgcn_sched_barrier(0);
+            update(q[(r + kPrev) % kRdRing], v[(r & 1) ^ 1]);
+            load(q[(r + kPrev) % kRdRing], j + r + kPrev);
+            __builtin_amdgcn_sched_barrier(0);
         }
     }
+    update(q[kRdRing - 1], v[(kRdRing - 1) & 1]);
     return acc;
 }
 
@@ -239,14 +300,20 @@ rd_fwd_kernel(const RdView* __restrict__ geom, int npix, const float* __restrict
     double p0 = 0.0;
     if (active) {
         float acc = (EPI == EPI_STORE && accumulate) ? out[soff + o] : 0.0f;
-        if (mat.ent) {
-            // the bin's cached updates, in order (bitwise the walk's or the sum's), from
-            // the image or its transpose as they were recorded
+        const float* imgT = imageT + (int64_t)z * img_stride;
+        if (mat.ent && g.kind == RD_RAYS) {
+            // the bin's cached updates, in order (bitwise the walk's), from the image or its
+            // transpose as they were recorded
             const int64_t chunk = (int64_t)v * gridDim.x + blockIdx.x;
-            const float* src = (!ONES && rd_fwd_transposed(g))
-                                   ? imageT + (int64_t)z * img_stride : image;
-            acc = rd_replay<ARITH, ONES, false>(acc, mat.ent + mat.off[chunk] + threadIdx.x,
-                                                mat.cnt[(int64_t)v * npix + b], src);
+            const int64_t off = mat.off[chunk];
+            const bool t = rd_fwd_transposed<ARITH>(g, b, npix);
+            acc = rd_replay<ARITH, ONES, false>(
+                acc, (const uint4*)(mat.ent + off) + threadIdx.x,
+                (int)((mat.off[chunk + 1] - off) / (64 * kRdBatch)),
+                t ? imgT : image, (unsigned)(npix * npix - 1), rd_fwd_steps(g, npix, t));
+        } else if (mat.ent && g.kind == RD_ROWSUM && !ONES) {
+#pragma unroll 8
+            for (int j = 0; j < npix; ++j) acc = __fadd_rn(acc, imgT[(int64_t)j * npix + b]);
         } else if (g.kind == RD_COLSUM) {
             const int i = npix - 1 - b;  // bin N-1-i <- column i, i >= 1
             if (i >= 1)
@@ -373,27 +440,51 @@ rd_back_gather_kernel(const RdView* __restrict__ geom, int nang, int npix,
 // ---- the cached system matrix ------------------------------------------------------
 //
 // With 288 GB of HBM per GPU the exact system matrix of a small ray-driven geometry fits
-// many times over (8 bytes per walk step, once per direction), and replaying it turns
-// both projections into streaming passes with full occupancy instead of latency-bound
-// walks.  The entries are what the walks compute: per bin the steps of its five sub-rays
-// that enter an image cell, in walk order, {pixel, credited length} (the pixel's index in
-// the transposed image for views whose bins step along image rows; a row-sum or
-// column-sum view's bin: its pixels {pixel | 1 << 31}, in order); per pixel, in view
-// order, the row-sum and column-sum views' bins {bin | 1 << 31} and every sub-ray step
-// entering it {bin, length}.  Replaying them in that order with the same update
-// arithmetic gives the walks' results bit for bit.
+// many times over (4 bytes per walk step, once per direction), and replaying it turns
+// both projections into streaming passes instead of latency-bound walks.  The words are what
+// the walks compute: per bin the steps of its five sub-rays that enter an image cell, in walk
+// order (indices into the image or its transpose, rd_fwd_transposed); per
+// pixel, in view order, the row-sum and column-sum views' bins and every sub-ray step entering
+// it.  Replaying them in that order with the same update arithmetic gives the walks' results
+// bit for bit.
+// Word n of lane k of a 64-output chunk lies at off[chunk] + 256 (n/4) + 4 k + n%4.
+// Against eight-byte {index, length} entries loaded in predicated batches, us per call forward
+// and back: 64^2 x 45 views 76 -> 31 and 39 -> 24, 256^2 x 304 404 -> 158 and 295 -> 146 (3.6
+// and 4.3 TB/s of words), two slices of it 826 -> 262 and 367 -> 280.
 
-// An entry of a row-sum or column-sum view: its input index with the top bit set.
-__device__ __forceinline__ int rd_sum_flag(int index)
-{
-    return (int)((unsigned)index | 0x80000000u);
-}
+// Writes (FILL) or counts an output's words.
+template <bool FILL>
+struct RdWords {
+    unsigned* out;
+    int n = 0;
+    unsigned bad = 0;
+
+    __device__ __forceinline__ void put(unsigned code, unsigned payload)
+    {
+        if (FILL) out[(n >> 2) * 256 + (n & 3)] = code << 30 | payload;
+        ++n;
+    }
+    __device__ __forceinline__ void credit(unsigned code, float l)
+    {
+        const unsigned u = __float_as_uint(l);
+        bad |= u & ~kRdPayload;
+        put(code, u & kRdPayload);
+    }
+    __device__ __forceinline__ void pad(int words)
+    {
+        if (FILL)
+            while (n < words) put(3, 0);
+        n = words;
+    }
+    // The number of words, or -1 when a length does not fit.
+    __device__ __forceinline__ int count() const { return bad ? -1 : n; }
+};
 
 // One sub-ray walk of radon_rd.c:15-71 (the steps of rd_walk) recording the steps that
-// enter an image cell: FILL == false counts them, FILL == true writes them to out[64 j].
+// enter an image cell.
 template <int ARITH, bool FILL>
-__device__ int rd_walk_record(int npix, const float p1[2], const float p2[2], int2* out, int j,
-                              bool transposed)
+__device__ void rd_walk_record(int npix, const float p1[2], const float p2[2],
+                               RdWords<FILL>& words, RdSteps st, bool transposed)
 {
     const int nh = (int)(npix * 0.5);
     const float d0 = __fsub_rn(p2[0], p1[0]), d1 = __fsub_rn(p2[1], p1[1]);
@@ -411,16 +502,22 @@ __device__ int rd_walk_record(int npix, const float p1[2], const float p2[2], in
     float ax = (float)__ddiv_rn(__dsub_rn(__dadd_rn((double)ii, hx), p1x), dd0);
     float ay = (float)__ddiv_rn(__dsub_rn(__dadd_rn((double)jj, hy), p1y), dd1);
     const int cap = 4 * npix + 16;
+    const int mi = (int)dx * (transposed ? 1 : npix), mj = (int)dy * (transposed ? npix : 1);
+    bool live = false;   // the step before was recorded
     for (int step = 0; alpha <= 1.0f && step < cap; ++step) {
+        int move;
         if (ax < ay) {
+            move = mi;
             alpha = ax;
             ii = (int)__fadd_rn((float)ii, dx);
             ax = (float)__ddiv_rn(__dsub_rn(__dadd_rn((double)ii, hx), p1x), dd0);
         } else if (ax > ay) {
+            move = mj;
             alpha = ay;
             jj = (int)__fadd_rn((float)jj, dy);
             ay = (float)__ddiv_rn(__dsub_rn(__dadd_rn((double)jj, hy), p1y), dd1);
         } else if (ax == ay) {
+            move = mi + mj;
             alpha = ay;
             ii = (int)__fadd_rn((float)ii, dx);
             jj = (int)__fadd_rn((float)jj, dy);
@@ -432,74 +529,75 @@ __device__ int rd_walk_record(int npix, const float p1[2], const float p2[2], in
         const float l = __fmul_rn(__fsub_rn(alpha, alpha_old), incr);
         const int i = ii + nh, jc = jj + nh;
         if (i > 0 && i < npix && jc > 0 && jc < npix) {
-            if (FILL)
-                out[(int64_t)j * 64] =
-                    make_int2(transposed ? jc * npix + i : i * npix + jc, __float_as_int(l));
-            ++j;
+            const int index = transposed ? jc * npix + i : i * npix + jc;
+            const int code = move == st.a ? 0 : move == st.b ? 1 : move == st.a + st.b ? 2 : -1;
+            // the cell before lies at most one step outside the image, so its index is >= 0
+            if (code < 0 || !live) words.put(3, (unsigned)(index - (code < 0 ? st.a : move)));
+            words.credit(code < 0 ? 0 : code, l);
+            live = true;
+        } else {
+            live = false;
         }
         alpha_old = alpha;
     }
-    return j;
 }
 
-// Forward rows: one thread per (bin, view), as rd_fwd_kernel: the sum views' pixels in the
-// order radon_rd.c:95-115 adds them, else the five sub-rays' steps.
+// Forward rows: one thread per (bin, view), as rd_fwd_kernel: the five sub-rays' steps (a sum
+// view has none: its bins add image rows or columns).
 template <int ARITH, bool FILL>
 __global__ void __launch_bounds__(64)
 rd_fwd_record_kernel(const RdView* __restrict__ geom, int npix, int* __restrict__ cnt,
-                     int2* __restrict__ ent, const int64_t* __restrict__ off)
+                     unsigned* __restrict__ ent, const int64_t* __restrict__ off)
 {
-    const int b = blockIdx.x * blockDim.x + threadIdx.x;
+    const int b = blockIdx.x * 64 + threadIdx.x;
     const int v = blockIdx.y;
-    if (b >= npix) return;
     const RdView g = geom[v];
-    int n = 0;
-    int2* out = FILL ? ent + off[(int64_t)v * gridDim.x + blockIdx.x] + threadIdx.x : nullptr;
-    if (g.kind == RD_COLSUM) {
-        const int i = npix - 1 - b;   // bin N-1-i <- column i, i >= 1
-        if (i >= 1)
-            for (int j = 0; j < npix; ++j, ++n)
-                if (FILL) out[(int64_t)n * 64] = make_int2(rd_sum_flag(j * npix + i), 0);
-    } else if (g.kind == RD_ROWSUM) {
-        for (int j = 0; j < npix; ++j, ++n)
-            if (FILL) out[(int64_t)n * 64] = make_int2(rd_sum_flag(b * npix + j), 0);
-    } else {
+    const int64_t chunk = (int64_t)v * gridDim.x + blockIdx.x;
+    RdWords<FILL> words{FILL ? ent + off[chunk] + 4 * threadIdx.x : nullptr};
+    if (g.kind == RD_RAYS) {
+        const bool t = rd_fwd_transposed<ARITH>(g, b, npix);
         for (int k = 1; k <= 5; ++k) {
-            float p1[2], p2[2];
-            rd_endpoints<ARITH>(6 * b + k, npix, g, p1, p2);
-            n = rd_walk_record<ARITH, FILL>(npix, p1, p2, out, n, rd_fwd_transposed(g));
+            if (b < npix) {
+                float p1[2], p2[2];
+                rd_endpoints<ARITH>(6 * b + k, npix, g, p1, p2);
+                rd_walk_record<ARITH, FILL>(npix, p1, p2, words, rd_fwd_steps(g, npix, t), t);
+            }
+            // the chunk's bins begin their next sub-ray together, as near to each other as they
+            // began the first (it costs no words: the longest list sets the chunk's length)
+            int m = words.n;
+            for (int off = 32; off > 0; off >>= 1) m = max(m, __shfl_xor(m, off, 64));
+            words.pad(m);
         }
     }
-    if (!FILL) cnt[(int64_t)v * npix + b] = n;
+    if (FILL)
+        words.pad((int)((off[chunk + 1] - off[chunk]) / 64));
+    else if (b < npix)
+        cnt[(int64_t)v * npix + b] = words.count();
 }
 
 // Back columns: one thread per pixel, the candidates of rd_back_gather_kernel.
 template <int ARITH, bool FILL>
 __global__ void __launch_bounds__(256)
 rd_back_record_kernel(const RdView* __restrict__ geom, int nang, int npix,
-                      int* __restrict__ cnt, int2* __restrict__ ent,
+                      int* __restrict__ cnt, unsigned* __restrict__ ent,
                       const int64_t* __restrict__ off)
 {
     const int cc = blockIdx.x * 16 + (threadIdx.x & 15);
     const int r = blockIdx.y * 16 + (threadIdx.x >> 4);
     if (r >= npix || cc >= npix) return;
     const int64_t o = (int64_t)r * npix + cc;
-    int2* out = FILL ? ent + off[o >> 6] + (o & 63) : nullptr;
+    RdWords<FILL> words{FILL ? ent + off[o >> 6] + 4 * (o & 63) : nullptr};
     const int nh = (int)(npix * 0.5);
     const int ii = r - nh, jj = cc - nh;
     const bool inner = r >= 1 && cc >= 1;
-    int n = 0;
+    int last = -2;
     for (int v = 0; v < nang; ++v) {
         const RdView g = geom[v];
         const int rowbase = v * npix;
         if (g.kind == RD_COLSUM) {
-            if (cc >= 1) {
-                if (FILL) out[(int64_t)n * 64] = make_int2(rd_sum_flag(rowbase + npix - 1 - cc), 0);
-                ++n;
-            }
+            if (cc >= 1) words.put(2, (unsigned)(last = rowbase + npix - 1 - cc));
         } else if (g.kind == RD_ROWSUM) {
-            if (FILL) out[(int64_t)n * 64] = make_int2(rd_sum_flag(rowbase + r), 0);
-            ++n;
+            words.put(2, (unsigned)(last = rowbase + r));
         } else if (inner) {
             const double sd = (double)g.s, cd = (double)g.c;
             const double tc = (double)jj * cd - (double)ii * sd;
@@ -517,64 +615,72 @@ rd_back_record_kernel(const RdView* __restrict__ geom, int nang, int npix,
                 float p1[2], p2[2], l;
                 rd_endpoints<ARITH>(i, npix, g, p1, p2);
                 if (!rd_cell_step<ARITH>(p1, p2, ii, jj, &l)) continue;
-                if (FILL) out[(int64_t)n * 64] = make_int2(rowbase + i / 6, __float_as_int(l));
-                ++n;
+                const int bin = rowbase + i / 6, d = bin - last;
+                const bool near = d == 0 || d == 1;
+                if (!near) words.put(3, (unsigned)bin);
+                words.credit(near ? d : 0, l);
+                last = bin;
             }
         }
     }
-    if (!FILL) cnt[o] = n;
+    if (FILL)
+        words.pad((int)((off[(o >> 6) + 1] - off[o >> 6]) / 64));
+    else
+        cnt[o] = words.count();
 }
 
 // Back projection from the cached columns: one thread per pixel, updates in view order
 // with rd_back_gather_kernel's arithmetic.
 template <int ARITH, bool ONES>
-__global__ void __launch_bounds__(256)
-rd_back_matrix_kernel(const int2* __restrict__ ent, const int64_t* __restrict__ off,
-                      const int* __restrict__ cnt, int npix, const float* __restrict__ sino,
-                      float* __restrict__ image, int64_t sino_stride, int64_t img_stride,
-                      int accumulate)
+__global__ void __launch_bounds__(64)
+rd_back_matrix_kernel(const unsigned* __restrict__ ent, const int64_t* __restrict__ off,
+                      int npix, const float* __restrict__ sino, float* __restrict__ image,
+                      int64_t sino_stride, int64_t img_stride, int accumulate)
 {
-    const int64_t o = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    const int64_t n2 = (int64_t)npix * npix;
-    if (o >= n2) return;
+    const int64_t o = (int64_t)blockIdx.x * 64 + threadIdx.x;
+    if (o >= (int64_t)npix * npix) return;
     image += (int64_t)blockIdx.y * img_stride;
     sino += (int64_t)blockIdx.y * sino_stride;
     const float pix = accumulate ? image[o] : 0.0f;
-    image[o] = rd_replay<ARITH, ONES, true>(pix, ent + off[o >> 6] + (o & 63), cnt[o], sino);
+    const int64_t base = off[blockIdx.x];
+    image[o] = rd_replay<ARITH, ONES, true>(
+        pix, (const uint4*)(ent + base) + threadIdx.x,
+        (int)((off[blockIdx.x + 1] - base) / (64 * kRdBatch)), sino, 0, RdSteps{0, 1});
 }
 
 namespace {
 
-// Chunk offsets of a matrix from its per-output counts: outputs are grouped 64 at a time
-// within rows of `row` outputs, and a chunk holds 64 x (its largest count) entries.
-// Returns the number of entries.
-int64_t chunk_layout(const std::vector<int>& cnt, int64_t nout, int64_t chunks_per_row,
-                     int64_t row, std::vector<int64_t>* off)
+// Chunk offsets of a matrix from its per-output word counts: outputs are grouped 64 at a time
+// within rows of `row` outputs, and a chunk holds 64 x (its largest count, padded) words; the
+// last offset is the total.  False when an output could not be recorded (a count below 0).
+bool chunk_layout(const std::vector<int>& cnt, int64_t nout, int64_t chunks_per_row,
+                  int64_t row, std::vector<int64_t>* off)
 {
     const int64_t nrows = nout / row;
-    off->assign((size_t)(nrows * chunks_per_row), 0);
+    off->assign((size_t)(nrows * chunks_per_row + 1), 0);
     int64_t total = 0;
     for (int64_t rr = 0; rr < nrows; ++rr)
         for (int64_t c = 0; c < chunks_per_row; ++c) {
-            int m = 0;
-            for (int64_t k = c * 64; k < std::min<int64_t>(row, c * 64 + 64); ++k)
-                m = std::max(m, cnt[(size_t)(rr * row + k)]);
-            (*off)[(size_t)(rr * chunks_per_row + c)] = total;
-            total += (int64_t)m * 64;
+            int64_t m = 0;
+            for (int64_t k = c * 64; k < std::min<int64_t>(row, c * 64 + 64); ++k) {
+                if (cnt[(size_t)(rr * row + k)] < 0) return false;
+                m = std::max<int64_t>(m, cnt[(size_t)(rr * row + k)]);
+            }
+            total += (m + kRdPad - 1) / kRdPad * kRdPad * 64;
+            (*off)[(size_t)(rr * chunks_per_row + c) + 1] = total;
         }
-    return total;
+    return true;
 }
 
 }  // namespace
 
 void rd_matrix_free(const Plan& p)
 {
-    void* ptrs[] = {p.rdf_ent, p.rdf_off, p.rdf_cnt, p.rdb_ent, p.rdb_off, p.rdb_cnt};
+    void* ptrs[] = {p.rdf_ent, p.rdf_off, p.rdb_ent, p.rdb_off};
     for (void* q : ptrs)
         if (q) (void)hipFree(q);
     p.rdf_ent = p.rdb_ent = nullptr;
     p.rdf_off = p.rdb_off = nullptr;
-    p.rdf_cnt = p.rdb_cnt = nullptr;
     p.rd_mat_bytes = 0;
 }
 
@@ -589,39 +695,39 @@ static bool try_alloc(T** ptr, size_t bytes)
     return false;
 }
 
+// The matrix of p, on st; returns ITOMO_OK with rd_mat_state unchanged when it is declined.
 template <int ARITH>
-static int rd_matrix_build(const Plan& p, hipStream_t st)
+static int rd_matrix_build(const Plan& p, int* cntf, int* cntb, hipStream_t st)
 {
     const int n = p.npix, V = p.nang;
     const int64_t n2 = (int64_t)n * n, nf = (int64_t)V * n;
     const int fcpr = (n + 63) / 64;                       // forward chunks per view
     const RdView* g = (const RdView*)p.d_geom;
-    if (!try_alloc(&p.rdf_cnt, nf * sizeof(int)) || !try_alloc(&p.rdb_cnt, n2 * sizeof(int)))
-        return ITOMO_OK;                                  // declined: the walks stay
     int rc;
-    rd_fwd_record_kernel<ARITH, false><<<dim3(fcpr, V), 64, 0, st>>>(g, n, p.rdf_cnt, nullptr,
+    rd_fwd_record_kernel<ARITH, false><<<dim3(fcpr, V), 64, 0, st>>>(g, n, cntf, nullptr,
                                                                        nullptr);
     rd_back_record_kernel<ARITH, false><<<dim3((n + 15) / 16, (n + 15) / 16), 256, 0, st>>>(
-        g, V, n, p.rdb_cnt, nullptr, nullptr);
+        g, V, n, cntb, nullptr, nullptr);
     rc = check_hip(hipGetLastError(), "rd matrix: count launch");
+    std::vector<int64_t> of, ob;
     std::vector<int> cf((size_t)nf), cb((size_t)n2);
-    if (!rc) rc = check_hip(hipMemcpyAsync(cf.data(), p.rdf_cnt, nf * sizeof(int),
+    if (!rc) rc = check_hip(hipMemcpyAsync(cf.data(), cntf, nf * sizeof(int),
                                            hipMemcpyDeviceToHost, st), "rd matrix: counts");
-    if (!rc) rc = check_hip(hipMemcpyAsync(cb.data(), p.rdb_cnt, n2 * sizeof(int),
+    if (!rc) rc = check_hip(hipMemcpyAsync(cb.data(), cntb, n2 * sizeof(int),
                                            hipMemcpyDeviceToHost, st), "rd matrix: counts");
     if (!rc) rc = check_hip(hipStreamSynchronize(st), "rd matrix: sync");
     if (rc) return rc;
-    std::vector<int64_t> of, ob;
-    const int64_t tf = chunk_layout(cf, nf, fcpr, n, &of);
     // back: pixels in row-major chunks of 64 (one "row" of all n2 outputs)
-    const int64_t tb = chunk_layout(cb, n2, (n2 + 63) / 64, n2, &ob);
-    const size_t bytes = (size_t)(tf + tb) * sizeof(int2);
-    if (bytes > kRdMatrixMaxBytes) return ITOMO_OK;      // declined: the walks stay
-    if (!try_alloc(&p.rdf_ent, std::max<int64_t>(tf, 1) * sizeof(int2)) ||
-        !try_alloc(&p.rdb_ent, std::max<int64_t>(tb, 1) * sizeof(int2)) ||
+    if (!chunk_layout(cf, nf, fcpr, n, &of) || !chunk_layout(cb, n2, (n2 + 63) / 64, n2, &ob))
+        return ITOMO_OK;
+    const int64_t tf = of.back(), tb = ob.back();
+    const size_t bytes = (size_t)(tf + tb) * sizeof(unsigned);
+    if (bytes > kRdMatrixMaxBytes) return ITOMO_OK;
+    if (!try_alloc(&p.rdf_ent, std::max<int64_t>(tf, 4) * sizeof(unsigned)) ||
+        !try_alloc(&p.rdb_ent, std::max<int64_t>(tb, 4) * sizeof(unsigned)) ||
         !try_alloc(&p.rdf_off, of.size() * sizeof(int64_t)) ||
         !try_alloc(&p.rdb_off, ob.size() * sizeof(int64_t)))
-        return ITOMO_OK;                                  // declined: the walks stay
+        return ITOMO_OK;
     rc = check_hip(hipMemcpy(p.rdf_off, of.data(), of.size() * sizeof(int64_t),
                              hipMemcpyHostToDevice), "rd matrix");
     if (!rc) rc = check_hip(hipMemcpy(p.rdb_off, ob.data(), ob.size() * sizeof(int64_t),
@@ -658,15 +764,26 @@ int rd_matrix_ensure(const Plan& p, hipStream_t st)
     int rc = check_hip(hipStreamIsCapturing(st, &cs), "rd matrix: capture status");
     if (rc || cs != hipStreamCaptureStatusNone) return rc;
     p.rd_mat_state = -1;
-    // upper bound of the entries (a walk takes at most 2 npix + 2 steps): skip the counting
+    // upper bound of the words (a walk takes at most 2 npix + 2 steps): skip the counting
     // passes when even a fraction of it cannot fit
-    const double bound = 16.0 * 5.0 * p.nang * (double)p.npix * (1.5 * p.npix);
+    const double bound = 8.0 * 5.0 * p.nang * (double)p.npix * (1.5 * p.npix);
     if (bound > 4.0 * (double)kRdMatrixMaxBytes) return ITOMO_OK;
-    // entry indices are 31-bit (the top bit flags a sum view's bin)
-    if ((int64_t)p.nang * p.npix >= ((int64_t)1 << 31)) return ITOMO_OK;
+    // the words hold 30-bit indices, of starts up to a row outside the image
+    const int64_t nf = (int64_t)p.nang * p.npix, n2 = (int64_t)p.npix * p.npix;
+    if (nf > kRdPayload || n2 + p.npix > kRdPayload) return ITOMO_OK;
     rc = check_hip(hipStreamSynchronize(st), "rd matrix: sync");
-    if (!rc) rc = p.arith == ITOMO_ARITH_FAST ? rd_matrix_build<ITOMO_ARITH_FAST>(p, st)
-                                              : rd_matrix_build<ITOMO_ARITH_IEEE>(p, st);
+    if (rc) return rc;
+    int *cntf = nullptr, *cntb = nullptr;
+    if (try_alloc(&cntf, nf * sizeof(int)) && try_alloc(&cntb, n2 * sizeof(int))) {
+        try {
+            rc = p.arith == ITOMO_ARITH_FAST
+                     ? rd_matrix_build<ITOMO_ARITH_FAST>(p, cntf, cntb, st)
+                     : rd_matrix_build<ITOMO_ARITH_IEEE>(p, cntf, cntb, st);
+        } catch (const std::bad_alloc&) {   // no host memory for the counts: declined
+        }
+    }
+    (void)hipFree(cntf);
+    (void)hipFree(cntb);
     if (p.rd_mat_state != 1) rd_matrix_free(p);
     return rc;
 }
@@ -690,8 +807,8 @@ int launch_rd_fwd(const Plan& p, const float* image, float* out, int nslices,
         }
     }
     const RdMat mat = p.rd_mat_state == 1
-                          ? RdMat{p.rdf_ent, p.rdf_off, p.rdf_cnt}
-                          : RdMat{nullptr, nullptr, nullptr};
+                          ? RdMat{p.rdf_ent, p.rdf_off}
+                          : RdMat{nullptr, nullptr};
     rd_fwd_kernel<ARITH, EPI, ONES><<<grid, block, 0, st>>>(
         (const RdView*)p.d_geom, p.npix, image, imageT, out, (int64_t)p.npix * p.npix,
         (int64_t)p.nang * p.npix, accumulate, e, mat);
@@ -743,11 +860,10 @@ static int rd_back_launch(const Plan& p, int ones, const float* sino, float* ima
     if (p.rd_mat_state == 1) {
         rd_matrix_note_use(p, st);
         const int64_t n2 = (int64_t)p.npix * p.npix;
-        dim3 mg((unsigned)((n2 + 255) / 256), nslices);
-#define ITOMO_RDM(A, O)                                                                  \
-    rd_back_matrix_kernel<A, O><<<mg, 256, 0, st>>>(p.rdb_ent, p.rdb_off, p.rdb_cnt, p.npix, \
-                                                   sino, image, sino_stride, img_stride,  \
-                                                   accumulate)
+        dim3 mg((unsigned)((n2 + 63) / 64), nslices);
+#define ITOMO_RDM(A, O)                                                                      \
+    rd_back_matrix_kernel<A, O><<<mg, 64, 0, st>>>(p.rdb_ent, p.rdb_off, p.npix, sino, image, \
+                                                   sino_stride, img_stride, accumulate)
         if (p.arith == ITOMO_ARITH_FAST) {
             if (ones) ITOMO_RDM(ITOMO_ARITH_FAST, true); else ITOMO_RDM(ITOMO_ARITH_FAST, false);
         } else {

@@ -109,3 +109,36 @@ def test_graph_keeps_the_matrix_it_replays():
         torch.cuda.synchronize()
         assert torch.equal(x, x_ref), "replay %d" % rep
     g.close()
+
+
+@pytest.mark.parametrize("arith,mode", [("fast", O.FAST), ("ieee", O.IEEE)])
+@pytest.mark.parametrize("n", [1, 2, 3, 7, 63, 64, 65, 130])
+def test_matrix_words_at_the_edges_of_chunks(n, arith, mode):
+    # sides around the 64-output chunks, walks through corners and along the diagonals, sum
+    # views first, between and last, negative angles and angles past 180 degrees
+    deg = [0.0, 0.3, 26.565, 44.9, 45.0, 45.1, 63.4, 89.7, 90.0, 90.3, 135.0, 179.6, 180.0,
+           200.0, 225.0, 290.0, -30.0, -135.0, 90.0]
+    ang = (np.array(deg) * np.pi / 180).astype(np.float32)
+    rng = np.random.default_rng(n)
+    x = rng.random((2, n, n), dtype=np.float32) - np.float32(0.25)
+    y = rng.random((2, ang.size, n), dtype=np.float32) - np.float32(0.25)
+    walks, matrix = Plan("rd", n, ang, arith), Plan("rd", n, ang, arith)
+    matrix.rd_matrix("build")
+    for k in range(2 if n > 1 else 0):   # at side 1 the reference never ends
+        for p in (walks, matrix):
+            np.testing.assert_array_equal(p.forward(gpu(x[k])).cpu().numpy(),
+                                          O.rd_forward(x[k], ang, mode))
+            np.testing.assert_array_equal(p.back(gpu(y[k])).cpu().numpy(),
+                                          O.rd_back(y[k], ang, mode))
+    f = matrix.forward(gpu(x))
+    assert torch.equal(f, walks.forward(gpu(x)))
+    assert torch.equal(matrix.back(gpu(y)), walks.back(gpu(y)))
+    # accumulation into values that a zero term must not change, and values that are not finite
+    x[0, n // 2, n // 2], y[0, 3, n // 2] = np.inf, np.nan
+    z = torch.full_like(f, -0.0)
+    a = matrix.forward(gpu(x), out=z.clone(), accumulate=True).cpu().numpy()
+    b = walks.forward(gpu(x), out=z.clone(), accumulate=True).cpu().numpy()
+    np.testing.assert_array_equal(a, b)
+    np.testing.assert_array_equal(np.signbit(a[~np.isnan(a)]), np.signbit(b[~np.isnan(b)]))
+    np.testing.assert_array_equal(matrix.back(gpu(y)).cpu().numpy(),
+                                  walks.back(gpu(y)).cpu().numpy())
