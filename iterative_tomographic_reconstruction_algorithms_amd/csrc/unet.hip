@@ -606,7 +606,7 @@ wgrad_tiled_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ dY,
     // word m of channel c's row from pixels a (low half) and b (high half)
     auto pair = [](const uint4& a, const uint4& b, int c) -> unsigned {
         const unsigned lo = ((const unsigned*)&a)[c >> 1], hi = ((const unsigned*)&b)[c >> 1];
-        return (c & 1) ? ((lo >> 16) | (hi & 0xffff0000u)) : ((lo & 0xffffu) | (hi << 16));
+        return __builtin_amdgcn_perm(hi, lo, (c & 1) ? 0x07060302u : 0x05040100u);
     };
     if ((int64_t)blockIdx.z < ntiles) load_unit(blockIdx.z);
 
@@ -1265,22 +1265,31 @@ int itomo_unet_wgrad(const void* x, const void* dy, int n, int h, int w, int cin
     const int64_t P = (int64_t)n * h * w;
     hipStream_t st = (hipStream_t)stream;
     if (cin == 1 && cout == 32 && ((uintptr_t)dy % 16) == 0) {
-        // about 2048 blocks, at least 4 row segments each
+        // at most one block per CU, at least 4 row segments each: every block adds its sums
+        // to the same 320 addresses (256^2 x 8: 2048, 1024, 512, 256, 128 blocks take 91, 57,
+        // 38, 38, 59 us; 512^2 52, 51, 31, 26, 30)
         const int64_t nseg = (int64_t)n * h * ((w + 63) / 64);
-        const int64_t g = std::max<int64_t>(1, std::min<int64_t>(2048, (nseg + 3) / 4));
+        const int64_t g = std::max<int64_t>(1, std::min<int64_t>(256, (nseg + 3) / 4));
         wgrad_c1_kernel<<<(unsigned)g, 256, 0, st>>>((const bf16_t*)x, (const bf16_t*)dy, dw, db,
                                                      n, h, w);
         return check_hip(hipGetLastError(), "unet_wgrad launch");
     }
     if (cin % 32 == 0 && cout % 32 == 0 && ((uintptr_t)x % 16) == 0 && ((uintptr_t)dy % 16) == 0) {
-        // 64 output channels per block where they divide, else 32; about 2048 blocks
+        // 64 output channels per block where they divide, else 32
         const bool wide = cout % 64 == 0;
         const int mb = wide ? 64 : 32;
         const int ci_chunks = cin / 32;
         const int gxw = (cout / mb) * ci_chunks;
         const int64_t ntiles = (int64_t)n * ((h + 7) / 8) * ((w + 15) / 16);
-        // at least 4 pixel tiles per block, so that the atomic adds stay few
-        int64_t gz = std::min<int64_t>(2048 / gxw, (ntiles + 3) / 4);
+        // Every block adds its 64 x 288 sums to dW atomically, and blocks of one weight tile
+        // queue at the same addresses: no more blocks than run at once (two per CU), and 8
+        // pixel tiles each, or 4 where 8 would leave CUs idle.  us with up to 2048 blocks of 4
+        // tiles or more, and so: 256^2 x 8, 96 to 32 channels 124 and 82; 128^2 x 8, 64 to 64
+        // 71 and 54, 192 to 64 128 and 75; 64^2 x 8, 128 to 128 51 and 41, 384 to 128 115 and
+        // 67.  (More than 512 blocks: 768 take 105, 54, 92, 41 and 83.)
+        int64_t gz = std::min<int64_t>(
+            512 / gxw, std::max<int64_t>((ntiles + 7) / 8,
+                                         std::min<int64_t>((ntiles + 3) / 4, 256 / gxw)));
         gz = std::max<int64_t>(1, std::min<int64_t>(gz, 65535));
         if (wide)
             wgrad_tiled_kernel<2><<<dim3((unsigned)gxw, 1, (unsigned)gz), 256, 0, st>>>(
