@@ -39,17 +39,18 @@ def alg_bytes_back(n, v):
 
 
 def forward_half_name(fwd_variant):
-    """The forward half of a SIRT step at launch shape `fwd_variant`: the transpose for
-    the column sweeps, the projection in two launches (views with at most 8 candidate
-    pixels per bin and line; the wider ones with 64-bin blocks on the plan's second stream
-    at the same time), the SIRT update pass.  Also the key of its traffic entry."""
-    return ("transpose + dd_fwd_kernel<FAST,STORE,%d> (main) beside dd_fwd_kernel<FAST,STORE,64> "
-            "(wide) + fwd_epi_kernel<SIRT_FWD>" % ([256, 128, 64][fwd_variant]))
+    """The forward half of a SIRT step at launch shape `fwd_variant`: the transpose for the
+    column sweeps, the projection in one launch (views with few candidate pixels per bin staged
+    through LDS, the wider ones along diagonals), the SIRT update pass.  Also the key of its
+    traffic entry."""
+    return ("transpose + dd_fwd_kernel<FAST,STORE,%d> + fwd_epi_kernel<SIRT_FWD>"
+            % ([256, 128, 64][fwd_variant]))
 
 
 def back_half_name(back_variant):
     """The back half (projection with the fused SIRT update) at launch shape `back_variant`."""
-    return "dd_back_kernel<FAST,SIRT_BACK,%d,%d>" % tuple([(64, 4), (32, 2), (32, 4)][back_variant])
+    return ("dd_back_kernel<FAST,SIRT_BACK,%d,%d>"
+            % tuple([(64, 4), (32, 2), (32, 4), (16, 1)][back_variant]))
 
 
 def measured_traffic(kernel):
@@ -561,7 +562,7 @@ def main():
                      # limited by VALU issue and LDS (measured below)
                      "accounting": "algorithmic bytes: 4 B gathered per pixel-view + compulsory "
                                    "input/output streams, per launch",
-                     "limiter": {"forward": measured_limiter("forward"),
+                     "limiter": {"forward": measured_limiter("forward_one_launch"),
                                  "back": measured_limiter("back")},
                      "pair": {"what": "forward + back of one SIRT step",
                               "alg_bytes": alg_bytes_forward(N, V) + alg_bytes_back(N, V),

@@ -1,8 +1,8 @@
 """Launch-shape autotuner for the distance-driven projector pair.
 
 The forward kernel can run 256, 128 or 64 bins of a view per block and the back kernel
-64x64 tiles (4x4 pixels per thread), 32x32 tiles (2x2) or 32x32 tiles (4x4).  Which is
-fastest depends on the image size, the view count and how many slices share a launch
+64x64 tiles (4x4 pixels per thread), 32x32 tiles (2x2 or 4x4) or 16x16 tiles (one pixel
+per thread); a plan that is not tuned picks the tile per launch.  Which is fastest depends on the image size, the view count and how many slices share a launch
 (a 256^2 single slice has only 16 of the large back tiles -- far too few blocks for 256
 compute units).  Every shape accumulates each output element in the same order, so the
 choice never changes a projection or an iterate.

@@ -126,7 +126,7 @@ int launch_transpose(const float* in, float* out, int npix, int nslices, hipStre
 // The transposed copies of a call's images, in a buffer of the plan, from the constructor to
 // the destructor: get() is null where there is none, because it is not wanted, st is capturing
 // (a replay would share the buffer unseen) or memory is short; the caller then reads the image
-// as it is.  Calls of one plan on several threads or streams take the buffer in turn: the
+// as it is.  Inside a caller-owned scratch region the copy lies there and nothing is allocated.  Calls of one plan on several threads or streams take the buffer in turn: the
 // object holds the plan's lock, the copy waits for the last reader and the destructor marks
 // the new one, so the caller enqueues what reads the copy before the object ends.
 class TransposedCopy {

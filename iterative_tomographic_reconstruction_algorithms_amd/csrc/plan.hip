@@ -304,6 +304,13 @@ TransposedCopy::TransposedCopy(const Plan& p, bool wanted, const float* image, i
     : p_(p), st_(st)
 {
     if (!wanted) return;
+    if (scratch_region_active()) {   // no allocation: the region has room for the copy
+        Scratch s;
+        if (get_scratch(p, nslices, &s, st) == ITOMO_OK &&
+            launch_transpose(image, s.xT, p.npix, nslices, st) == ITOMO_OK)
+            copy_ = s.xT;
+        return;
+    }
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(st, &cs) != hipSuccess) {
         (void)hipGetLastError();
@@ -341,7 +348,7 @@ TransposedCopy::TransposedCopy(const Plan& p, bool wanted, const float* image, i
 
 TransposedCopy::~TransposedCopy()
 {
-    if (copy_ && hipEventRecord(p_.copy_read, st_) != hipSuccess) {
+    if (copy_ && lock_.owns_lock() && hipEventRecord(p_.copy_read, st_) != hipSuccess) {
         (void)hipGetLastError();
         (void)hipStreamSynchronize(st_);  // no mark: nothing may be left to read the copy
     }

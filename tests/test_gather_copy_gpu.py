@@ -93,3 +93,21 @@ def test_copy_under_capture_and_on_two_streams(oper):
             p.forward(other, out=o2)
     torch.cuda.synchronize()
     assert torch.equal(o1, want) and torch.equal(o2, want2)
+
+
+@pytest.mark.parametrize("oper", ["pd", "ss"])
+def test_copy_in_an_iteration_that_allocates_nothing(oper):
+    from iterative_tomographic_reconstruction_algorithms_amd import _lib as L
+    from iterative_tomographic_reconstruction_algorithms_amd.core import stream_handle
+    n, nz = 65, LINE[oper] // (2 * V) + 8
+    p = plan(oper, n)
+    x = torch.rand((nz, n, n), device="cuda")
+    b = torch.rand((nz, V, n), device="cuda")
+    R, C = p.sirt_weights()
+    work = torch.empty_like(b)
+    y = x.clone()
+    p.sirt_iterate(x, b, R, C, work)
+    L.check(L.lib().itomo_sirt_iterate_noalloc(
+        p._h, y.data_ptr(), b.data_ptr(), R.data_ptr(), C.data_ptr(), work.data_ptr(), nz, -1.0,
+        None, stream_handle()), "sirt_iterate_noalloc")
+    assert torch.equal(x, y)
