@@ -5,9 +5,10 @@
 // FFT.  For outputs 0..npix-1 that is the linear convolution with the real, even taps
 // h[k] = (1/L) sum_j H[j] cos(2 pi j k / L) at lags |k| < npix (no wrap-around: L >= 4 npix).
 // The taps are computed once on the host in FP64; the GPU convolves each row with them in
-// FP64, as a circular convolution of length L = 2^k >= 2 npix - 1 by FFT (fft_device.h).  The
-// taps' spectrum is real (they are real and even), so two rows ride in one complex transform,
-// one in the real and one in the imaginary part, and neither reaches the other's result.
+// FP64, as a circular convolution of length L = 2^k >= 2 npix - 1 by FFT (fft_device.h).  A row
+// is real, so it takes a complex transform of M = L / 2 values, its even samples in the real
+// and its odd ones in the imaginary part.  Rows share nothing: a row's bits do not depend on the
+// rows beside it.
 #include <cmath>
 #include <vector>
 
@@ -32,10 +33,10 @@ static double filter_value(int k, int nfreq, int ftype)
     }
 }
 
-constexpr int kFilterMinLog = 6, kFilterMaxLog = 13;   // L up to 8192: 128 KB of LDS
+constexpr int kFilterMinLog = 6, kFilterMaxLog = 13;   // L up to 8192: 64 KB of LDS
 
-// Row r convolved directly, the way the sum is written down: for rows with an infinity or a
-// NaN, whose effect a transform would spread over the whole row (and its partner).
+// A row convolved directly, the way the sum is written down: for rows with an infinity or a
+// NaN, whose effect a transform would spread over the whole row.
 __device__ void conv_row(const float* __restrict__ in, float* __restrict__ out,
                          const double* __restrict__ taps, int npix, int tid, int nt)
 {
@@ -49,20 +50,30 @@ __device__ void conv_row(const float* __restrict__ in, float* __restrict__ out,
     }
 }
 
-// Blocks take pairs of rows in turn; each transforms the taps once.  Bound by LDS: 2 (k/2 + 1)
-// passes of 32 bytes per value and transform.  One output costs about 10 k FP64 operations
-// instead of 2 npix (a direct sum over LDS took 687 us for 3600 rows of 1024, this 74).  The error stays at FP64 rounding of the row's norm: rows whose largest
-// values differ by more than 2^20 (a zero row beside another included) go through on their own.
+// Blocks take rows in turn; each transforms the taps once.  Bound by LDS: 2 (k/2 + 1) passes of
+// 32 bytes per value and transform.  One output costs about 10 k FP64 operations instead of
+// 2 npix (3600 rows of 1024: 59 us; a direct sum over LDS 602).  The error of an output
+// is FP64 rounding of the norm of its own row, below 1e-13 of the sum of the terms' sizes.
+//
+// With Z the transform of the M complex values, E_k = (Z_k + conj Z_M-k) / 2 and
+// O_k = (Z_k - conj Z_M-k) / 2i are those of the even and the odd samples, and the row's own
+// transform is X_k = E_k + w_k O_k, X_k+M = E_k - w_k O_k, w_k = exp(-2 pi i k / L).  Times the
+// taps' spectrum (real, for the taps are real and even; H_k+M = H_M-k) and taken apart again,
+// with s = (H_k + H_M-k) / 2 and d = (H_k - H_M-k) / 2:
+//   E'_k = s E_k + d w_k O_k,   O'_k = s O_k + d conj(w_k) E_k.
+// The taps' own E and O give s = Re E_k and d = Re(w_k O_k).
 template <int LOGL>
-__global__ void __launch_bounds__((fft_threads<LOGL>()))
+__global__ void __launch_bounds__((fft_threads<LOGL - 1>()))
 filter_rows_kernel(const float* __restrict__ in, float* __restrict__ out,
                    const double* __restrict__ taps, int nrows, int npix)
 {
-    constexpr int L = 1 << LOGL, T = fft_threads<LOGL>(), E = (L + T - 1) / T;
-    constexpr int NA = L / 64 > 0 ? L / 64 : 1;
-    __shared__ double2 buf[L];
-    __shared__ double2 sA[NA], sB[64];      // exp(-2 pi i 64 a / L), exp(-2 pi i b / L)
-    __shared__ float sMax[2][T / 64];
+    constexpr int L = 1 << LOGL, M = L / 2, T = fft_threads<LOGL - 1>();
+    constexpr int E = (L + T - 1) / T;          // samples per thread
+    constexpr int P = M / 2 / T + 1;            // pairs (k, M - k), k = 0 .. M / 2, per thread
+    constexpr int NA = L / 64;
+    __shared__ double2 buf[M];
+    __shared__ double2 sA[NA], sB[64];          // exp(-2 pi i 64 a / L), exp(-2 pi i b / L)
+    double* const re = (double*)buf;            // re[n]: sample n
     const int tid = threadIdx.x;
     for (int q = tid; q < NA + 64; q += T) {
         const int k = q < NA ? 64 * q : q - NA;
@@ -70,84 +81,82 @@ filter_rows_kernel(const float* __restrict__ in, float* __restrict__ out,
         sincospi(-2.0 * k / L, &w.y, &w.x);
         if (q < NA) sA[q] = w; else sB[q - NA] = w;
     }
-    auto tw = [&](int q) { return c_mul(sA[q >> 6], sB[q & 63]); };
-    // the spectrum of the even extension of the taps, 1/L folded in
+    auto twl = [&](int q) { return c_mul(sA[q >> 6], sB[q & 63]); };
+    auto tw = [&](int q) { return twl(2 * q); };
+    // E_k and O_k of the transform in buf
+    auto split = [&](int k, double2& ek, double2& ok) {
+        const double2 a = buf[k], b = buf[(M - k) & (M - 1)];
+        ek = make_double2(0.5 * (a.x + b.x), 0.5 * (a.y - b.y));
+        ok = make_double2(0.5 * (a.y + b.y), 0.5 * (b.x - a.x));
+    };
+    // the spectrum of the even extension of the taps, 1/M folded in
 #pragma unroll
     for (int e = 0; e < E; ++e) {
         const int i = tid + e * T, lag = min(i, L - i);
-        if (i < L) buf[i] = make_double2(lag < npix ? taps[lag] : 0.0, 0.0);
+        if (i < L) re[i] = lag < npix ? taps[lag] : 0.0;
     }
     __syncthreads();
-    fft_lds<LOGL, T>(buf, tid, 1, tw);
-    double H[E];
+    fft_lds<LOGL - 1, T>(buf, tid, 1, tw);
+    double hs[P], hd[P];
 #pragma unroll
-    for (int e = 0; e < E; ++e) {
-        const int i = tid + e * T;
-        H[e] = i < L ? buf[i].x * (1.0 / L) : 0.0;
+    for (int e = 0; e < P; ++e) {
+        const int k = tid + e * T;
+        hs[e] = hd[e] = 0.0;
+        if (k <= M / 2) {
+            double2 ek, ok;
+            split(k, ek, ok);
+            hs[e] = ek.x * (1.0 / M);
+            hd[e] = c_mul(twl(k), ok).x * (1.0 / M);
+        }
     }
-    const int pairs = (nrows + 1) / 2;
-    for (int p = blockIdx.x; p < pairs; p += gridDim.x) {
-        const float* r0 = in + (int64_t)(2 * p) * npix;
-        const bool two = 2 * p + 1 < nrows;
-        float x[E], y[E], mx = 0.0f, my = 0.0f;
+    for (int row = blockIdx.x; row < nrows; row += gridDim.x) {
+        const float* r = in + (int64_t)row * npix;
+        float* o = out + (int64_t)row * npix;
+        float x[E];
         bool finite = true;
 #pragma unroll
         for (int e = 0; e < E; ++e) {
             const int i = tid + e * T;
-            x[e] = i < npix ? r0[i] : 0.0f;
-            y[e] = two && i < npix ? r0[npix + i] : 0.0f;
-            mx = fmaxf(mx, fabsf(x[e]));
-            my = fmaxf(my, fabsf(y[e]));
-            finite = finite && isfinite(x[e]) && isfinite(y[e]);
+            x[e] = i < npix ? r[i] : 0.0f;
+            finite = finite && isfinite(x[e]);
         }
-        if (!finite) mx = INFINITY;
-        for (int off = 32; off > 0; off >>= 1) {
-            mx = fmaxf(mx, __shfl_xor(mx, off, 64));
-            my = fmaxf(my, __shfl_xor(my, off, 64));
-        }
-        __syncthreads();   // the last pair's (or the taps') buffer is consumed
-        if ((tid & 63) == 0) {
-            sMax[0][tid >> 6] = mx;
-            sMax[1][tid >> 6] = my;
-        }
-        __syncthreads();
-        for (int w = 0; w < T / 64; ++w) {
-            mx = fmaxf(mx, sMax[0][w]);
-            my = fmaxf(my, sMax[1][w]);
-        }
-        float* o0 = out + (int64_t)(2 * p) * npix;
-        if (mx == INFINITY) {
-            conv_row(r0, o0, taps, npix, tid, T);
-            if (two) conv_row(r0 + npix, o0 + npix, taps, npix, tid, T);
+        // also: the last row's (or the taps') buffer is consumed
+        if (__syncthreads_or(!finite)) {
+            conv_row(r, o, taps, npix, tid, T);
             continue;
         }
-        const bool apart = fmaxf(mx, my) * 9.5367431640625e-7f > fminf(mx, my);   // 2^-20
-        for (int part = 0; part < (apart && two ? 2 : 1); ++part) {
-            if (part) __syncthreads();
 #pragma unroll
-            for (int e = 0; e < E; ++e) {
-                const int i = tid + e * T;
-                const float re = part ? 0.0f : x[e], im = part || !apart ? y[e] : 0.0f;
-                if (i < L) buf[i] = make_double2(re, im);
-            }
-            __syncthreads();
-            fft_lds<LOGL, T>(buf, tid, 1, tw);
-            // the inverse transform is the forward one with the parts exchanged
+        for (int e = 0; e < E; ++e) {
+            const int i = tid + e * T;
+            if (i < L) re[i] = x[e];
+        }
+        __syncthreads();
+        fft_lds<LOGL - 1, T>(buf, tid, 1, tw);
+        // the inverse transform is the forward one with the parts exchanged; a pair (k, M - k)
+        // is read and written by one thread
 #pragma unroll
-            for (int e = 0; e < E; ++e) {
-                const int i = tid + e * T;
-                if (i < L) buf[i] = make_double2(buf[i].y * H[e], buf[i].x * H[e]);
+        for (int e = 0; e < P; ++e) {
+            const int k = tid + e * T;
+            if (k <= M / 2) {
+                double2 ek, ok, w = twl(k);
+                split(k, ek, ok);
+                const double2 wo = c_mul(w, ok);
+                w.y = -w.y;
+                const double2 we = c_mul(w, ek);
+                const double2 en = make_double2(hs[e] * ek.x + hd[e] * wo.x,
+                                                hs[e] * ek.y + hd[e] * wo.y);
+                const double2 on = make_double2(hs[e] * ok.x + hd[e] * we.x,
+                                                hs[e] * ok.y + hd[e] * we.y);
+                buf[(M - k) & (M - 1)] = make_double2(on.x - en.y, en.x + on.y);
+                buf[k] = make_double2(en.y + on.x, en.x - on.y);
             }
-            __syncthreads();
-            fft_lds<LOGL, T>(buf, tid, 1, tw);
+        }
+        __syncthreads();
+        fft_lds<LOGL - 1, T>(buf, tid, 1, tw);
 #pragma unroll
-            for (int e = 0; e < E; ++e) {
-                const int i = tid + e * T;
-                if (i < npix) {
-                    if (!part) o0[i] = (float)buf[i].y;
-                    if (two && (part || !apart)) o0[npix + i] = (float)buf[i].x;
-                }
-            }
+        for (int e = 0; e < E; ++e) {
+            const int i = tid + e * T;
+            if (i < npix) o[i] = (float)re[i ^ 1];
         }
     }
 }
@@ -159,11 +168,11 @@ static void launch_filter(const float* in, float* out, int nrows, int npix, cons
     if constexpr (LOGL <= kFilterMaxLog) {
         if (LOGL == kFilterMaxLog || (1 << LOGL) >= 2 * npix - 1) {
             // as many blocks as the LDS of 256 compute units holds, at least one per unit
-            constexpr int lds = (16 << LOGL) + 16 * ((1 << LOGL) / 64 + 64) + 128;
-            constexpr int T = fft_threads<LOGL>();
+            constexpr int lds = (8 << LOGL) + 16 * ((1 << LOGL) / 64 + 64);
+            constexpr int T = fft_threads<LOGL - 1>();
             constexpr int fit = 163840 / lds < 2048 / T ? 163840 / lds : 2048 / T;
-            const int pairs = (nrows + 1) / 2, most = 256 * fit;
-            filter_rows_kernel<LOGL><<<pairs < most ? pairs : most, T, 0, st>>>(in, out, taps,
+            const int most = 256 * fit;
+            filter_rows_kernel<LOGL><<<nrows < most ? nrows : most, T, 0, st>>>(in, out, taps,
                                                                              nrows, npix);
         } else {
             launch_filter<LOGL + 1>(in, out, nrows, npix, taps, st);

@@ -42,15 +42,30 @@ def test_filter_many_rows():
     check(rng.standard_normal((4099, 100)).astype(np.float32))   # blocks take several pairs
 
 
-@pytest.mark.parametrize("scale", [0.0, 1e-30, 1e-9, 1e9, 1e30])
-def test_filter_rows_do_not_reach_each_other(scale):
+@pytest.mark.parametrize("npix", [300, 1024, 4096])
+@pytest.mark.parametrize("scale", [0.0, 1e-30, 1e-9, 1.2e-6, 1e-5, 1e-3, 1e-1, 10.0, 1e3, 1e5, 8e5, 1e9,
+                                   1e30])
+def test_filter_rows_do_not_reach_each_other(scale, npix):
     rng = np.random.default_rng(5)
-    rows = rng.standard_normal((6, 300)).astype(np.float32)
+    rows = rng.standard_normal((6, npix)).astype(np.float32)
     rows[1] *= np.float32(scale)
     rows[2] *= np.float32(scale)
     got = check(rows)
     if scale == 0.0:
         assert (got[1:3] == 0).all()
+
+
+@pytest.mark.parametrize("npix", [17, 64, 300, 1000])
+def test_filter_row_is_the_same_alone_and_in_any_stack(npix):
+    rng = np.random.default_rng(npix)
+    rows = rng.standard_normal((3, 17, npix)).astype(np.float32)   # an odd number of views
+    rows *= np.float32(10.0) ** rng.integers(-6, 7, (3, 17, 1)).astype(np.float32)
+    sino = torch.from_numpy(rows).cuda()
+    stack = filter_sino(sino)
+    for z in range(3):
+        assert torch.equal(stack[z], filter_sino(sino[z].contiguous()))
+        for v in (0, 1, 8, 16):
+            assert torch.equal(stack[z, v], filter_sino(sino[z, v].contiguous()))
 
 
 @pytest.mark.parametrize("bad", [np.inf, -np.inf, np.nan])
