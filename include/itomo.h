@@ -388,7 +388,8 @@ int itomo_admm_l1_update(const float *x, float *u, float *alpha, int npix, int n
  *   reference's zero-padded FFT filter; ftype 0 ramp, 1 shepp-logan, 2 cosine,
  *   3 hamming, 4 hanning, 5 none.  npix <= 4096.
  * itomo_filter_rows: out[r][n] = sum_m in[r][m] * taps[|n-m|] (DEVICE arrays, FP64
- *   accumulation) -- identical to the reference's FFT filtering for n < npix.
+ *   accumulation) -- identical to the reference's FFT filtering for n < npix.  A row's result
+ *   depends on that row alone; out may be in itself, but may not overlap it otherwise.
  * ------------------------------------------------------------------------------- */
 int itomo_filter_taps(int npix, int ftype, double *taps_host);
 int itomo_filter_rows(const float *in, float *out, int nrows, int npix, const double *taps,

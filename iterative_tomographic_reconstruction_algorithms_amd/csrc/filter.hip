@@ -35,10 +35,11 @@ static double filter_value(int k, int nfreq, int ftype)
 
 constexpr int kFilterMinLog = 6, kFilterMaxLog = 13;   // L up to 8192: 64 KB of LDS
 
-// A row convolved directly, the way the sum is written down: for rows with an infinity or a
-// NaN, whose effect a transform would spread over the whole row.
-__device__ void conv_row(const float* __restrict__ in, float* __restrict__ out,
-                         const double* __restrict__ taps, int npix, int tid, int nt)
+// A row (in LDS: out may be where it came from) convolved directly, the way the sum is written
+// down: for rows with an infinity or a NaN, whose effect a transform would spread over the whole
+// row.
+__device__ void conv_row(const float* in, float* out, const double* __restrict__ taps, int npix,
+                         int tid, int nt)
 {
     for (int n = tid; n < npix; n += nt) {
         double acc = 0.0;
@@ -50,7 +51,8 @@ __device__ void conv_row(const float* __restrict__ in, float* __restrict__ out,
     }
 }
 
-// Blocks take rows in turn; each transforms the taps once.  Bound by LDS: 2 (k/2 + 1) passes of
+// Blocks take rows in turn; each transforms the taps once.  A row is read whole before any of it
+// is written, so in and out may be the same array.  Bound by LDS: 2 (k/2 + 1) passes of
 // 32 bytes per value and transform.  One output costs about 10 k FP64 operations instead of
 // 2 npix (3600 rows of 1024: 59 us; a direct sum over LDS 602).  The error of an output
 // is FP64 rounding of the norm of its own row, below 1e-13 of the sum of the terms' sizes.
@@ -64,8 +66,8 @@ __device__ void conv_row(const float* __restrict__ in, float* __restrict__ out,
 // The taps' own E and O give s = Re E_k and d = Re(w_k O_k).
 template <int LOGL>
 __global__ void __launch_bounds__((fft_threads<LOGL - 1>()))
-filter_rows_kernel(const float* __restrict__ in, float* __restrict__ out,
-                   const double* __restrict__ taps, int nrows, int npix)
+filter_rows_kernel(const float* in, float* out, const double* __restrict__ taps, int nrows,
+                   int npix)
 {
     constexpr int L = 1 << LOGL, M = L / 2, T = fft_threads<LOGL - 1>();
     constexpr int E = (L + T - 1) / T;          // samples per thread
@@ -122,7 +124,14 @@ filter_rows_kernel(const float* __restrict__ in, float* __restrict__ out,
         }
         // also: the last row's (or the taps') buffer is consumed
         if (__syncthreads_or(!finite)) {
-            conv_row(r, o, taps, npix, tid, T);
+            float* const row_in = (float*)buf;
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                const int i = tid + e * T;
+                if (i < npix) row_in[i] = x[e];
+            }
+            __syncthreads();
+            conv_row(row_in, o, taps, npix, tid, T);
             continue;
         }
 #pragma unroll
