@@ -627,15 +627,17 @@ __device__ __forceinline__ float fwd_ones(const DdView& g, const float* __restri
 // diagonals: in step k lane d takes line L(d) + k, where L(d) is its own first line.  Every
 // step then serves all lanes (a block that walks the union of its bins' lines, as the
 // staged path does, spends npix/w + 64 line steps where npix/w are needed; staged, the wide
-// views alone took 94 us at 64^2 x 45 where the whole forward now takes 16), and the lanes' first pixels on their lines agree to within a line's shift.
+// views alone took 94 us at 64^2 x 45 where the whole forward now takes 18), and the lanes'
+// first pixels on their lines agree to within a line's shift.
 // Hence candidate j of the wave lies in 64 neighbouring lines at nearly the same place
 // along the line: `img` is the orientation in which neighbouring lines are neighbours in
 // memory (the transpose of what the staged path reads), and candidate j of the whole wave
 // is one nearly contiguous load.  No LDS, no barriers; bounds: vector L1 accesses (one
 // 4-byte load per candidate and lane) and the five VALU operations of a candidate.
 //
-// Lines outside the image (a lane's diagonal before its first or after its last line) load
-// nothing and get the right end -1e30, which makes every weight 0.  Away from the end of
+// Lines outside the image or past the lane's own last line load nothing and get the right end
+// -1e30, which makes every weight 0: only pixels on a bin's own lines and among its
+// candidates are multiplied at all (a weight of 0 makes a NaN of an infinity).  Away from the end of
 // the line (q + NC < npix for every lane) the candidates need no bounds check and L* does
 // not clip (see dd_fwd_block); the last bin of a view always takes the checked form.
 template <int ARITH, int NC, int GL>
@@ -662,6 +664,7 @@ __device__ __forceinline__ float fwd_diag(const DdView& g, const float* __restri
     const int La = __builtin_amdgcn_readlane(L, 0), Lb = __builtin_amdgcn_readlane(L, 63);
     const int k0 = max(0, -max(La, Lb));
     const int k1 = min(steps - 1, npix - 1 - min(La, Lb));
+    const unsigned end = max(0, min(npix, L + steps));   // past the lane's last line
     const int stride = npix * 4;
     if constexpr (NC > 0) {
         for (int k = k0; k <= k1; k += GL) {
@@ -672,7 +675,7 @@ __device__ __forceinline__ float fwd_diag(const DdView& g, const float* __restri
 #pragma unroll
             for (int l = 0; l < GL; ++l) {
                 const int i = L + k + l;
-                ok[l] = (unsigned)i < (unsigned)npix;
+                ok[l] = (unsigned)i < end;
                 K[l] = key_K<ARITH>(g, line_coord(i, nh));
                 xq[l] = first_pixel_near(Dlo, Dlh, K[l], nh, npix);
                 q[l] = (int)xq[l] + nh;
@@ -710,7 +713,7 @@ __device__ __forceinline__ float fwd_diag(const DdView& g, const float* __restri
         constexpr int CH = 16;   // candidates loaded together
         for (int k = k0; k <= k1; ++k) {
             const int i = L + k;
-            const bool ok = (unsigned)i < (unsigned)npix;
+            const bool ok = (unsigned)i < end;
             const float K = key_K<ARITH>(g, line_coord(i, nh));
             const float x = first_pixel(Dlo, K, nh, npix);
             const int q = (int)x + nh;
@@ -721,16 +724,17 @@ __device__ __forceinline__ float fwd_diag(const DdView& g, const float* __restri
             float xk = x, Rp = __fsub_rn(x, K);
             for (int j0 = 0; j0 < g.ncand; j0 += CH) {
                 float v[CH];
-                if (!__any(ok && q + j0 + CH > npix)) {
+                if (j0 + CH <= g.ncand && !__any(ok && q + j0 + CH > npix)) {
 #pragma unroll
                     for (int j = 0; j < CH; ++j)
                         v[j] = __int_as_float((int)__builtin_amdgcn_raw_buffer_load_b32(
                             rs, vo, (j0 + j) * stride, 0));
                 } else {
+                    const int last = min(npix - q, g.ncand) - j0;
 #pragma unroll
                     for (int j = 0; j < CH; ++j)
                         v[j] = __int_as_float((int)__builtin_amdgcn_raw_buffer_load_b32(
-                            rs, ok && q + j0 + j < npix ? vo + (j0 + j) * stride : -1, 0, 0));
+                            rs, ok && j < last ? vo + (j0 + j) * stride : -1, 0, 0));
                 }
 #pragma unroll
                 for (int j = 0; j < CH; ++j)
@@ -770,8 +774,8 @@ constexpr int fwd_window_extra()
 // that each first candidate, clamped into the line, lies in the window, whatever the bin.
 // Lines run over the union of the block's per-bin line ranges; lines that
 // miss a bin add nothing to it.  A chunk always runs all its FL lines (straight-line code, so
-// the LDS reads of one line hide behind the sums of another): those past the image get the
-// line end kNoLine, which makes every weight 0.  Every thread of the block takes part
+// the LDS reads of one line hide behind the sums of another): those past the block's last line
+// are zeros with the line end kNoLine, which makes every weight 0.  Every thread of the block takes part
 // (inactive threads, past the last bin, compute a copy of the last bin and store nothing).
 // sImg holds FLOATS floats, sMeta kFwdStageMaxLines entries {byte offset of pixel 0, L*}.
 constexpr float kNoLine = -1e30f;
@@ -826,7 +830,7 @@ __device__ __forceinline__ float fwd_staged(const DdView& g, const float* __rest
             const int i = c0 + l;
             const int q = start(i) + 4 * j4;
             const int idx = i * npix + q;
-            const bool ok = (N4 % B == 0 || k < N4) && i < npix && q >= 0;
+            const bool ok = (N4 % B == 0 || k < N4) && i <= i_hi && q >= 0;
             if (!ragged || !ok || idx + 3 < total) {
                 v[r] = load_px4(rs, ok ? idx : 0x3fffffff);
             } else {
@@ -839,7 +843,7 @@ __device__ __forceinline__ float fwd_staged(const DdView& g, const float* __rest
         const int i = c0 + tid;
         if (tid < FL) {
             meta.x = __int_as_float(4 * (nh - start(i) + tid * W));
-            meta.y = i < npix ? ls[i] : kNoLine;
+            meta.y = i <= i_hi ? ls[i] : kNoLine;
         }
     };
     auto store = [&]() {

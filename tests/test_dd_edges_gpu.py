@@ -72,3 +72,43 @@ def test_large_launches_match_oracle(n, nz):
         for z in (0, nz // 2, nz - 1):
             np.testing.assert_array_equal(
                 got[z], O.dd_forward(x[z], np.fft.ifftshift(ANGLES), O.FAST))
+
+
+def lines_met(n, theta, s, c):
+    """Of one sweep view, per bin: the block's line range (64 bins, three lines of margin) and
+    the bin's first pixel on every line, in float64."""
+    nh = n // 2
+    w, t = (1 / s, c / s) if theta > np.pi / 2 else (1 / c, s / c)
+    d = np.arange(n)
+    lo, hi = d // 64 * 64, np.minimum(d // 64 * 64 + 64, n)
+    e0, e1 = (-nh - (hi - nh) * w) / t + nh - 0.5, (n - nh - (lo - nh) * w) / t + nh - 0.5
+    first = (d[:, None] - nh) * w + (np.arange(n)[None, :] - nh + 0.5) * t + nh
+    return np.minimum(e0, e1) - 3.01, np.maximum(e0, e1) + 3.01, first, w
+
+
+@pytest.mark.parametrize("n,nz", [(130, 16), (130, 120), (65, 190)])
+def test_infinite_pixel_reaches_only_bins_about_its_line(n, nz):
+    """A bin that no line range or candidate run takes to the pixel stays finite (weights of
+    zero do reach the rest: the reference's own build assumes finite data)."""
+    rng = np.random.default_rng(nz)
+    r, c = rng.integers(0, n, nz), rng.integers(0, n, nz)
+    x = np.ones((nz, n, n), np.float32)
+    x[np.arange(nz), r, c] = np.inf
+    p = Plan("dd", n, ANGLES)
+    sin, cos = (a.astype(np.float64) for a in p.trig())
+    got = np.isfinite(p.forward(torch.from_numpy(x).cuda()).cpu().numpy())
+    for v, theta in enumerate(ANGLES):
+        if abs(sin[v]) < 1e-4 or abs(cos[v]) < 1e-4:
+            continue
+        a, b, first, w = lines_met(n, theta, sin[v], cos[v])
+        cand = (int(np.floor(w + 0.25)) + 2 + 3) // 4 * 4 if w > 30.75 else n
+        for z in range(nz):
+            line, q = (r[z], c[z]) if theta > np.pi / 2 else (c[z], r[z])
+            start = np.clip(first[:, line], 0, n - 1)
+            # the first pixels of a line are also read as the run past the end of the line before
+            away = (line < a) | (line > b + (q < 6)) | (q > start + cand + 1.01)
+            bad = away & ~got[z, ANGLES.size - 1 - v]
+            assert not bad.any(), (DEG[v], z, line, q, np.flatnonzero(bad))
+            overlap = np.minimum(q + 1, first[:, line] + w) - np.maximum(q, first[:, line])
+            assert not (got[z, ANGLES.size - 1 - v] & (overlap > 0.01) & (np.arange(n) < n - 1)
+                        & (q < n - 1)).any()
