@@ -98,6 +98,13 @@ int itomo_radon_ss(float *image, int npix, const float *angles, int nang, int op
  * Distance-driven plans reject (ITOMO_EANGLE) views that sweep rows with sin <= 0 or
  * columns with cos <= 0: for those the reference's sweep indexes bin -1 (undefined
  * behaviour in radon_dd.c:158-188).  Angles in [0, pi) are always accepted.
+ * Pixel-driven and slant-stacking plans keep a transposed copy of the images of a large
+ * forward call (from 8192 and 2048 waves of 64 bins), at most 256 MiB or one slice and, while
+ * calls grow, the smaller copies before it; a call with more slices takes them in turns.  It is
+ * allocated on first use, which neither waits for the GPU nor disturbs another thread's stream
+ * capture.  While `stream` itself is captured, or without memory for it, the call reads the
+ * images as they are: the same bits, up to twice the time (1024^2 x 720 slant-stacking 2.2 ms for
+ * 1.1).  Inside itomo_sirt_iterate_noalloc and captured iterations it lies in their scratch.
  * Replaces class_projectors_radon.projectors.__init__ (class_projectors_radon.py:47-55).
  * ------------------------------------------------------------------------------- */
 int itomo_plan_create(itomo_plan **plan, int projector, int npix, const float *angles,

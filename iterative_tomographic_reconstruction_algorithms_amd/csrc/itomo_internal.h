@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 #include <cstdint>
 #include <mutex>
+#include <vector>
 
 #include "itomo.h"
 
@@ -108,9 +109,10 @@ struct Plan {
     mutable unsigned* rdb_ent;
     mutable int64_t* rdb_off;
     mutable size_t rd_mat_bytes;
-    // Pixel-driven and slant-stacking plans: the buffer of TransposedCopy, grown on first use.
+    // Pixel-driven and slant-stacking plans: the buffer of TransposedCopy (the last one, of
+    // copy_bytes; the others are outgrown), grown on first use.
     mutable std::mutex copy_mutex;
-    mutable float* copy;
+    mutable std::vector<float*> copies;
     mutable size_t copy_bytes;
     mutable hipEvent_t copy_read;  // recorded behind the last launch that reads the copy
 };
@@ -123,11 +125,25 @@ int rd_matrix_ensure(const Plan& p, hipStream_t st);
 void rd_matrix_free(const Plan& p);
 // out = the transposes of nslices npix x npix images (npix^2 apart); stream-ordered.
 int launch_transpose(const float* in, float* out, int npix, int nslices, hipStream_t st);
-// The transposed copies of a call's images, in a buffer of the plan, from the constructor to
-// the destructor: get() is null where there is none, because it is not wanted, st is capturing
-// (a replay would share the buffer unseen) or memory is short; the caller then reads the image
-// as it is.  Inside a caller-owned scratch region the copy lies there and nothing is allocated.  Calls of one plan on several threads or streams take the buffer in turn: the
-// object holds the plan's lock, the copy waits for the last reader and the destructor marks
+// Waves of 64 bins of a pixel-driven or slant-stacking forward call, and the number from which it
+// reads a transposed copy.  PD, us with and without: 511^2 x 360 views (2880 waves) 597 and 593;
+// 512^2 x 361 x 2 slices (5776) 991 and 989; 1024^2 x 720 (11520) 3552 and 3902.  SS: 257^2 x 180
+// (900) 102 and 85; 511^2 x 360 230 and 255; 512^2 x 361 x 2 306 and 569; 1024^2 x 720 1125 and 2196.
+inline int64_t copy_waves(const Plan& p, int nslices)
+{
+    return (int64_t)((p.npix + 63) / 64) * p.nang * nslices;
+}
+inline int64_t copy_line(const Plan& p) { return p.projector == ITOMO_PROJ_PD ? 8192 : 2048; }
+// The most a plan keeps for the copy (one slice if that is more): a larger call takes its slices
+// in turns.
+constexpr int64_t kCopyBytes = (int64_t)256 << 20;
+// The transposed copies of the first slices() of a call's images, in a buffer of the plan, from
+// the constructor to the destructor.  get() is null, and slices() all of them, where there is none:
+// it is not wanted (unit pixels), the call is below the line, st is capturing (a replay would
+// share the buffer unseen) or memory is short; the caller then reads the images as they are.
+// Inside a caller-owned scratch region the copy lies there and nothing is allocated.  The host never
+// waits for the GPU.  Calls of one plan on several threads or streams take the buffer in turn:
+// the object holds the plan's lock, the copy waits for the last reader and the destructor marks
 // the new one, so the caller enqueues what reads the copy before the object ends.
 class TransposedCopy {
 public:
@@ -136,11 +152,13 @@ public:
     TransposedCopy(const TransposedCopy&) = delete;
     TransposedCopy& operator=(const TransposedCopy&) = delete;
     const float* get() const { return copy_; }
+    int slices() const { return slices_; }
 
 private:
     const Plan& p_;
     hipStream_t st_;
     const float* copy_ = nullptr;
+    int slices_;
     std::unique_lock<std::mutex> lock_;
 };
 // Marks the matrix as held by a graph when st is capturing.

@@ -386,14 +386,6 @@ int dispatch_pd_back(const Plan& p, int epi, int ones, const float* sino, float*
 
 }  // namespace
 
-// Whether a forward call reads a transposed copy for its flat views: from about 8192 waves (us
-// with and without: 511^2 x 360, 2880 waves, 597 and 593; 512^2 x 361 x 2 slices, 5776, 991 and
-// 989; 1024^2 x 720, 11520, 3552 and 3902).
-static bool pd_transposes(const Plan& p, int nslices)
-{
-    return (int64_t)((p.npix + 63) / 64) * p.nang * nslices >= 8192;
-}
-
 int pd_forward_epi(const Plan& p, int epi, int ones, const float* image, float* out,
                    int nslices, int accumulate, const EpiArgs& e, hipStream_t st,
                    int* blocks_per_slice)
@@ -407,18 +399,24 @@ int pd_forward_epi(const Plan& p, int epi, int ones, const float* image, float* 
                                         blocks_per_slice);
     }
     if (blocks_per_slice) *blocks_per_slice = 0;
-    const TransposedCopy tc(p, !ones && pd_transposes(p, nslices), image, nslices, st);
-    const float* imageT = tc.get();
-    int rc;
-    if (p.arith == ITOMO_ARITH_FAST)
-        rc = p.method == 0
-                 ? dispatch_pd_fwd<ITOMO_ARITH_FAST, 0>(p, epi, ones, image, imageT, out, nslices, accumulate, e, st)
-                 : dispatch_pd_fwd<ITOMO_ARITH_FAST, 1>(p, epi, ones, image, imageT, out, nslices, accumulate, e, st);
-    else
-        rc = p.method == 0
-                 ? dispatch_pd_fwd<ITOMO_ARITH_IEEE, 0>(p, epi, ones, image, imageT, out, nslices, accumulate, e, st)
-                 : dispatch_pd_fwd<ITOMO_ARITH_IEEE, 1>(p, epi, ones, image, imageT, out, nslices, accumulate, e, st);
-    if (rc) return rc;
+    for (int z = 0; z < nslices;) {
+        const float* im = image ? image + (int64_t)z * p.npix * p.npix : nullptr;
+        float* o = out + (int64_t)z * p.nang * p.npix;
+        const TransposedCopy tc(p, !ones, im, nslices - z, st);
+        const float* imT = tc.get();
+        const int n = tc.slices();
+        int rc;
+        if (p.arith == ITOMO_ARITH_FAST)
+            rc = p.method == 0
+                     ? dispatch_pd_fwd<ITOMO_ARITH_FAST, 0>(p, epi, ones, im, imT, o, n, accumulate, e, st)
+                     : dispatch_pd_fwd<ITOMO_ARITH_FAST, 1>(p, epi, ones, im, imT, o, n, accumulate, e, st);
+        else
+            rc = p.method == 0
+                     ? dispatch_pd_fwd<ITOMO_ARITH_IEEE, 0>(p, epi, ones, im, imT, o, n, accumulate, e, st)
+                     : dispatch_pd_fwd<ITOMO_ARITH_IEEE, 1>(p, epi, ones, im, imT, o, n, accumulate, e, st);
+        if (rc) return rc;
+        z += n;
+    }
     return check_hip(hipGetLastError(), "pd forward launch");
 }
 

@@ -4,6 +4,7 @@
 // reference C as its own build compiles it (gcc -O3 -ffast-math: sincosf for the
 // trigonometry, reciprocals hoisted out of the loops), or as written (IEEE), so the
 // device kernels only multiply, subtract and fuse -- never divide -- in FAST mode.
+#include <algorithm>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -299,12 +300,40 @@ int get_scratch(const Plan& p, int nslices, Scratch* s, hipStream_t st)
     return ITOMO_OK;
 }
 
+// Room for `bytes` in p.copies.back(), the caller holding p.copy_mutex; false without memory.  The
+// host does not wait: a smaller buffer, which queued launches may still read, stays until the
+// plan goes (at most as much again, for the size doubles).  Another thread's global-mode
+// capture allows an allocation only in the relaxed mode; this one is no part of any capture.
+static bool copy_buffer(const Plan& p, size_t bytes)
+{
+    if (bytes <= p.copy_bytes && p.copy_read) return true;
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) return false;
+    bool ok = p.copy_read ||
+              hipEventCreateWithFlags(&p.copy_read, hipEventDisableTiming) == hipSuccess;
+    const size_t most = std::max(bytes, (size_t)kCopyBytes);
+    const size_t want = std::max(bytes, std::min(2 * p.copy_bytes, most));
+    float* buf = nullptr;
+    ok = ok && hipMalloc(&buf, want) == hipSuccess;
+    if (ok) {
+        try {
+            p.copies.push_back(buf);
+            p.copy_bytes = want;
+        } catch (const std::bad_alloc&) {
+            (void)hipFree(buf);
+            ok = false;
+        }
+    }
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    return ok;
+}
+
 TransposedCopy::TransposedCopy(const Plan& p, bool wanted, const float* image, int nslices,
                                hipStream_t st)
-    : p_(p), st_(st)
+    : p_(p), st_(st), slices_(nslices)
 {
-    if (!wanted) return;
-    if (scratch_region_active()) {   // no allocation: the region has room for the copy
+    if (!wanted || copy_waves(p, nslices) < copy_line(p)) return;
+    if (scratch_region_active()) {   // no buffer of the plan's: the region has room for the copy
         Scratch s;
         if (get_scratch(p, nslices, &s, st) == ITOMO_OK &&
             launch_transpose(image, s.xT, p.npix, nslices, st) == ITOMO_OK)
@@ -317,33 +346,21 @@ TransposedCopy::TransposedCopy(const Plan& p, bool wanted, const float* image, i
         return;
     }
     if (cs != hipStreamCaptureStatusNone) return;
+    const int64_t slice = (int64_t)sizeof(float) * p.npix * p.npix;
+    const int most = (int)std::max<int64_t>(1, std::min<int64_t>(nslices, kCopyBytes / slice));
+    // turns of equal size, so that the last one is no small remainder
+    const int turns = (nslices + most - 1) / most;
+    const int n = (nslices + turns - 1) / turns;
+    if (copy_waves(p, n) < copy_line(p)) return;
     lock_ = std::unique_lock<std::mutex>(p.copy_mutex);
-    if (!p.copy_read &&
-        hipEventCreateWithFlags(&p.copy_read, hipEventDisableTiming) != hipSuccess) {
+    if (!copy_buffer(p, n * (size_t)slice) || hipStreamWaitEvent(st, p.copy_read, 0) != hipSuccess ||
+        launch_transpose(image, p.copies.back(), p.npix, n, st) != ITOMO_OK) {
         (void)hipGetLastError();
-        p.copy_read = nullptr;
+        lock_.unlock();
         return;
     }
-    const size_t bytes = sizeof(float) * (size_t)p.npix * p.npix * nslices;
-    if (bytes > p.copy_bytes) {
-        if (p.copy) {
-            (void)hipEventSynchronize(p.copy_read);  // queued launches may still read it
-            (void)hipFree(p.copy);
-        }
-        p.copy_bytes = 0;
-        if (hipMalloc(&p.copy, bytes) != hipSuccess) {
-            (void)hipGetLastError();
-            p.copy = nullptr;
-            return;
-        }
-        p.copy_bytes = bytes;
-    }
-    if (hipStreamWaitEvent(st, p.copy_read, 0) != hipSuccess ||
-        launch_transpose(image, p.copy, p.npix, nslices, st) != ITOMO_OK) {
-        (void)hipGetLastError();
-        return;
-    }
-    copy_ = p.copy;
+    copy_ = p.copies.back();
+    slices_ = n;
 }
 
 TransposedCopy::~TransposedCopy()
@@ -501,8 +518,8 @@ int itomo_plan_destroy(itomo_plan* p)
         int st2 = check_hip(hipFree(p->scratch), "plan_destroy: hipFree scratch");
         if (!st) st = st2;
     }
-    if (p->copy) {
-        int st2 = check_hip(hipFree(p->copy), "plan_destroy: hipFree copy");
+    for (float* c : p->copies) {
+        int st2 = check_hip(hipFree(c), "plan_destroy: hipFree copy");
         if (!st) st = st2;
     }
     if (p->copy_read) {

@@ -305,14 +305,6 @@ int dispatch_ss_back(const Plan& p, int epi, int ones, const float* sino, float*
 
 }  // namespace
 
-// Whether a forward call reads a transposed copy: once its waves fill the GPU, contiguous loads
-// are worth the copy (us with and without: 257^2 x 180 102 and 85, 511^2 x 360 230 and 255,
-// 512^2 x 361 x 2 slices 306 and 569, 1024^2 x 720 1125 and 2196).
-static bool ss_transposes(const Plan& p, int nslices)
-{
-    return (int64_t)((p.npix + 63) / 64) * p.nang * nslices >= 2048;
-}
-
 int ss_forward_epi(const Plan& p, int epi, int ones, const float* image, float* out,
                    int nslices, int accumulate, const EpiArgs& e, hipStream_t st,
                    int* blocks_per_slice)
@@ -325,18 +317,24 @@ int ss_forward_epi(const Plan& p, int epi, int ones, const float* image, float* 
                                         blocks_per_slice);
     }
     if (blocks_per_slice) *blocks_per_slice = 0;
-    const TransposedCopy tc(p, !ones && ss_transposes(p, nslices), image, nslices, st);
-    const float* imageT = tc.get();
-    int rc;
-    if (p.arith == ITOMO_ARITH_FAST)
-        rc = p.method == 0
-                 ? dispatch_ss_fwd<ITOMO_ARITH_FAST, 0>(p, epi, ones, image, imageT, out, nslices, accumulate, e, st)
-                 : dispatch_ss_fwd<ITOMO_ARITH_FAST, 1>(p, epi, ones, image, imageT, out, nslices, accumulate, e, st);
-    else
-        rc = p.method == 0
-                 ? dispatch_ss_fwd<ITOMO_ARITH_IEEE, 0>(p, epi, ones, image, imageT, out, nslices, accumulate, e, st)
-                 : dispatch_ss_fwd<ITOMO_ARITH_IEEE, 1>(p, epi, ones, image, imageT, out, nslices, accumulate, e, st);
-    if (rc) return rc;
+    for (int z = 0; z < nslices;) {
+        const float* im = image ? image + (int64_t)z * p.npix * p.npix : nullptr;
+        float* o = out + (int64_t)z * p.nang * p.npix;
+        const TransposedCopy tc(p, !ones, im, nslices - z, st);
+        const float* imT = tc.get();
+        const int n = tc.slices();
+        int rc;
+        if (p.arith == ITOMO_ARITH_FAST)
+            rc = p.method == 0
+                     ? dispatch_ss_fwd<ITOMO_ARITH_FAST, 0>(p, epi, ones, im, imT, o, n, accumulate, e, st)
+                     : dispatch_ss_fwd<ITOMO_ARITH_FAST, 1>(p, epi, ones, im, imT, o, n, accumulate, e, st);
+        else
+            rc = p.method == 0
+                     ? dispatch_ss_fwd<ITOMO_ARITH_IEEE, 0>(p, epi, ones, im, imT, o, n, accumulate, e, st)
+                     : dispatch_ss_fwd<ITOMO_ARITH_IEEE, 1>(p, epi, ones, im, imT, o, n, accumulate, e, st);
+        if (rc) return rc;
+        z += n;
+    }
     return check_hip(hipGetLastError(), "ss forward launch");
 }
 

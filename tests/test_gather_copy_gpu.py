@@ -111,3 +111,42 @@ def test_copy_in_an_iteration_that_allocates_nothing(oper):
         p._h, y.data_ptr(), b.data_ptr(), R.data_ptr(), C.data_ptr(), work.data_ptr(), nz, -1.0,
         None, stream_handle()), "sirt_iterate_noalloc")
     assert torch.equal(x, y)
+
+
+@pytest.mark.parametrize("oper", ["pd", "ss"])
+def test_first_calls_and_growing_stacks_leave_another_capture_alone(oper):
+    n, nz = 65, LINE[oper] // (2 * V) + 8
+    x = torch.rand((4 * nz, n, n), device="cuda")
+    p, q = plan(oper, n), plan(oper, n)
+    want = p.forward(x).clone()
+    out, a, g = torch.zeros_like(want), torch.zeros(64, device="cuda"), torch.cuda.CUDAGraph()
+    side = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(g):               # global mode: a plain allocation anywhere breaks it
+        a += 1
+        with torch.cuda.stream(side):       # not captured
+            for k in (1, nz, 2 * nz, 4 * nz, nz):
+                q.forward(x[:k], out=out[:k])
+    torch.cuda.synchronize()
+    assert torch.equal(out, want)
+    g.replay()
+    torch.cuda.synchronize()
+    assert (a == 1).all()
+    free = torch.cuda.mem_get_info()[0]
+    with torch.cuda.stream(side):
+        for k in (4 * nz, nz, 3 * nz):
+            q.forward(x[:k], out=out[:k])
+    torch.cuda.synchronize()
+    assert torch.cuda.mem_get_info()[0] == free
+
+
+@pytest.mark.parametrize("oper", ["pd", "ss"])
+def test_stack_whose_copies_come_in_turns(oper):
+    n, nz = 257, 1200       # 1015 slices of 257^2 fill 256 MiB
+    x = torch.rand((nz, n, n), device="cuda")
+    ang = ANGLES[::4].copy()
+    p = Plan(oper, n, np.fft.fftshift(ang) if oper == "pd" else ang)
+    got = p.forward(x)
+    for z in (0, 599, 600, 1014, 1015, nz - 1):
+        same(got[z].cpu().numpy(), FWD[oper](x[z].cpu().numpy(), ang, O.FAST, 1))
+    assert torch.equal(p.forward(x, out=torch.zeros_like(got), accumulate=True), got)
