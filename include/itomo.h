@@ -126,14 +126,16 @@ int itomo_plan_trig(const itomo_plan *plan, float *s_host, float *c_host);
  * C has no launch shapes; used by the autotuner).  Forward variant f in
  * [0, ITOMO_FWD_VARIANTS): 256 / 128 / 64 bins per block.  Back variant b in
  * [0, ITOMO_BACK_VARIANTS): 64x64 tile with 4x4 pixels per thread / 32x32 with 2x2 /
- * 32x32 with 4x4 / 16x16 with one.  A plan starts with 64 bins and a back tile chosen per
- * call from the number of pixels in it (get_shapes reports the choice for one slice).
+ * 32x32 with 4x4 / 16x16 with one; or ITOMO_BACK_AUTO, chosen per call from the number of
+ * pixels in it.  A plan starts with 64 bins and ITOMO_BACK_AUTO; get_shapes reports what
+ * set_shapes would take to keep it so.
  * Every shape produces bit-identical projections and iterates; FP64
  * monitor sums follow the block partition and may differ in the last bits.
  * Ray-, pixel-driven and slant-stacking plans accept only (0, 0).  Not to be called while work using the plan is
  * queued on another stream. */
 #define ITOMO_FWD_VARIANTS 3
 #define ITOMO_BACK_VARIANTS 4
+#define ITOMO_BACK_AUTO 255
 int itomo_plan_set_shapes(itomo_plan *plan, int fwd_variant, int back_variant);
 int itomo_plan_get_shapes(const itomo_plan *plan, int *fwd_variant, int *back_variant);
 

@@ -106,6 +106,7 @@ _SIGS = {
 UNET_MSE_WORK = 1024  # ITOMO_UNET_MSE_WORK
 FWD_VARIANTS = 3      # ITOMO_FWD_VARIANTS
 BACK_VARIANTS = 4     # ITOMO_BACK_VARIANTS
+BACK_AUTO = 255       # ITOMO_BACK_AUTO
 FILTERS = {"ramp": 0, "shepp-logan": 1, "cosine": 2, "hamming": 3, "hanning": 4, "none": 5}
 
 VEC_WORK_PER_SLICE = 771

@@ -114,7 +114,8 @@ class Plan:
     # -- launch shapes --------------------------------------------------------------
     @property
     def shapes(self):
-        """(forward variant, back variant) of the distance-driven launches."""
+        """(forward variant, back variant) of the distance-driven launches; back variant
+        ``_lib.BACK_AUTO``: chosen per call."""
         f, b = ctypes.c_int(), ctypes.c_int()
         L.check(L.lib().itomo_plan_get_shapes(self._h, ctypes.byref(f), ctypes.byref(b)),
                 "plan_get_shapes")

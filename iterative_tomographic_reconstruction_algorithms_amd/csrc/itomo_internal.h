@@ -92,7 +92,7 @@ struct Plan {
     int* d_range;    // slant-stacking: [view][bin] stepped range [u0, u1) (int2), clipped
                      // to the image
     int fwd_var;     // distance-driven launch shapes (kFwdBins / kBackTiles index)
-    int back_var;    // kBackAuto: chosen per launch (back_variant)
+    int back_var;    // ITOMO_BACK_AUTO: chosen per launch (back_variant)
     int method;      // pixel-driven: 0 nearest bin, 1 linear split (radon_pd.c:57-85)
     // Device scratch owned by the plan (FP64 partial sums, ray-driven back-projection
     // image).  Grown on first use; a plan must not be used from two streams at once.
@@ -179,7 +179,6 @@ constexpr int kNumBackVariants = 4;
 constexpr int kBackTiles[kNumBackVariants][2] = {{64, 4}, {32, 2}, {32, 4}, {16, 1}};
 constexpr int kDdFwdDefault = 2;            // 64 bins: the fastest or within 2% of it from 64^2
                                             // to 2048^2 (256-bin blocks: 9-50% slower)
-constexpr int kBackAuto = -1;
 constexpr int kRdBlock = 64;
 constexpr int kEpiChunk = 256 * 8;          // pixels per elementwise-epilogue block
 
@@ -214,7 +213,7 @@ inline int back_variant_for(size_t tiles64, size_t tiles32)
 
 inline int back_variant(const Plan& p, int nslices)
 {
-    if (p.back_var != kBackAuto) return p.back_var;
+    if (p.back_var != ITOMO_BACK_AUTO) return p.back_var;
     return back_variant_for(dd_back_blocks(p.npix, 64) * nslices,
                             dd_back_blocks(p.npix, 32) * nslices);
 }

@@ -411,7 +411,7 @@ static int plan_create(itomo_plan** out, int projector, int npix, const float* a
     p->method = method;
     if (projector == ITOMO_PROJ_DD) {
         p->fwd_var = kDdFwdDefault;
-        p->back_var = kBackAuto;
+        p->back_var = ITOMO_BACK_AUTO;
     }
     size_t bytes = 0;
     int st = ITOMO_OK;
@@ -556,7 +556,9 @@ int itomo_plan_set_shapes(itomo_plan* p, int fwd_variant, int back_variant)
     if (!p) return set_error(ITOMO_EINVAL, "plan_set_shapes: null plan");
     const int nf = p->projector == ITOMO_PROJ_DD ? kNumFwdVariants : 1;
     const int nb = p->projector == ITOMO_PROJ_DD ? kNumBackVariants : 1;
-    if (fwd_variant < 0 || fwd_variant >= nf || back_variant < 0 || back_variant >= nb)
+    const bool by_call = p->projector == ITOMO_PROJ_DD && back_variant == ITOMO_BACK_AUTO;
+    if (fwd_variant < 0 || fwd_variant >= nf || back_variant < 0 ||
+        (back_variant >= nb && !by_call))
         return set_error(ITOMO_EINVAL, "plan_set_shapes: variants (%d, %d) outside [0, %d) x "
                                        "[0, %d)", fwd_variant, back_variant, nf, nb);
     p->fwd_var = fwd_variant;
@@ -569,7 +571,7 @@ int itomo_plan_get_shapes(const itomo_plan* p, int* fwd_variant, int* back_varia
     if (!p || !fwd_variant || !back_variant)
         return set_error(ITOMO_EINVAL, "plan_get_shapes: null pointer");
     *fwd_variant = p->fwd_var;
-    *back_variant = itomo::back_variant(*p, 1);
+    *back_variant = p->back_var;
     return ITOMO_OK;
 }
 

@@ -91,6 +91,26 @@ def test_bad_shapes_rejected():
         rd.set_shapes(1, 0)
 
 
+def test_saving_and_restoring_shapes_keeps_the_choice_per_call():
+    p = dd_plan(64, 20)
+    assert p.shapes[1] == L.BACK_AUTO
+    p.set_shapes(*p.shapes)
+    p.set_shapes(1, p.shapes[1])
+    assert p.shapes == (1, L.BACK_AUTO)
+    p.set_shapes(0, 2)
+    assert p.shapes == (0, 2)
+    p.set_shapes(2, L.BACK_AUTO)
+    assert p.shapes == (2, L.BACK_AUTO)
+    for b in (L.BACK_VARIANTS, L.BACK_AUTO - 1, L.BACK_AUTO + 1):
+        with pytest.raises(L.ItomoError):
+            p.set_shapes(0, b)
+    for oper in ("rd", "pd", "ss"):
+        q = Plan(oper, 32, (angles_deg(8) * np.pi / 180).astype(np.float32))
+        assert q.shapes == (0, 0)
+        with pytest.raises(L.ItomoError):
+            q.set_shapes(0, L.BACK_AUTO)
+
+
 def test_tune_sets_valid_shapes_and_caches(tmp_path):
     path = str(tmp_path / "shapes.json")
     p = dd_plan(256, 90)
