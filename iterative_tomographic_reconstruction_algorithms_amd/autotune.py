@@ -2,16 +2,18 @@
 
 The forward kernel can run 256, 128 or 64 bins of a view per block and the back kernel
 64x64 tiles (4x4 pixels per thread), 32x32 tiles (2x2 or 4x4) or 16x16 tiles (one pixel
-per thread); a plan that is not tuned picks the tile per launch.  Which is fastest depends on the image size, the view count and how many slices share a launch
-(a 256^2 single slice has only 16 of the large back tiles -- far too few blocks for 256
-compute units).  Every shape accumulates each output element in the same order, so the
-choice never changes a projection or an iterate.
+per thread); a plan that is not tuned picks the tile per launch.  Which is fastest depends
+on the image size, the view count and how many slices share a launch (a 256^2 single
+slice has only 16 of the large back tiles -- far too few blocks for 256 compute units).
+Every shape accumulates each output element in the same order, so the choice never changes
+a projection or an iterate.
 
 :func:`tune` times each forward and each back shape of a plan on the GPU with HIP
 events on the current stream, keeps the fastest and records it in a JSON cache keyed by
 (device, projector, arithmetic, npix, nang, nslices); the bucket widths make one entry
-serve nearby geometries.  The cache lives at ``$ITOMO_SHAPE_CACHE`` or
-``~/.cache/itomo/shapes.json``.
+serve nearby geometries.  An entry names the revision of the kernels that it was timed with
+(``KERNELS``); one of another revision is timed again.  The cache lives at
+``$ITOMO_SHAPE_CACHE`` or ``~/.cache/itomo/shapes.json``.
 """
 import json
 import os
@@ -19,7 +21,9 @@ import tempfile
 
 from . import _lib as L
 
-__all__ = ["tune", "bucket_key", "load_cache", "store_entry", "cache_path", "fastest"]
+__all__ = ["tune", "bucket_key", "load_cache", "store_entry", "cache_path", "fastest", "usable"]
+
+KERNELS = 2   # to be raised with every change of the kernels' relative speeds
 
 
 def cache_path(path=None):
@@ -69,6 +73,13 @@ def store_entry(key, entry, path=None):
     os.replace(tmp, p)
 
 
+def usable(entry):
+    """Whether a cache entry holds shapes of this build, timed with its kernels."""
+    return (isinstance(entry, dict) and entry.get("kernels") == KERNELS
+            and entry.get("fwd") in range(L.FWD_VARIANTS)
+            and entry.get("back") in range(L.BACK_VARIANTS))
+
+
 def fastest(times):
     """Index of the smallest time (first one on ties)."""
     best = 0
@@ -105,10 +116,9 @@ def tune(plan, nslices=1, reps=3, use_cache=True, path=None):
                      plan.nang, nslices)
     if use_cache:
         hit = load_cache(path).get(key)
-        if (isinstance(hit, dict) and 0 <= hit.get("fwd", -1) < L.FWD_VARIANTS
-                and 0 <= hit.get("back", -1) < L.BACK_VARIANTS):
+        if usable(hit):
             plan.set_shapes(hit["fwd"], hit["back"])
-            return dict(hit, cached=True)
+            return dict({k: v for k, v in hit.items() if k != "kernels"}, cached=True)
 
     g = torch.Generator(device=dev).manual_seed(0)
     x = torch.rand((nslices, plan.npix, plan.npix), device=dev, generator=g)
@@ -126,5 +136,5 @@ def tune(plan, nslices=1, reps=3, use_cache=True, path=None):
              "fwd_ms": [round(t, 4) for t in fwd_ms], "back_ms": [round(t, 4) for t in back_ms]}
     plan.set_shapes(entry["fwd"], entry["back"])
     if use_cache:
-        store_entry(key, entry, path)
+        store_entry(key, dict(entry, kernels=KERNELS), path)
     return dict(entry, cached=False)

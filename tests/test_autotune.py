@@ -42,3 +42,14 @@ def test_fastest_takes_first_minimum():
     assert T.fastest([3.0, 1.0, 1.0]) == 1
     assert T.fastest([0.5]) == 0
     assert T.fastest([2.0, 2.0, 3.0]) == 0
+
+
+def test_entries_of_other_kernels_are_not_used():
+    e = {"kernels": T.KERNELS, "fwd": 2, "back": 3, "fwd_ms": [1.0] * 3, "back_ms": [1.0] * 4}
+    assert T.usable(e)
+    assert T.usable(json.loads(json.dumps(e)))
+    assert not T.usable({k: v for k, v in e.items() if k != "kernels"})   # written before them
+    assert not T.usable(dict(e, kernels=T.KERNELS - 1))
+    for bad in (None, [], 3, "x", dict(e, fwd=3), dict(e, fwd=-1), dict(e, back=4), dict(e, back="1"),
+                dict(e, back=None)):
+        assert not T.usable(bad)

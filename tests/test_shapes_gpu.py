@@ -122,3 +122,7 @@ def test_tune_sets_valid_shapes_and_caches(tmp_path):
     q = dd_plan(250, 80)        # same bucket
     r2 = autotune.tune(q, nslices=1, path=path)
     assert r2["cached"] and q.shapes == p.shapes
+    entry = autotune.load_cache(path)
+    autotune.store_entry(*[(k, dict(e, kernels=autotune.KERNELS - 1)) for k, e in entry.items()][0], path)
+    assert not autotune.tune(q, nslices=1, reps=1, path=path)["cached"]   # other kernels' times
+    assert autotune.tune(q, nslices=1, path=path)["cached"]
