@@ -52,6 +52,7 @@ struct itomo_batch {
     int total_slices = 0;
     int nfwd = 0, nback = 0;
     int grid = 0;
+    int max_npix = 0;
     int back_var = 0;   // one back tile for all members (back_variant_for over all slices)
     std::vector<itomo::BatchMember> h_members;
     std::vector<const itomo_plan*> plans;
@@ -89,8 +90,8 @@ __device__ __forceinline__ int next_item(int* counter)
 
 // Five waves per SIMD (96 registers): the kernel holds every forward path and the fused
 // update.  Measured on 16 slices of 1024^2 x 900 (forward and back): 14.68 ms per iteration at
-// four waves, 14.47 at five, 15.03 at six, 16.23 at eight.  PATH: kFwdSmall up to kFwdLargeWaves
-// items, kFwdLarge beyond, as the per-plan launches choose.
+// four waves, 14.47 at five, 15.03 at six, 16.23 at eight.  PATH: as a launch of all items
+// would choose for the largest member.
 template <int PATH>
 __global__ void __launch_bounds__(kBatchFwdBlock) __attribute__((amdgpu_waves_per_eu(5)))
 batch_fwd_kernel(const BatchMember* __restrict__ mem, const BatchItem* __restrict__ items,
@@ -203,6 +204,7 @@ int itomo_batch_create(itomo_batch** out, int nmembers, const itomo_plan* const*
     size_t tiles64 = 0, tiles32 = 0;
     for (int m = 0; m < nmembers; ++m)
         if (plans[m] && nslices[m] > 0) {
+            B->max_npix = std::max(B->max_npix, plans[m]->npix);
             tiles64 += dd_back_blocks(plans[m]->npix, 64) * nslices[m];
             tiles32 += dd_back_blocks(plans[m]->npix, 32) * nslices[m];
         }
@@ -320,7 +322,7 @@ int itomo_batch_sirt_iterate(itomo_batch* B, float pc_beta, void* stream)
     }
     reset_counter_kernel<<<1, 1, 0, st>>>(B->d_counter);
     const int fgrid = std::min(B->grid * (256 / kBatchFwdBlock), B->nfwd);
-    if (B->nfwd <= kFwdLargeWaves)
+    if (fwd_path(B->max_npix, B->nfwd) == kFwdSmall)
         batch_fwd_kernel<kFwdSmall><<<fgrid, kBatchFwdBlock, 0, st>>>(B->d_members, B->d_fwd,
                                                                       B->nfwd, B->d_counter);
     else

@@ -91,7 +91,7 @@ void launch_fwd_b(const Plan& p, const float* image, const float* imageT, float*
                   int nslices, int accumulate, const EpiArgs& e, hipStream_t st)
 {
     const int64_t waves = (int64_t)((p.npix + 63) / 64) * p.nang * nslices;
-    if (ONES || waves <= kFwdLargeWaves)
+    if (ONES || fwd_path(p.npix, waves) == kFwdSmall)
         launch_fwd_path<ARITH, EPI, ONES, B, kFwdSmall>(p, image, imageT, out, nslices,
                                                         accumulate, e, st);
     else

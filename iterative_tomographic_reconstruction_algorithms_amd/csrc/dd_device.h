@@ -894,16 +894,9 @@ __device__ __forceinline__ float fwd_staged(const DdView& g, const float* __rest
 }
 
 // How a forward launch takes its views: those with at most fwd_staged_max(path) candidates are
-// staged, the others go along diagonals.  A staged block reads each line once through LDS, a
-// diagonal one through the L1; staging wins for up to 6 candidates once the launch fills the
-// GPU, the diagonals from 4 on while it does not (their chains are shorter).  Staged up to 6
-// against up to 3, in us: 363^2 x 251 x 3 slices (4518 waves) 123 and 112, 724^2 x 512 (6144)
-// 245 and 223, 1024^2 x 720 (11520) 531 and 525, 1448^2 x 900 (20700) 1186 and 1364,
-// 2048^2 x 1800 (57600) 4432 and 6014; the line is drawn at kFwdLargeWaves.  Both kinds of views
-// share one launch: their waves wait for different units.  (The diagonal ones in a launch of
-// their own: 4967 us at 2048^2 x 1800 after the staged ones, 4603 beside them on another stream.)
-constexpr int kFwdSmall = 0, kFwdLarge = 1;
-constexpr int64_t kFwdLargeWaves = 10240;
+// staged, the others go along diagonals (which path: fwd_path).  Both kinds of views share one
+// launch: their waves wait for different units.  (The diagonal ones in a launch of their own: 4967
+// us at 2048^2 x 1800 after the staged ones, 4603 beside them on another stream, 4432 so.)
 constexpr int fwd_staged_max(int path) { return path == kFwdSmall ? 3 : 6; }
 
 // Forward projection: one thread per (bin, view, slice).

@@ -211,6 +211,21 @@ inline int back_variant_for(size_t tiles64, size_t tiles32)
     return tiles32 >= 384 ? 1 : 3;
 }
 
+// How a forward launch takes the views with 4 to 6 candidates per bin and line: along diagonals
+// through the L1 (kFwdSmall) or staged line by line in LDS (kFwdLarge), see fwd_staged_max.  The
+// diagonals' chains are shorter, and their loads hit the caches while the image is small; staging
+// reads each line once.  `waves` is that of the launch (64 bins each).  Staged against diagonal,
+// MLEM iterations in us: 512^2 x 360 views x 6 slices (17280 waves) 709/690, x 27 2494/2412; 640^2
+// x 450 x 2 (9000) 517/521, x 4 (18000) 851/886; 800^2 x 560 (7280) 560/523; 1024^2 x 656 (10496)
+// 828/807, x 720 (11520) 897/890, x 900 (14400) 1088/1143; 1100^2 x 500 (9000) 744/720; 1200^2 x
+// 400 (7600) 723/761; 1448^2 x 200 (4600) 600/668; 2048^2 x 100 (3200) 692/746, x 328 (10496)
+// 1419/1380, x 1800 (57600, forward alone) 4432/6014.
+constexpr int kFwdSmall = 0, kFwdLarge = 1;
+inline int fwd_path(int npix, int64_t waves)
+{
+    return npix >= 1200 || (npix >= 600 && waves >= 12288) ? kFwdLarge : kFwdSmall;
+}
+
 inline int back_variant(const Plan& p, int nslices)
 {
     if (p.back_var != ITOMO_BACK_AUTO) return p.back_var;

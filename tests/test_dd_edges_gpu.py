@@ -60,11 +60,14 @@ def test_forward_matches_oracle(n, arith):
         np.testing.assert_array_equal(p.forward(xt).cpu().numpy()[0], want, err_msg="shape %d" % f)
 
 
-@pytest.mark.parametrize("n,nz", [(65, 190), (130, 120), (17, 400)])
+@pytest.mark.parametrize("n,nz", [(65, 190), (130, 120), (17, 400), (601, 42), (1199, 24), (1201, 1)])
 def test_large_launches_match_oracle(n, nz):
-    # more than 10240 waves of 64 bins: views with 4 to 6 candidates are staged
+    # large stacks of small images, and launches whose views with 4 to 6 candidates are staged:
+    # from 600 pixels a side from 12288 waves of 64 bins on, from 1200 always
     x, _ = arrays(n, ANGLES.size, nz)
-    assert (n + 63) // 64 * ANGLES.size * nz > 10240
+    waves = (n + 63) // 64 * ANGLES.size * nz
+    assert waves > 10240 or n >= 1200
+    assert n < 600 or n >= 1200 or waves >= 12288
     p = Plan("dd", n, ANGLES)
     for f in range(L.FWD_VARIANTS):
         p.set_shapes(f, p.shapes[1])
@@ -86,7 +89,7 @@ def lines_met(n, theta, s, c):
     return np.minimum(e0, e1) - 3.01, np.maximum(e0, e1) + 3.01, first, w
 
 
-@pytest.mark.parametrize("n,nz", [(130, 16), (130, 120), (65, 190)])
+@pytest.mark.parametrize("n,nz", [(130, 16), (130, 120), (65, 190), (1201, 4)])
 def test_infinite_pixel_reaches_only_bins_about_its_line(n, nz):
     """A bin that no line range or candidate run takes to the pixel stays finite (weights of
     zero do reach the rest: the reference's own build assumes finite data)."""
