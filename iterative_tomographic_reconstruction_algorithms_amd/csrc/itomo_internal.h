@@ -197,14 +197,18 @@ inline size_t dd_back_blocks(int npix, int tile)
     return t * t;
 }
 
-// Back tile for `pixels` pixels in a launch (npix^2 x slices, rounded up to tiles): the
-// largest that still gives the 256 compute units blocks enough.  A wave alone on its SIMD
-// issues about every 8th cycle, four together about every 2nd, so 64 x 64 tiles (1.6 times
+// Back tile for a launch of so many 64 x 64 or 32 x 32 tiles (npix^2 x slices, rounded up to
+// tiles): the largest that still gives the 256 compute units blocks enough.  A wave alone on its
+// SIMD issues about every 8th cycle, four together about every 2nd, so 64 x 64 tiles (1.6 times
 // the work per instruction of single pixels) pay from 3 blocks of 4 waves per compute unit,
-// 32 x 32 tiles from 1.5.  64/32/16 tiles, in us: 363^2 x 251 207/96/57, 363^2 x 3 slices
-// 202/100/88, 512^2 x 360 288/137/92, 724^2 x 512 406/223/221, 1024^2 x 720 578/360/507,
-// 1448^2 x 900 1010/850/1181, 1024^2 x 900 x 4 slices 1287/1437/2235, 2048^2 x 1800
-// 2500/2970/4434.
+// 32 x 32 tiles from 1.5.  The line is drawn for iterations, where a launch begins on the tail
+// of the forward one and reduces its blocks' sums: MLEM iterations with 64/32/16 tiles, us,
+// 512^2 x 360 views (64 and 256 tiles) 400/243/194; 363^2 x 251 x 2 slices (72, 288) 295/185/156;
+// 448^2 x 310 x 2 (98, 392) 403/268/265; 363^2 x 251 x 3 (108, 432) 328/216/218; 672^2 x 470
+// (121, 441) 566/366/387; 512^2 x 360 x 2 (128, 512) 457/300/329; 724^2 x 512 x 4 (576, 2116)
+// 1271/1196/1398; 512^2 x 360 x 11 (704, 2816) 1132/1161/1374.  A back projection by itself
+// favours the smaller tiles a little longer: 363^2 x 251 x 3 203/101/88, 672^2 x 470 372/187/167,
+// 512^2 x 360 x 2 288/143/151.
 inline int back_variant_for(size_t tiles64, size_t tiles32)
 {
     if (tiles64 >= 768) return 0;

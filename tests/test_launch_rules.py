@@ -22,6 +22,13 @@ def evaluate(tmp_path, expressions):
     return [int(v) for v in out.split()]
 
 
+# npix, slices: us with 64^2, 32^2 and 16^2 tiles
+BACK = {(512, 1): (400, 243, 194), (363, 2): (295, 185, 156), (448, 2): (403, 268, 265),
+        (363, 3): (328, 216, 218), (384, 3): (348, 228, 230), (480, 2): (435, 290, 297),
+        (672, 1): (566, 366, 387), (192, 13): (195, 131, 138), (704, 1): (608, 395, 417),
+        (320, 5): (311, 209, 218), (512, 2): (457, 300, 329), (363, 4): (344, 245, 251),
+        (724, 4): (1271, 1196, 1398), (512, 11): (1132, 1161, 1374)}
+
 # npix, views, slices: us with views of 4 to 6 candidates along diagonals and staged
 FORWARD = {(64, 45, 200): (78, 90), (64, 45, 400): (117, 131), (130, 100, 133): (392, 417),
            (256, 180, 14): (242, 257), (256, 180, 111): (1259, 1347), (363, 251, 53): (1710, 1750),
@@ -32,6 +39,13 @@ FORWARD = {(64, 45, 200): (78, 90), (64, 45, 400): (117, 131), (130, 100, 133): 
            (1100, 500, 1): (720, 744), (1100, 800, 1): (1200, 1092), (1200, 400, 1): (761, 723),
            (1448, 200, 1): (668, 600), (1448, 900, 1): (2246, 2026), (2048, 100, 1): (746, 692),
            (2048, 180, 1): (991, 861), (2048, 328, 1): (1380, 1419)}
+
+
+def test_back_tile(tmp_path):
+    got = evaluate(tmp_path, ["back_variant_for(dd_back_blocks(%d, 64) * %d, dd_back_blocks(%d, 32) * %d)"
+                              % (n, z, n, z) for n, z in BACK])
+    for (case, us), v in zip(BACK.items(), got):
+        assert us[{0: 0, 1: 1, 3: 2}[v]] <= 1.04 * min(us), (case, us, v)
 
 
 def test_forward_path(tmp_path):
