@@ -59,6 +59,15 @@ static int dd_multi_cross(const DdView& g, int npix)
     return (r - 1.0) <= 4.0 * m * std::ldexp(1.0, -23) ? 1 : 0;
 }
 
+// Pixels that can overlap one bin on one line, w = |rinv| of them long: floor(w + 1/4) + 2 while
+// the keys' rounding stays below 1/16 (w < 30.75, npix <= 32766).  Wider views are counted in fours:
+// at 32766 pixels a side and w = 5730 the keys lie 8 apart and a bin can reach one pixel further.
+static int dd_candidates(float rinv)
+{
+    const int n = (int)std::floor((double)rinv + 0.25) + 2;
+    return n <= 32 ? n : (n + 3) & ~3;
+}
+
 static int make_dd_view(float theta, int arith, int row, int npix, DdView* g)
 {
     float s, c;
@@ -79,7 +88,7 @@ static int make_dd_view(float theta, int arith, int row, int npix, DdView* g)
                              (double)theta);
         g->kind = DD_SWEEP_ROWS;
         g->rinv = 1.0f / s;
-        g->ncand = (int)std::floor((double)g->rinv + 0.25) + 2;
+        g->ncand = dd_candidates(g->rinv);
         g->t = c * g->rinv;
         g->a = c;
         g->b = s;
@@ -92,7 +101,7 @@ static int make_dd_view(float theta, int arith, int row, int npix, DdView* g)
                              (double)theta);
         g->kind = DD_SWEEP_COLS;
         g->rinv = 1.0f / c;
-        g->ncand = (int)std::floor((double)g->rinv + 0.25) + 2;
+        g->ncand = dd_candidates(g->rinv);
         g->t = s * g->rinv;
         g->a = s;
         g->b = c;
