@@ -751,14 +751,6 @@ template <int B>
 constexpr int fwd_stage_floats() { return 16 * B; }
 constexpr int kFwdStageMaxLines = 8;
 
-// Pixels of the staged window beyond (NC-1)*B, so that it holds every candidate of a
-// block (see fwd_staged): max(0, NC + 7 - B/4), rounded up to a multiple of 4.
-template <int B, int NC>
-constexpr int fwd_window_extra()
-{
-    return NC + 7 - B / 4 > 0 ? (NC + 7 - B / 4 + 3) / 4 * 4 : 0;
-}
-
 // Forward projection of one sweep view with at most NC candidate pixels per bin and line
 // (bins narrower than w < NC - 1.25 pixels), for the B bins [bx*B, +B) of a block.
 // Lines are processed in chunks of FL: for each line of a chunk the block copies the
@@ -768,15 +760,15 @@ constexpr int fwd_window_extra()
 // LDS.  A bin's first candidate lies less than B*w + 6 pixels past q0: less than
 // (B-1)*w + 1 + 5 for a bin that starts on the line, and for the last bin up to one bin
 // width more where it starts left of the line's first pixel and its first candidate is
-// clamped up to that pixel.  With W = (NC-1)*B + max(0, NC + 7 - B/4) >= B*w + 6 + NC
-// the window holds every candidate of every bin that meets the line.  q0 itself is kept in
-// [-(W - NC), npix - 1], which moves it only on lines that every bin of the block misses, so
-// that each first candidate, clamped into the line, lies in the window, whatever the bin.
-// Lines run over the union of the block's per-bin line ranges; lines that
-// miss a bin add nothing to it.  A chunk always runs all its FL lines (straight-line code, so
-// the LDS reads of one line hide behind the sums of another): those past the block's last line
-// are zeros with the line end kNoLine, which makes every weight 0.  Every thread of the block takes part
-// (inactive threads, past the last bin, compute a copy of the last bin and store nothing).
+// clamped up to that pixel.  With W = (NC-1)*B >= B*w + 6 + NC (for w < NC - 1.25 and B >=
+// 4 (NC + 6)) the window holds every candidate of every bin that meets the line.  q0 itself is
+// kept in [-(W - NC), npix - 1], which moves it only on lines that every bin of the block misses,
+// so that each first candidate, clamped into the line, lies in the window, whatever the bin.
+// Lines run over the union of the block's per-bin line ranges; lines that miss a bin add nothing
+// to it.  A chunk always runs all its FL lines (straight-line code, so the LDS reads of one line
+// hide behind the sums of another): those past the block's last line are zeros with the line end
+// kNoLine, which makes every weight 0.  Every thread of the block takes part (inactive threads,
+// past the last bin, compute a copy of the last bin and store nothing).
 // sImg holds FLOATS floats, sMeta kFwdStageMaxLines entries {byte offset of pixel 0, L*}.
 constexpr float kNoLine = -1e30f;
 
@@ -786,7 +778,8 @@ __device__ __forceinline__ float fwd_staged(const DdView& g, const float* __rest
                                             int bx, int d, float acc, float* sImg,
                                             float2* sMeta)
 {
-    constexpr int W = (NC - 1) * B + fwd_window_extra<B, NC>();
+    static_assert(B >= 4 * (NC + 6), "the window holds a block's candidates");
+    constexpr int W = (NC - 1) * B;
     constexpr int FL = FLOATS / W < kFwdStageMaxLines ? FLOATS / W : kFwdStageMaxLines;
     constexpr int N4 = FL * (W / 4);          // 16-byte pieces per chunk
     constexpr int PER = (N4 + B - 1) / B;     // pieces per thread
