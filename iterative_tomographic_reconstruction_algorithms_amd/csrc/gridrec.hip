@@ -281,9 +281,11 @@ __device__ __forceinline__ void gr_gather(float2& acc, const float2* __restrict_
 // Polar -> Cartesian gridding, gathered per grid point (a = iu row, b = iv column).  A block
 // takes 8 x 8 grid points.  It first lists the angles whose ray comes within a kernel window of
 // the tile (away from the centre a few per cent of them: tested point by point, all angles took
-// 905 us at 512^2 x 360, now 151), then its 8 waves share the list, a wave evaluating one angle for all
-// 64 points; the waves' sums are added in wave order.  The tiles around the centre, where every
-// angle passes, set the time: hence the small tile and the split over waves.
+// 905 us at 512^2 x 360, now 151), then its 8 waves share the list, a wave evaluating one angle for
+// all 64 points; the waves' sums are added in wave order (eight partial sums, where one thread
+// took all angles in turn: results differ from that in the last bits, and not from run to run).
+// The tiles around the centre, where every angle passes, set the time: hence the small tile and
+// the split over waves.
 template <bool LDS_LUT>
 __global__ void __launch_bounds__(64 * kGridWaves)
 gr_grid_back_kernel(const float2* __restrict__ c1, const float2* __restrict__ c2,

@@ -25,11 +25,12 @@
 // overflow of views r-1 and r+1); flat indices outside the array, where the reference
 // writes out of bounds, are skipped.
 //
-// Both are bound by instruction issue, about a third of it FP64 (every update converts, adds
-// and rounds), so the loops are straight-line: candidates are evaluated several at a time, a
-// hit selects the updated sum instead of branching to it, and the products, exact in
-// double, are formed once for a sample's two additions.  Method 1, us before and after that and
-// the transposed copy: 64^2 x 45 views forward 62 -> 55, back 31 -> 23; 511^2 x 360 741 -> 595
+// Every update converts, adds in double and rounds: a third of the forward's and half of the
+// back's instructions are conversions and FP64, at half rate, and each sum is one chain.  At
+// 511^2 x 360 the VALU is busy 49% and 56% of the time with 1.5 and 3.4 waves per SIMD.  So the
+// loops are straight-line: candidates are evaluated several at a time, a hit selects the
+// updated sum instead of branching to it, and the products, exact in double, are formed once
+// for a sample's two additions.  Method 1, us before and after that and the transposed copy: 64^2 x 45 views forward 62 -> 55, back 31 -> 23; 511^2 x 360 741 -> 595
 // and 320 -> 237; 1024^2 x 720 5517 -> 3551 and 1810 -> 1379.
 #include "epilogue.h"
 

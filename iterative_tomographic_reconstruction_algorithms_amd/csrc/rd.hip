@@ -563,7 +563,9 @@ rd_fwd_record_kernel(const RdView* __restrict__ geom, int npix, int* __restrict_
                 rd_walk_record<ARITH, FILL>(npix, p1, p2, words, rd_fwd_steps(g, npix, t), t);
             }
             // the chunk's bins begin their next sub-ray together, as near to each other as they
-            // began the first (it costs no words: the longest list sets the chunk's length)
+            // began the first: a chunk is then as long as its longest sub-rays one after
+            // another, not as its longest list (256^2 x 304: 0.01% more words; the call 157 us
+            // instead of 234)
             int m = words.n;
             for (int off = 32; off > 0; off >>= 1) m = max(m, __shfl_xor(m, off, 64));
             words.pad(m);

@@ -18,9 +18,10 @@
 // No atomics; both directions are bit-identical to the reference wherever its samples
 // stay inside the image.
 //
-// The forward is bound by its gathers (a lane per bin reads the sampled index, so one of the
-// two view families strides by rows) and the back by instruction issue; us before and after
-// lockstep steps, the transposed copy and the two or three candidate bins, method 1:
+// Both wait for their gathers (a lane per bin reads the sampled index, so in the forward one of
+// the two view families strides by rows): at 512^2 x 361 for 66% and 54% of the wave cycles, at
+// 2.1 and 2.5 waves per SIMD, the VALU busy 23% and 28% of the time.  us before and after lockstep
+// steps, the transposed copy and the two or three candidate bins, method 1:
 // 511^2 x 360 views forward 346 -> 231, back 397 -> 331; 512^2 x 361 x 2 slices 767 -> 306 and
 // 540 -> 441; 1024^2 x 720 3398 -> 1126 and 2301 -> 1665; 64^2 x 45 19 -> 19.5 and 43 -> 40.
 #include "epilogue.h"

@@ -1,10 +1,10 @@
 """The back walk's single-crossing bound, checked by brute force.
 
 A view whose bin width is not within rounding of the pixel width lets each pixel span
-hold at most one bin key, so the back walk takes one crossing per pixel with selects;
-only views flagged `multi` (plan.hip, dd_multi_cross: (r - 1) <= 4 * M * 2^-23 with
-r = min(rinv, 1/|b|) and M = (npix + 4) * (1 + |t| + r)) run the loop for further
-crossings.  Here every unflagged view of several geometries is checked in float32: the
+hold at most one bin key, so the back walk gives a pixel two bins, the crossing taken with
+selects; only views flagged `multi` (plan.hip, dd_multi_cross: (r - 1) <= 4 * M * 2^-23 with
+r = min(rinv, 1/|b|) and M = (npix + 4) * (1 + |t| + r)) look at a third bin.  Here every
+unflagged view of several geometries is checked in float32: the
 smallest gap between consecutive bin keys (both arithmetic forms) exceeds the largest
 pixel span on every line.
 """
