@@ -103,8 +103,8 @@ int itomo_radon_ss(float *image, int npix, const float *angles, int nang, int op
  * calls grow, the smaller copies before it; a call with more slices takes them in turns.  It is
  * allocated on first use, which neither waits for the GPU nor disturbs another thread's stream
  * capture.  While `stream` itself is captured, or without memory for it, the call reads the
- * images as they are: the same bits, up to twice the time (1024^2 x 720 slant-stacking 2.2 ms for
- * 1.1).  Inside itomo_sirt_iterate_noalloc and captured iterations it lies in their scratch.
+ * images as they are: the same bits, up to 2.3 times the time (1024^2 x 720 slant-stacking 1.8 ms
+ * for 0.76).  Inside itomo_sirt_iterate_noalloc and captured iterations it lies in their scratch.
  * Replaces class_projectors_radon.projectors.__init__ (class_projectors_radon.py:47-55).
  * ------------------------------------------------------------------------------- */
 int itomo_plan_create(itomo_plan **plan, int projector, int npix, const float *angles,

@@ -128,7 +128,8 @@ int launch_transpose(const float* in, float* out, int npix, int nslices, hipStre
 // Waves of 64 bins of a pixel-driven or slant-stacking forward call, and the number from which it
 // reads a transposed copy.  PD, us with and without: 511^2 x 360 views (2880 waves) 597 and 593;
 // 512^2 x 361 x 2 slices (5776) 991 and 989; 1024^2 x 720 (11520) 3552 and 3902.  SS: 257^2 x 180
-// (900) 102 and 85; 511^2 x 360 230 and 255; 512^2 x 361 x 2 306 and 569; 1024^2 x 720 1125 and 2196.
+// (900) 54 and 43; 400^2 x 280 (1960) 90 and 87; 450^2 x 300 (2400) 120 and 123; 511^2 x 360 (2880)
+// 135 and 163; 512^2 x 361 x 2 (5776) 213 and 418; 1024^2 x 720 (11520) 756 and 1772.
 inline int64_t copy_waves(const Plan& p, int nslices)
 {
     return (int64_t)((p.npix + 63) / 64) * p.nang * nslices;

@@ -19,11 +19,12 @@
 // stay inside the image.
 //
 // Both wait for their gathers (a lane per bin reads the sampled index, so in the forward one of
-// the two view families strides by rows): at 512^2 x 361 for 66% and 54% of the wave cycles, at
-// 2.1 and 2.5 waves per SIMD, the VALU busy 23% and 28% of the time.  us before and after lockstep
-// steps, the transposed copy and the two or three candidate bins, method 1:
-// 511^2 x 360 views forward 346 -> 231, back 397 -> 331; 512^2 x 361 x 2 slices 767 -> 306 and
-// 540 -> 441; 1024^2 x 720 3398 -> 1126 and 2301 -> 1665; 64^2 x 45 19 -> 19.5 and 43 -> 40.
+// the two view families strides by rows): at 512^2 x 361 for 36% and 54% of the wave cycles, at
+// 1.9 and 2.5 waves per SIMD, the VALU busy 42% and 28% of the time.  us before and after lockstep
+// steps, the transposed copy and the two or three candidate bins, and now that the forward's
+// steps without a pixel add -0 (see there), method 1: 64^2 x 45 views forward 19.1 -> 19.7 -> 11.6,
+// back 43 -> 40; 257^2 x 180 91 -> 85 -> 43, 173 -> 148; 511^2 x 360 349 -> 235 -> 135, 397 -> 331;
+// 512^2 x 361 x 2 slices 768 -> 309 -> 212, 540 -> 441; 1024^2 x 720 3176 -> 1125 -> 754, 2301 -> 1665.
 #include "epilogue.h"
 
 namespace itomo {
@@ -87,7 +88,9 @@ __device__ __forceinline__ float ss_upd0(float acc, double rab, float v)
 // neighbouring bins, step the same u together, from the first lane's start to the last
 // lane's end, and read the orientation in which the sampled index is contiguous (imageT, when
 // there is one, for views that step columns): a wave's loads are then nearly contiguous, and
-// four steps' loads are in flight before the first is added.
+// four steps' loads are in flight before the first is added.  A bin's sum is one serial chain: a
+// step outside the bin's range or the image adds -0, which leaves any sum as it is, where a
+// select after every addition lengthened the chain (and small calls, 3-5% slower by it).
 template <int ARITH, int METHOD, int EPI, bool ONES>
 __global__ void __launch_bounds__(kSsFwdBlock)
 ss_fwd_kernel(const SsView* __restrict__ geom, const int2* __restrict__ range, int npix,
@@ -119,41 +122,36 @@ ss_fwd_kernel(const SsView* __restrict__ geom, const int2* __restrict__ range, i
     const int ss = g.ybranch || flip ? npix : 1, sq = g.ybranch || flip ? 1 : npix;
     for (int u0 = first; u0 < last; u0 += U) {
         float fa[U], fb[U], wa[U], wb[U];
-        bool oa[U], ob[U];
 #pragma unroll
         for (int c = 0; c < U; ++c) {
             const int u = u0 + c;
             const bool in = u >= ur.x && u < ur.y;
             const float q = ss_q<ARITH>(g, u, tf);
             const float* __restrict__ line = img + (unsigned)((u + nh) * ss);
-            fb[c] = 1.0f;
-            wb[c] = 0.0f;
+            // what is added where there is no pixel: any sum plus -0 is that sum
+            fa[c] = fb[c] = -0.0f;
+            wa[c] = wb[c] = 1.0f;
             if (METHOD == 0) {
                 const int p = ss_round<ARITH>(q) + nh;
-                oa[c] = in && p >= 0 && p < npix;
-                ob[c] = false;
-                fa[c] = ONES || !oa[c] ? 1.0f : line[__umul24(p, sq)];
-                wa[c] = 1.0f;
+                if (in && p >= 0 && p < npix) fa[c] = ONES ? 1.0f : line[__umul24(p, sq)];
             } else {
                 float fl, w, wl;
                 ss_split<ARITH>(q, fl, w, wl);
                 const int p = (int)fl + nh;
-                oa[c] = in && p >= 0 && p <= npix - 1;
-                ob[c] = in && p + 1 >= 0 && p + 1 <= npix - 1;
-                fa[c] = ONES || !oa[c] ? 1.0f : line[__umul24(p, sq)];
-                fb[c] = ONES || !ob[c] ? 1.0f : line[__umul24(p + 1, sq)];
+                if (in && p >= 0 && p <= npix - 1) fa[c] = ONES ? 1.0f : line[__umul24(p, sq)];
+                if (in && p + 1 >= 0 && p + 1 <= npix - 1)
+                    fb[c] = ONES ? 1.0f : line[__umul24(p + 1, sq)];
                 wa[c] = wl;
                 wb[c] = w;
             }
         }
 #pragma unroll
         for (int c = 0; c < U; ++c) {
-            const float na = METHOD == 0 ? ss_upd0<ARITH>(acc, g.rab, fa[c])
-                                         : ss_fwd_upd<ARITH>(acc, wa[c], g.rab, fa[c]);
-            acc = oa[c] ? na : acc;
-            if (METHOD != 0) {
-                const float nb = ss_fwd_upd<ARITH>(acc, wb[c], g.rab, fb[c]);
-                acc = ob[c] ? nb : acc;
+            if (METHOD == 0) {
+                acc = ss_upd0<ARITH>(acc, g.rab, fa[c]);
+            } else {
+                acc = ss_fwd_upd<ARITH>(acc, wa[c], g.rab, fa[c]);
+                acc = ss_fwd_upd<ARITH>(acc, wb[c], g.rab, fb[c]);
             }
         }
     }

@@ -113,6 +113,19 @@ def test_copy_in_an_iteration_that_allocates_nothing(oper):
     assert torch.equal(x, y)
 
 
+@pytest.mark.parametrize("arith", ["fast", "ieee"])
+@pytest.mark.parametrize("method", [0, 1])
+@pytest.mark.parametrize("start", [-0.0, 0.0, -1.5, float("inf"), float("-inf")])
+def test_steps_without_a_pixel_leave_any_sum_as_it_is(start, method, arith):
+    n = 33                                   # odd: the last bin has no line
+    p = plan("ss", n, arith, method)
+    out = torch.full((V, n), start, device="cuda")
+    p.forward(torch.zeros((n, n), device="cuda"), out=out, accumulate=True)
+    got = out.cpu().numpy()
+    same(got[:, -1], np.full(V, start, np.float32))
+    np.testing.assert_array_equal(got, np.full((V, n), start, np.float32))
+
+
 @pytest.mark.parametrize("oper", ["pd", "ss"])
 def test_first_calls_and_growing_stacks_leave_another_capture_alone(oper):
     n, nz = 65, LINE[oper] // (2 * V) + 8
