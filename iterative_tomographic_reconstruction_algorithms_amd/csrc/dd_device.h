@@ -635,11 +635,14 @@ __device__ __forceinline__ float fwd_ones(const DdView& g, const float* __restri
 // is one nearly contiguous load.  No LDS, no barriers; bounds: vector L1 accesses (one
 // 4-byte load per candidate and lane) and the five VALU operations of a candidate.
 //
-// Lines outside the image or past the lane's own last line load nothing and get the right end
-// -1e30, which makes every weight 0: only pixels on a bin's own lines and among its
-// candidates are multiplied at all (a weight of 0 makes a NaN of an infinity).  Away from the end of
-// the line (q + NC < npix for every lane) the candidates need no bounds check and L* does
-// not clip (see dd_fwd_block); the last bin of a view always takes the checked form.
+// Lines outside the image (a lane's diagonal before its first or after its last line) load
+// nothing and get the right end -1e30, which makes every weight 0.  A weight of 0 makes a NaN of
+// an infinity, so the diagonals stay close to the bin's own lines: of the up to GL - 1 lines that
+// fill the last group two lie before them and one after (all after, an infinite pixel reached
+// bins four lines away; a test of every lane against its own last line cost 1% at 100^2 to
+// 256^2), and candidates past g.ncand are not loaded.  Away from the end of the line (q + NC < npix
+// for every lane) the candidates need no bounds check and L* does not clip (see dd_fwd_block);
+// the last bin of a view always takes the checked form.
 template <int ARITH, int NC, int GL>
 __device__ __forceinline__ float fwd_diag(const DdView& g, const float* __restrict__ ls,
                                           int npix, int nh, const float* __restrict__ img,
@@ -662,9 +665,9 @@ __device__ __forceinline__ float fwd_diag(const DdView& g, const float* __restri
     const int steps = (int)floor(((double)npix + (double)g.rinv) * fabs(rt) + 0.14) + 1;
     // L is monotonic in the bin: its extremes are in the first and the last lane
     const int La = __builtin_amdgcn_readlane(L, 0), Lb = __builtin_amdgcn_readlane(L, 63);
-    const int k0 = max(0, -max(La, Lb));
     const int k1 = min(steps - 1, npix - 1 - min(La, Lb));
-    const unsigned end = max(0, min(npix, L + steps));   // past the lane's last line
+    int k0 = max(0, -max(La, Lb));
+    k0 -= min(2, (GL - (k1 - k0 + 1) % GL) % GL);   // groups of GL lines, see above
     const int stride = npix * 4;
     if constexpr (NC > 0) {
         for (int k = k0; k <= k1; k += GL) {
@@ -675,7 +678,7 @@ __device__ __forceinline__ float fwd_diag(const DdView& g, const float* __restri
 #pragma unroll
             for (int l = 0; l < GL; ++l) {
                 const int i = L + k + l;
-                ok[l] = (unsigned)i < end;
+                ok[l] = (unsigned)i < (unsigned)npix;
                 K[l] = key_K<ARITH>(g, line_coord(i, nh));
                 xq[l] = first_pixel_near(Dlo, Dlh, K[l], nh, npix);
                 q[l] = (int)xq[l] + nh;
@@ -713,7 +716,7 @@ __device__ __forceinline__ float fwd_diag(const DdView& g, const float* __restri
         constexpr int CH = 16;   // candidates loaded together
         for (int k = k0; k <= k1; ++k) {
             const int i = L + k;
-            const bool ok = (unsigned)i < end;
+            const bool ok = (unsigned)i < (unsigned)npix;
             const float K = key_K<ARITH>(g, line_coord(i, nh));
             const float x = first_pixel(Dlo, K, nh, npix);
             const int q = (int)x + nh;
